@@ -58,6 +58,12 @@ enum {
   LSMF_CACHING_SCALAR_REFERENTIAL = 4
 };
 
+/* The variants differ in what they keep per quadrature point, not in the
+ * operator.  On meshes with the Q1 metric and formulation 1, TENSOR2 and
+ * TENSOR4 keep the same compact form of the tangent (J_cur^-1 and c dw per
+ * point, the rest per cell on affine cells); curved meshes and formulation 0
+ * keep the stored tensors. */
+
 /* operator number type: the reference instantiates NeoHookOperator with
  * number = double on the fine level and float on the MG levels
  * (include/mf_elasticity.h:673-674, 900-902). */

@@ -22,6 +22,9 @@
 //             M = (2c S + 2 lambda IxI) det(J_ref) w (Voigt 6x6 upper, 21)
 //   tensor2 : K, T, c1 = 2c det(J_ref) w, c2 = 2 lambda det(J_ref) w
 //   scalar  : c = mu - 2 lambda ln J   (F, J_ref recomputed per vmult)
+// tensor2 and tensor4 operators of formulation 1 with the Q1 metric store the
+// compact form instead (qp_compact): K, c dw, and A = mu dw J_ref^-1 J_ref^-T
+// and 2 lambda dw per point or, on affine cells, per cell.
 // With these, flux = Q K^T where Q = g T + M : sym(g) (or the tensor2 form)
 // and g = Grad_xi v K, i.e. exactly the reference's
 // Q = [g tau + Jc : sym g] / J integrated with JxW_cur = J det(J_ref) w.
@@ -61,6 +64,8 @@ enum Variant {
   V_TENSOR4 = 2,
   V_TENSOR4_NS = 3,
   V_SCALAR_REF = 4,
+  V_COMPACT = 5,  // tensor2 / tensor4 operators in compact form
+  V_COMPACT_AFFINE = 6,
   V_RESIDUAL = 100,
   V_ADJOINT = 101
 };
@@ -98,6 +103,8 @@ template <int NV> __host__ __device__ constexpr int sym_index(int v, int w) {
 //   tensor4_ns  J_ref^-1 (D2), dP/dF packed by its major symmetry (D2(D2+1)/2)
 //   scalar      c
 //   scalar_ref  c, u at the point (DIM)
+//   compact     K (D2), c dw, 2 lambda dw, A dw (NV); affine cells: K, c dw
+//               (A and 2 lambda det(J_ref) per cell, P.caff)
 template <int DIM, int VAR> struct CacheFields {
   static constexpr int NV = Voigt<DIM>::NV;
   static constexpr int D2 = DIM * DIM;
@@ -106,6 +113,8 @@ template <int DIM, int VAR> struct CacheFields {
                                : VAR == V_TENSOR4_NS ? D2 + D2 * (D2 + 1) / 2
                                : VAR == V_SCALAR_REF ? 1 + DIM
                                : VAR == V_SCALAR     ? 1
+                               : VAR == V_COMPACT    ? D2 + 2 + NV
+                               : VAR == V_COMPACT_AFFINE ? D2 + 1
                                                      : 0;
 };
 
@@ -148,6 +157,11 @@ template <typename T, int NF> __device__ __forceinline__ void load_cache(const T
     for (int k = 0; k < TAIL; ++k) v[FULL + k] = ct[k];
   }
 }
+
+// values per cell of the affine compact form: 2 lambda det(J_ref), then A (NV);
+// FP64 also for FP32 operators, so that a point's values, the product with its
+// weight, are rounded once, as the stored ones are
+constexpr int kAffineStride = 8;
 
 // 1D tables: S, D, St, Dt (N*N each), Gauss points and weights (N each),
 // then the collocation derivative on the Gauss points (N*N, used by
@@ -798,6 +812,55 @@ __device__ __forceinline__ void qp_tensor4_ns(const T (&G)[DIM][DIM], const T *c
   flux_times_kt<DIM>(P, Kr, Phi);
 }
 
+// Compact form of the formulation-1 tangent on cells with the Q1 metric.
+// With R = J_ref^-1 and K = J_cur^-1 = R F^-1 the flux of tensor2 / tensor4,
+// Phi = (g tau + 2 c sym g + 2 lambda tr(g) I) K^T dw, g = G K,
+// tau = mu F F^T - c I, loses its -c g K^T against the first half of
+// 2 c sym g, and K F = R turns mu g F F^T K^T into mu G R R^T:
+//   Phi = G A + c dw (K G K)^T + 2 lambda dw tr(K G) K^T,  A = mu dw R R^T.
+// Same tangent, but only K and c vary with the displacement: A and lambda dw
+// are one set per cell (times the point's weight) where the Q1 map is affine,
+// so a point needs 10 cached values in 3D instead of 17 (tensor2) or 36
+// (tensor4).  No difference of large terms is left for the product: in
+// tau = mu F F^T - c I they cancel at small strain.
+// The products are bound by the cached stream: 128^3 Q2 tensor4 FP64 3.86 ->
+// 1.77 ms (16.3 -> 4.5 GB cached), 61 x 67 x 59 Q2 tensor4 FP32 0.246 -> 0.165
+// ms, 64^3 Q4 tensor2 FP64 1.47 -> 1.33 ms; error against 64-bit references
+// 6.9e-15 -> 1.6e-15 (128^3 FP64), 1.4e-7 unchanged (FP32).
+template <int DIM, typename T>
+__device__ __forceinline__ void qp_compact(const T (&G)[DIM][DIM], const T *K, T cdw, T ldw, const T *A,
+                                           T (&Phi)[DIM][DIM]) {
+  T X[DIM][DIM];  // K G
+#pragma unroll
+  for (int d = 0; d < DIM; ++d)
+#pragma unroll
+    for (int e = 0; e < DIM; ++e) {
+      T s = K[d * DIM] * G[0][e];
+#pragma unroll
+      for (int j = 1; j < DIM; ++j) s = fma(K[d * DIM + j], G[j][e], s);
+      X[d][e] = s;
+    }
+  T tr = X[0][0];
+#pragma unroll
+  for (int d = 1; d < DIM; ++d) tr += X[d][d];
+  const T lt = ldw * tr;
+#pragma unroll
+  for (int d = 0; d < DIM; ++d) {
+    T Y[DIM];  // row d of c dw X
+#pragma unroll
+    for (int e = 0; e < DIM; ++e) Y[e] = cdw * X[d][e];
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) {
+      T s = lt * K[d * DIM + c];
+#pragma unroll
+      for (int e = 0; e < DIM; ++e) s = fma(Y[e], K[e * DIM + c], s);
+#pragma unroll
+      for (int e = 0; e < DIM; ++e) s = fma(G[c][e], A[voigt_index<DIM>(e, d)], s);
+      Phi[c][d] = s;
+    }
+  }
+}
+
 // Formulation 0, the volumetric/isochoric split (include/material.h:116-141,
 // 171-226, 260-295; include/mf_nh_operator.h:1005-1180), with
 // kappa = lambda + 2 mu / 3, b_bar = sbar^2 F F^T (sbar = J^{-1/d}),
@@ -929,6 +992,23 @@ __device__ __forceinline__ void q1_jacobian(const TC *X, const T *qp, int i0, in
   }
 }
 
+// J_ref of an affine cell: the mean edge vector of each direction.  Differences
+// of neighbouring vertices keep the digits that q1_jacobian's weighted sums of
+// all eight lose (J ~ h from terms ~ |X|).
+template <int DIM, typename T, typename TC>
+__device__ __forceinline__ void affine_jacobian(const TC *X, T (&J)[DIM][DIM]) {
+#pragma unroll
+  for (int i = 0; i < DIM; ++i)
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+      T s = T(0);
+#pragma unroll
+      for (int v = 0; v < (1 << DIM); ++v)
+        if (!((v >> d) & 1)) s += T(X[(v | (1 << d)) * DIM + i]) - T(X[v * DIM + i]);
+      J[i][d] = s * (T(2) / T(1 << DIM));
+    }
+}
+
 // local node index of Q1 corner v
 template <int DIM, int N> __host__ __device__ constexpr int corner_node(int v) {
   return ((v & 1) ? N - 1 : 0) + ((v >> 1 & 1) ? (N - 1) * N : 0) + (DIM == 3 && (v >> 2 & 1) ? (N - 1) * N * N : 0);
@@ -983,11 +1063,22 @@ template <typename Number> struct VmultParams {
   double *__restrict__ dmu;
   double *__restrict__ dlambda;
   const int32_t *__restrict__ perm;
+  const double *__restrict__ caff;  // affine compact form: [sorted cell][kAffineStride]
+  double qw[3];                     // 1D quadrature weights, the first half (symmetric)
   // even-odd forms of the 1D matrices S and D (EvenOdd<N>::PK values each,
   // N <= 5) for the line-per-lane sum factorization: uniform across lanes,
   // read from the kernel arguments
   Number sf[2 * 15];
 };
+
+// 1D weight of Gauss point i from the symmetric half in the kernel arguments
+template <int N> __device__ __forceinline__ double weight_1d(const double *qw, int i) {
+  const int k = i < N - 1 - i ? i : N - 1 - i;
+  double w = qw[0];
+#pragma unroll
+  for (int j = 1; j < (N + 1) / 2; ++j) w = k == j ? qw[j] : w;
+  return w;
+}
 
 // Kinematic prologue shared by the scalar vmult and the residual: gathers u
 // and the corner coordinates, returns F = I + Grad_xi u J_ref^-1 and
@@ -1033,7 +1124,8 @@ __device__ __forceinline__ void eulerian_metric(const T (&GX)[DIM][DIM], const T
 // LINE: 3D gradient by the line-per-lane sum factorization (P.sf set,
 // lds = the workgroup's slot buffers, t = thread, slot = this lane's cell).
 // Gu = Grad_xi u (rows: components, columns: xi directions).
-template <int DIM, int N, typename T, bool LINE = false, int CPW = CellShape<DIM, N>::CPW, int WG = kWG>
+template <int DIM, int N, typename T, bool LINE = false, int CPW = CellShape<DIM, N>::CPW, int WG = kWG,
+          bool AFFINE = false>
 __device__ __forceinline__ void kinematics_prologue(const VmultParams<T> &P, const T *tab, T *A, T *B, T *Xc,
                                                     bool on, bool active, uint32_t code, int r, int i0, int i1, int i2,
                                                     T (&F)[DIM][DIM], T (&Jri)[DIM][DIM], T &detJr, T (&Gu)[DIM][DIM],
@@ -1054,7 +1146,8 @@ __device__ __forceinline__ void kinematics_prologue(const VmultParams<T> &P, con
   else
     SF<DIM, N, T>::template evaluate<DIM>(tab, A, B, on, r, i0, i1, i2, Gu);
   T Jr[DIM][DIM];
-  q1_jacobian<DIM, T, T>(Xc, tab + 4 * N * N, i0, i1, i2, Jr);
+  if constexpr (AFFINE) affine_jacobian<DIM>(Xc, Jr);
+  else q1_jacobian<DIM, T, T>(Xc, tab + 4 * N * N, i0, i1, i2, Jr);
   detJr = inverse<DIM>(Jr, Jri);
   grad_times<DIM>(Gu, Jri, F);
 #pragma unroll
@@ -1124,7 +1217,7 @@ __device__ __forceinline__ void kinematics_collocation(const VmultParams<T> &P, 
 // workgroups per CU, at most 128 VGPRs); the wide tensor2 kernel 6 (three
 // workgroups, at most 80 VGPRs, which its FP64 form needs no more than).
 template <int VAR, int TILE> constexpr int vmult_min_waves() {
-  return TILE != kTileWide ? 1 : VAR == V_TENSOR2 ? 6 : 4;
+  return TILE != kTileWide ? 1 : VAR == V_TENSOR2 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE ? 6 : 4;
 }
 
 template <int DIM, int N, typename T, int VAR, bool ADD, bool CONSTR, unsigned PH, int TILE>
@@ -1216,6 +1309,10 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
   __builtin_amdgcn_sched_barrier(0);
   T cch[NF > 0 ? NF : 1];
   if constexpr ((PH & PH_QD) && NF > 0 && !RECOMP) load_cache<T, NF>(P.cache, cell_s * NQP + r_s, P.fs, cch);
+  double caff[VAR == V_COMPACT_AFFINE ? 1 + Voigt<DIM>::NV : 1];
+  if constexpr ((PH & PH_QD) && VAR == V_COMPACT_AFFINE)
+#pragma unroll
+    for (int k = 0; k < 1 + Voigt<DIM>::NV; ++k) caff[k] = P.caff[cell_s * kAffineStride + k];
   __builtin_amdgcn_sched_barrier(0);
 
   // tile-local index of this lane's node (tiled layout)
@@ -1314,6 +1411,16 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
       for (int c = 0; c < DIM; ++c)
 #pragma unroll
         for (int d = 0; d < DIM; ++d) Phi[c][d] = G[c][d];
+    } else if constexpr (VAR == V_COMPACT) {
+      constexpr int D2 = DIM * DIM;
+      qp_compact<DIM, T>(G, cch, cch[D2], cch[D2 + 1], cch + D2 + 2, Phi);
+    } else if constexpr (VAR == V_COMPACT_AFFINE) {
+      double w = weight_1d<N>(P.qw, i0) * weight_1d<N>(P.qw, i1);
+      if constexpr (DIM == 3) w *= weight_1d<N>(P.qw, i2);
+      T aw[1 + Voigt<DIM>::NV];
+#pragma unroll
+      for (int k = 0; k < 1 + Voigt<DIM>::NV; ++k) aw[k] = T(caff[k] * w);
+      qp_compact<DIM, T>(G, cch, cch[DIM * DIM], aw[0], aw + 1, Phi);
     } else if constexpr (VAR == V_TENSOR4) {
       qp_tensor4<DIM, T>(G, cch, Phi);
     } else if constexpr (VAR == V_TENSOR4_NS) {
@@ -1586,6 +1693,7 @@ struct CacheParams {
   const double *__restrict__ mu;
   const double *__restrict__ lambda;
   void *cache;
+  double *caff;  // affine compact form: per-cell values
   size_t fs;
   int n_cells;
   int formulation;
@@ -1618,7 +1726,7 @@ template <int DIM, int N, typename T, int VAR> __global__ void __launch_bounds__
   KP.u = P.u;
   KP.coords = P.coords;
   double F[DIM][DIM], Jri[DIM][DIM], detJr, Gu[DIM][DIM], GX[DIM][DIM];
-  kinematics_prologue<DIM, N, double>(KP, tab, A, B, Xc, on, active, code, r, i0, i1, i2, F, Jri, detJr, Gu);
+  kinematics_prologue<DIM, N, double, false, CPW, kWG, VAR == V_COMPACT_AFFINE>(KP, tab, A, B, Xc, on, active, code, r, i0, i1, i2, F, Jri, detJr, Gu);
   // the spatial caches carry the current metric: Eulerian Q_p on curved meshes
   constexpr bool SPATIAL = (VAR == V_TENSOR2 || VAR == V_TENSOR4);
   if (SPATIAL && P.curved)
@@ -1698,6 +1806,27 @@ template <int DIM, int N, typename T, int VAR> __global__ void __launch_bounds__
     for (int v = 0; v < NV; ++v) put(D2 + v, Tv[v]);
 #pragma unroll
     for (int k = 0; k < NV * (NV + 1) / 2; ++k) put(D2 + NV + k, M[k]);
+  } else if constexpr (VAR == V_COMPACT || VAR == V_COMPACT_AFFINE) {
+    // K and c dw per point; A = mu dw R R^T and 2 lambda dw per point, or
+    // without the quadrature weight once per cell where R is one per cell
+#pragma unroll
+    for (int d = 0; d < DIM; ++d)
+#pragma unroll
+      for (int j = 0; j < DIM; ++j) put(d * DIM + j, K[d][j]);
+    put(D2, cs * dw);
+    const double aw = VAR == V_COMPACT ? dw : detJr;
+    double *ca = P.caff + (size_t)cell * kAffineStride;
+    if (VAR == V_COMPACT) put(D2 + 1, 2.0 * l * aw);
+    else if (r == 0) ca[0] = 2.0 * l * aw;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int i = voigt_first<DIM>(v), j = voigt_second<DIM>(v);
+      double s = 0;
+#pragma unroll
+      for (int k = 0; k < DIM; ++k) s += Jri[i][k] * Jri[j][k];
+      if (VAR == V_COMPACT) put(D2 + 2 + v, m * s * aw);
+      else if (r == 0) ca[1 + v] = m * s * aw;
+    }
   } else {  // tensor2 (include/mf_nh_operator.h:535-547)
 #pragma unroll
     for (int d = 0; d < DIM; ++d)
@@ -1734,7 +1863,9 @@ __global__ void __launch_bounds__(kWG) k_diagonal(const VmultParams<T> P) {
   constexpr int NV = Voigt<DIM>::NV;
   // the scalar variant evaluates the tensor4 fields per point (either
   // formulation) and shares the tensor4 closed form
+  constexpr bool COMPACT = VAR == V_COMPACT || VAR == V_COMPACT_AFFINE;  // V_COMPACT's fields in LDS
   constexpr int NF = (VAR == V_TENSOR2) ? CacheFields<DIM, V_TENSOR2>::value
+                     : COMPACT              ? CacheFields<DIM, V_COMPACT>::value
                      : (VAR == V_TENSOR4_NS) ? CacheFields<DIM, V_TENSOR4_NS>::value
                                              : CacheFields<DIM, V_TENSOR4>::value;
   constexpr int TABN = 4 * N * N + 2 * N;
@@ -1816,10 +1947,17 @@ __global__ void __launch_bounds__(kWG) k_diagonal(const VmultParams<T> P) {
     }
   } else {
     if (active) {
-      T v[NF];
-      load_cache<T, NF>(P.cache, (size_t)cell * NQP + r, P.fs, v);
+      constexpr int NFC = CacheFields<DIM, VAR>::value;
+      T v[NFC];
+      load_cache<T, NFC>(P.cache, (size_t)cell * NQP + r, P.fs, v);
 #pragma unroll
-      for (int f = 0; f < NF; ++f) qd[f * NQP + r] = v[f];
+      for (int f = 0; f < NFC; ++f) qd[f * NQP + r] = v[f];
+      if constexpr (VAR == V_COMPACT_AFFINE) {
+        double w = weight_1d<N>(P.qw, i0) * weight_1d<N>(P.qw, i1);
+        if constexpr (DIM == 3) w *= weight_1d<N>(P.qw, i2);
+#pragma unroll
+        for (int k = 0; k < 1 + NV; ++k) qd[(NFC + k) * NQP + r] = T(P.caff[(size_t)cell * kAffineStride + k] * w);
+      }
     }
   }
   lds_barrier();
@@ -1861,6 +1999,19 @@ __global__ void __launch_bounds__(kWG) k_diagonal(const VmultParams<T> P) {
           for (int f = 0; f < DIM; ++f) s = fma(gam[e] * gam[f], Am[sym_index<D2>(c * DIM + e, c * DIM + f) * NQP + q], s);
         acc[c] += s;
       }
+      return;
+    }
+    if constexpr (COMPACT) {
+      // e_c (x) grad phi in qp_compact: gph.A gph + (c + 2 lambda) dw gam_c^2
+      const T *qA = qd + (DIM * DIM + 2) * NQP;
+      T s = T(0);
+#pragma unroll
+      for (int i = 0; i < DIM; ++i)
+#pragma unroll
+        for (int j = 0; j < DIM; ++j) s = fma(gph[i] * gph[j], qA[voigt_index<DIM>(i, j) * NQP + q], s);
+      const T cl = qd[DIM * DIM * NQP + q] + qd[(DIM * DIM + 1) * NQP + q];
+#pragma unroll
+      for (int c = 0; c < DIM; ++c) acc[c] += fma(cl * gam[c], gam[c], s);
       return;
     }
     T geo = T(0);

@@ -15,7 +15,8 @@ template <int DIM, int N> struct Launch {
   // tensor4 operators (their products, residual and residual VJP)
   template <int VAR> static constexpr bool wide_ok() {
     return DIM == 3 && (N == 5 || N == 3) &&
-           (VAR == V_TENSOR2 || VAR == V_TENSOR4 || VAR == V_RESIDUAL || VAR == V_ADJOINT);
+           (VAR == V_TENSOR2 || VAR == V_TENSOR4 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE ||
+            VAR == V_RESIDUAL || VAR == V_ADJOINT);
   }
 
   // one colour's fused cell kernel: n tiles (tiled layouts) or n cells, nv
@@ -69,6 +70,8 @@ template <int DIM, int N> struct Launch {
     P.dmu = op->adj_dmu;
     P.dlambda = op->adj_dlambda;
     P.perm = op->d_perm;
+    P.caff = op->d_caff;
+    for (int k = 0; k < 3; ++k) P.qw[k] = op->h_qw[k];
     using EO = EvenOdd<N, T>;
     static_assert(sizeof(P.sf) / sizeof(P.sf[0]) >= 2 * EO::PK, "1D matrices do not fit the kernel arguments");
     // even-odd forms of S (rows r < R) and D, from the plain tables
@@ -203,12 +206,14 @@ template <int DIM, int N> struct Launch {
 #define LSMF_BATCH(V)                                                                          \
   return f64 ? vmult_batched_t<double, V>(op, (double *)dst, (const double *)src, nvec, s) \
              : vmult_batched_t<float, V>(op, (float *)dst, (const float *)src, nvec, s)
-    switch (op->caching) {
-      case LSMF_CACHING_TENSOR4: LSMF_BATCH(V_TENSOR4);
-      case LSMF_CACHING_TENSOR2: LSMF_BATCH(V_TENSOR2);
-      case LSMF_CACHING_SCALAR: LSMF_BATCH(V_SCALAR);
-      case LSMF_CACHING_TENSOR4_NS: LSMF_BATCH(V_TENSOR4_NS);
-      case LSMF_CACHING_SCALAR_REFERENTIAL: LSMF_BATCH(V_SCALAR_REF);
+    switch (cache_variant(op)) {
+      case V_COMPACT: LSMF_BATCH(V_COMPACT);
+      case V_COMPACT_AFFINE: LSMF_BATCH(V_COMPACT_AFFINE);
+      case V_TENSOR4: LSMF_BATCH(V_TENSOR4);
+      case V_TENSOR2: LSMF_BATCH(V_TENSOR2);
+      case V_SCALAR: LSMF_BATCH(V_SCALAR);
+      case V_TENSOR4_NS: LSMF_BATCH(V_TENSOR4_NS);
+      case V_SCALAR_REF: LSMF_BATCH(V_SCALAR_REF);
       default:
         return fail(LSMF_ERR_UNKNOWN_CACHING, "vmult_batched: caching variant not available on the GPU");
     }
@@ -218,20 +223,26 @@ template <int DIM, int N> struct Launch {
   static int vmult(const lsmf_op *op, void *dst, const void *src, bool add, bool constr, unsigned ph,
                    hipStream_t s) {
     const bool f64 = op->precision == LSMF_FP64;
-    switch (op->caching) {
-      case LSMF_CACHING_TENSOR4:
+    switch (cache_variant(op)) {
+      case V_COMPACT:
+        return f64 ? vmult_t<double, V_COMPACT>(op, dst, src, add, constr, ph, s)
+                   : vmult_t<float, V_COMPACT>(op, dst, src, add, constr, ph, s);
+      case V_COMPACT_AFFINE:
+        return f64 ? vmult_t<double, V_COMPACT_AFFINE>(op, dst, src, add, constr, ph, s)
+                   : vmult_t<float, V_COMPACT_AFFINE>(op, dst, src, add, constr, ph, s);
+      case V_TENSOR4:
         return f64 ? vmult_t<double, V_TENSOR4>(op, dst, src, add, constr, ph, s)
                    : vmult_t<float, V_TENSOR4>(op, dst, src, add, constr, ph, s);
-      case LSMF_CACHING_TENSOR2:
+      case V_TENSOR2:
         return f64 ? vmult_t<double, V_TENSOR2>(op, dst, src, add, constr, ph, s)
                    : vmult_t<float, V_TENSOR2>(op, dst, src, add, constr, ph, s);
-      case LSMF_CACHING_SCALAR:
+      case V_SCALAR:
         return f64 ? vmult_t<double, V_SCALAR>(op, dst, src, add, constr, ph, s)
                    : vmult_t<float, V_SCALAR>(op, dst, src, add, constr, ph, s);
-      case LSMF_CACHING_TENSOR4_NS:
+      case V_TENSOR4_NS:
         return f64 ? vmult_t<double, V_TENSOR4_NS>(op, dst, src, add, constr, ph, s)
                    : vmult_t<float, V_TENSOR4_NS>(op, dst, src, add, constr, ph, s);
-      case LSMF_CACHING_SCALAR_REFERENTIAL:
+      case V_SCALAR_REF:
         return f64 ? vmult_t<double, V_SCALAR_REF>(op, dst, src, add, constr, ph, s)
                    : vmult_t<float, V_SCALAR_REF>(op, dst, src, add, constr, ph, s);
       default:
@@ -248,6 +259,7 @@ template <int DIM, int N> struct Launch {
     P.mu = op->d_mu64;
     P.lambda = op->d_lambda64;
     P.cache = op->d_cache;
+    P.caff = op->d_caff;
     P.fs = op->field_stride;
     P.n_cells = op->n_cells;
     P.formulation = op->formulation;
@@ -259,16 +271,20 @@ template <int DIM, int N> struct Launch {
 
   static int cache(const lsmf_op *op, int *bad, hipStream_t s) {
     const bool f64 = op->precision == LSMF_FP64;
-    switch (op->caching) {
-      case LSMF_CACHING_TENSOR4:
+    switch (cache_variant(op)) {
+      case V_COMPACT:
+        return f64 ? cache_t<double, V_COMPACT>(op, bad, s) : cache_t<float, V_COMPACT>(op, bad, s);
+      case V_COMPACT_AFFINE:
+        return f64 ? cache_t<double, V_COMPACT_AFFINE>(op, bad, s) : cache_t<float, V_COMPACT_AFFINE>(op, bad, s);
+      case V_TENSOR4:
         return f64 ? cache_t<double, V_TENSOR4>(op, bad, s) : cache_t<float, V_TENSOR4>(op, bad, s);
-      case LSMF_CACHING_TENSOR2:
+      case V_TENSOR2:
         return f64 ? cache_t<double, V_TENSOR2>(op, bad, s) : cache_t<float, V_TENSOR2>(op, bad, s);
-      case LSMF_CACHING_SCALAR:
+      case V_SCALAR:
         return f64 ? cache_t<double, V_SCALAR>(op, bad, s) : cache_t<float, V_SCALAR>(op, bad, s);
-      case LSMF_CACHING_TENSOR4_NS:
+      case V_TENSOR4_NS:
         return f64 ? cache_t<double, V_TENSOR4_NS>(op, bad, s) : cache_t<float, V_TENSOR4_NS>(op, bad, s);
-      case LSMF_CACHING_SCALAR_REFERENTIAL:
+      case V_SCALAR_REF:
         return f64 ? cache_t<double, V_SCALAR_REF>(op, bad, s) : cache_t<float, V_SCALAR_REF>(op, bad, s);
       default:
         return fail(LSMF_ERR_UNKNOWN_CACHING, "cache: caching variant not available on the GPU");
@@ -320,15 +336,19 @@ template <int DIM, int N> struct Launch {
 
   static int diagonal(const lsmf_op *op, hipStream_t s) {
     const bool f64 = op->precision == LSMF_FP64;
-    switch (op->caching) {
-      case LSMF_CACHING_TENSOR4:
+    switch (cache_variant(op)) {
+      case V_COMPACT:
+        return f64 ? diagonal_t<double, V_COMPACT>(op, s) : diagonal_t<float, V_COMPACT>(op, s);
+      case V_COMPACT_AFFINE:
+        return f64 ? diagonal_t<double, V_COMPACT_AFFINE>(op, s) : diagonal_t<float, V_COMPACT_AFFINE>(op, s);
+      case V_TENSOR4:
         return f64 ? diagonal_t<double, V_TENSOR4>(op, s) : diagonal_t<float, V_TENSOR4>(op, s);
-      case LSMF_CACHING_TENSOR2:
+      case V_TENSOR2:
         return f64 ? diagonal_t<double, V_TENSOR2>(op, s) : diagonal_t<float, V_TENSOR2>(op, s);
-      case LSMF_CACHING_SCALAR:
-      case LSMF_CACHING_SCALAR_REFERENTIAL:  // c is field 0 of both caches; F from u
+      case V_SCALAR:
+      case V_SCALAR_REF:  // c is field 0 of both caches; F from u
         return f64 ? diagonal_t<double, V_SCALAR>(op, s) : diagonal_t<float, V_SCALAR>(op, s);
-      case LSMF_CACHING_TENSOR4_NS:
+      case V_TENSOR4_NS:
         return f64 ? diagonal_t<double, V_TENSOR4_NS>(op, s) : diagonal_t<float, V_TENSOR4_NS>(op, s);
       default:
         return fail(LSMF_ERR_UNKNOWN_CACHING, "diagonal: caching variant not available on the GPU");

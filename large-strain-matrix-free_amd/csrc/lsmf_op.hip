@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <array>
 #include <cstring>
+#include <limits>
 #include <mutex>
 #include <new>
 #include <string>
@@ -44,17 +45,41 @@ const LaunchTable *launch_table(int dim, int N) {
 
 size_t elem_size(const lsmf_op *op) { return op->precision == LSMF_FP64 ? sizeof(double) : sizeof(float); }
 
-int n_cache_fields(int dim, int caching) {
-  const int nv = dim == 3 ? 6 : 3;
-  switch (caching) {
-    case LSMF_CACHING_TENSOR4: return dim * dim + nv + nv * (nv + 1) / 2;
-    case LSMF_CACHING_TENSOR2: return dim * dim + nv + 2;
-    case LSMF_CACHING_TENSOR4_NS: return dim * dim + dim * dim * (dim * dim + 1) / 2;
-    case LSMF_CACHING_SCALAR: return 1;
-    case LSMF_CACHING_SCALAR_REFERENTIAL: return 1 + dim;
+// Tensor2 and tensor4 operators run the compact form of the same tangent
+// where it exists: formulation 1 with the Q1 metric.  Curved meshes (Eulerian
+// Q_p metric: K F is no longer J_ref^-1) and formulation 0 keep the stored
+// tensors.
+int cache_variant(const lsmf_op *op) {
+  const bool compact = op->formulation == 1 && !op->curved;
+  switch (op->caching) {
+    case LSMF_CACHING_TENSOR4:
+    case LSMF_CACHING_TENSOR2:
+      if (compact) return op->affine ? V_COMPACT_AFFINE : V_COMPACT;
+      return op->caching == LSMF_CACHING_TENSOR4 ? V_TENSOR4 : V_TENSOR2;
+    case LSMF_CACHING_TENSOR4_NS: return V_TENSOR4_NS;
+    case LSMF_CACHING_SCALAR: return V_SCALAR;
+    case LSMF_CACHING_SCALAR_REFERENTIAL: return V_SCALAR_REF;
     default: return -1;
   }
 }
+
+namespace {
+template <int DIM> int fields_of(int variant) {
+  switch (variant) {
+    case V_COMPACT: return CacheFields<DIM, V_COMPACT>::value;
+    case V_COMPACT_AFFINE: return CacheFields<DIM, V_COMPACT_AFFINE>::value;
+    case V_TENSOR4: return CacheFields<DIM, V_TENSOR4>::value;
+    case V_TENSOR2: return CacheFields<DIM, V_TENSOR2>::value;
+    case V_TENSOR4_NS: return CacheFields<DIM, V_TENSOR4_NS>::value;
+    case V_SCALAR: return CacheFields<DIM, V_SCALAR>::value;
+    case V_SCALAR_REF: return CacheFields<DIM, V_SCALAR_REF>::value;
+    default: return -1;
+  }
+}
+int n_cache_fields(const lsmf_op *op) {
+  return op->dim == 3 ? fields_of<3>(cache_variant(op)) : fields_of<2>(cache_variant(op));
+}
+}  // namespace
 
 namespace {
 
@@ -80,7 +105,7 @@ template <typename T> int dalloc(T **p, size_t n, const char *what) {
 
 void free_op(lsmf_op *op) {
   void *ptrs[] = {op->d_idx,  op->d_coords,    op->d_tab,  op->d_tab64, op->d_mu64,     op->d_lambda64,
-                  op->d_mu,   op->d_lambda,    op->d_cache, op->d_diag, op->d_inv_diag, op->d_cons,
+                  op->d_mu,   op->d_lambda,    op->d_cache, op->d_caff, op->d_diag, op->d_inv_diag, op->d_cons,
                   op->d_bad,  op->d_perm,      op->d_tile_nodes, op->d_tile_info, op->d_orphan, op->d_hang, op->d_hptr,
                   op->d_hmaster, op->d_hw, op->d_hcons, op->d_hg_node, op->d_hg_ptr, op->d_hg_inst, op->d_hg_w,
                   op->d_hbuf, op->d_dcell, op->d_deptr, op->d_dtptr, op->d_dta, op->d_dtw, op->d_dbuf,
@@ -283,6 +308,38 @@ bool support_points_curved(const lsmf_mesh_desc *m, int dim, int p, int nqp) {
   return false;
 }
 
+// Every cell's Q1 vertex map is affine to the rounding of the coordinates:
+// the mixed differences of its vertices (xy, yz, zx, xyz) vanish, so J_ref
+// is one matrix per cell.  The bound is absolute, a few units in the last
+// place of the largest coordinate: what representing the vertices costs.
+bool cells_affine(const lsmf_mesh_desc *m, int dim, int p, int nqp) {
+  const int N = p + 1, NV = 1 << dim;
+  int corner[8];
+  for (int v = 0; v < NV; ++v) {
+    int a = 0, stride = 1;
+    for (int d = 0; d < dim; ++d, stride *= N) a += ((v >> d) & 1) * p * stride;
+    corner[v] = a;
+  }
+  double top = 0.0;
+  for (size_t i = 0; i < (size_t)m->n_nodes * dim; ++i) top = std::max(top, std::fabs(m->coords[i]));
+  const double tol = 8.0 * std::numeric_limits<double>::epsilon() * top;
+  for (int c = 0; c < m->n_cells; ++c) {
+    const int32_t *cn = m->cell_nodes + (size_t)c * nqp;
+    for (int i = 0; i < dim; ++i) {
+      double X[8];
+      for (int v = 0; v < NV; ++v) X[v] = m->coords[(size_t)cn[corner[v]] * dim + i];
+      // vertex v against the affine map of vertex 0 and its neighbours
+      for (int v = 3; v < NV; ++v) {
+        double x = X[0];
+        for (int d = 0; d < dim; ++d)
+          if ((v >> d) & 1) x += X[1 << d] - X[0];
+        if (!(std::fabs(x - X[v]) <= tol)) return false;
+      }
+    }
+  }
+  return true;
+}
+
 struct TileDims {
   int tx, ty, tz, nx, ny, nz, tn;
 };
@@ -405,6 +462,13 @@ __global__ void k_convert_f64_f32(const double *__restrict__ a, float *__restric
 
 namespace lsmf {
 namespace {
+// bytes of the cached values a product reads
+size_t cache_bytes(const lsmf_op *op) {
+  const size_t es = elem_size(op);
+  return (size_t)op->n_fields * op->field_stride * es +
+         (cache_variant(op) == V_COMPACT_AFFINE ? (size_t)op->n_cells * kAffineStride * sizeof(double) : 0);
+}
+
 // cache(): zero the det F <= 0 counter bad_dev, run the cache kernel, read
 // the count back (synchronising the stream)
 lsmf_status cache_with_counter(lsmf_op *op, int *bad_dev, hipStream_t s, const char *what) {
@@ -469,7 +533,7 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
   if (dim != 2 && dim != 3) return fail(LSMF_ERR_INVALID_ARGUMENT, "lsmf_op_create: dim must be 2 or 3");
   if (opt->precision != LSMF_FP64 && opt->precision != LSMF_FP32)
     return fail(LSMF_ERR_INVALID_ARGUMENT, "lsmf_op_create: unknown precision");
-  if (n_cache_fields(dim, opt->caching) < 0)
+  if (opt->caching < LSMF_CACHING_SCALAR || opt->caching > LSMF_CACHING_SCALAR_REFERENTIAL)
     return fail(LSMF_ERR_UNKNOWN_CACHING, "Unknown caching");
   if (nq != p + 1 || !launch_table(dim, nq))
     return fail(LSMF_ERR_UNSUPPORTED, "lsmf_op_create: (dim, degree, n_q_1d) = (" + std::to_string(dim) + ", " +
@@ -497,7 +561,6 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
   op->n_cells = nc;
   op->n_nodes = mesh->n_nodes;
   op->n_dofs = (size_t)mesh->n_nodes * dim;
-  op->n_fields = n_cache_fields(dim, opt->caching);
   op->field_stride = (size_t)nc * nqp;
 
   // --- node (hanging) constraints: validated, closed (masters are free)
@@ -605,6 +668,8 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
       }
     }
   op->curved = p > 1 && support_points_curved(mesh, dim, p, nqp);
+  op->affine = cells_affine(mesh, dim, p, nqp);
+  op->n_fields = n_cache_fields(op);
   // --- cell order of the tiled layout (structured meshes) replaces the
   // colour order; the per-cell index table then carries no first-touch bits
   std::vector<uint32_t> tnodes;
@@ -798,6 +863,7 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
     tab[4 * N * N + N + q] = t1.qw[q];
   }
   for (int i = 0; i < 2 * N * N; ++i) op->h_sf[i] = tab[i];
+  for (int k = 0; k < (N + 1) / 2; ++k) op->h_qw[k] = t1.qw[k];
 
   const size_t es = elem_size(op);
   int rc = 0;
@@ -810,6 +876,8 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
       (rc = dalloc((char **)&op->d_lambda, (size_t)nc * es, "lambda")) ||
       (rc = dalloc(&op->d_u64, op->n_dofs, "displacement")) ||
       (rc = dalloc((char **)&op->d_cache, (size_t)op->n_fields * op->field_stride * es, "cache")) ||
+      (cache_variant(op) == V_COMPACT_AFFINE &&
+       (rc = dalloc(&op->d_caff, (size_t)nc * kAffineStride, "cell constants"))) ||
       (rc = dalloc((char **)&op->d_diag, op->n_dofs * es, "diagonal")) ||
       (rc = dalloc((char **)&op->d_inv_diag, op->n_dofs * es, "inverse diagonal")) ||
       (rc = dalloc(&op->d_cons, cons.size(), "constrained list")) || (rc = dalloc(&op->d_bad, 1, "counter")) ||
@@ -848,7 +916,7 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
     return rc;
   }
   op->bytes_idx = idx.size() * sizeof(uint32_t);
-  op->bytes_cache = (size_t)op->n_fields * op->field_stride * es;
+  op->bytes_cache = cache_bytes(op);
   hipError_t e = hipSuccess;
   e = hipMemcpy(op->d_idx, idx.data(), idx.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
   if (e == hipSuccess)
@@ -976,9 +1044,26 @@ lsmf_status lsmf_set_formulation(lsmf_op *op, int formulation) {
     return fail(LSMF_ERR_INVALID_ARGUMENT, "set_formulation: Unknown material formulation");
   if (formulation == 0 && op->caching != LSMF_CACHING_SCALAR && op->caching != LSMF_CACHING_TENSOR4)
     return fail(LSMF_ERR_UNSUPPORTED, "set_formulation: formulation 0 needs scalar or tensor4 caching");
-  op->formulation = formulation;
   op->cached = false;
   op->diag_ok = false;
+  if (formulation == op->formulation) return LSMF_OK;
+  // the cached values of the other formulation take another amount of memory
+  const int before = op->formulation;
+  op->formulation = formulation;
+  const int nf = n_cache_fields(op);
+  if (nf != op->n_fields) {
+    void *p = nullptr;
+    const size_t es = elem_size(op);
+    const int rc = dalloc((char **)&p, (size_t)nf * op->field_stride * es, "cache");
+    if (rc) {
+      op->formulation = before;
+      return rc;
+    }
+    (void)hipFree(op->d_cache);
+    op->d_cache = p;
+    op->n_fields = nf;
+  }
+  op->bytes_cache = cache_bytes(op);
   return LSMF_OK;
 }
 

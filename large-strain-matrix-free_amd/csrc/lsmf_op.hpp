@@ -53,6 +53,7 @@ struct lsmf_op {
   int precision = LSMF_FP64, caching = LSMF_CACHING_TENSOR4;
   int formulation = 1;  // material formulation (include/material.h:82-94)
   bool curved = false;  // some support point off its cell's Q1 map: Eulerian Q_p current metric
+  bool affine = false;  // every cell's Q1 map is affine: one J_ref per cell
   int n_cells = 0, n_nodes = 0;
   size_t n_dofs = 0;
   int n_fields = 0;
@@ -67,11 +68,13 @@ struct lsmf_op {
   void *d_tab = nullptr;            // S, D, St, Dt, qp, qw in operator precision
   double *d_tab64 = nullptr;        // same tables in FP64 (cache kernel)
   double h_sf[2 * 25] = {};         // S[q][k] then D[q][k] (N x N each), kernel-argument copy
+  double h_qw[3] = {};              // 1D quadrature weights, the first half
   double *d_mu64 = nullptr, *d_lambda64 = nullptr;  // per sorted cell
   void *d_mu = nullptr, *d_lambda = nullptr;        // operator precision
   double *d_u64 = nullptr;          // linearisation state copy
   void *d_u = nullptr;              // operator precision copy (scalar variant)
   void *d_cache = nullptr;
+  double *d_caff = nullptr;         // affine compact form: [sorted cell][kAffineStride]
   void *d_diag = nullptr, *d_inv_diag = nullptr;
   int32_t *d_cons = nullptr;        // constrained DoF list
   int n_cons = 0;
@@ -129,6 +132,7 @@ struct LaunchTable {
 };
 
 const LaunchTable *launch_table(int dim, int N);
-int n_cache_fields(int dim, int caching);
+// the Variant whose cached values the operator's products read
+int cache_variant(const lsmf_op *op);
 
 }  // namespace lsmf

@@ -1,0 +1,99 @@
+"""The compact form of the tensor2 / tensor4 products (K, c dw per point, the
+rest per affine cell or per point) against the oracle's stored tensors, on
+parallelepiped cells (affine, J_ref not diagonal), on the Cook geometry
+(bilinear cells) and over the formulation switch, at mesh sizes that leave
+tiles full, ragged and nearly empty.  FP64 to 1e-12, FP32 to 2e-5 (max-norm),
+the tolerances of the operator's other parity tests.
+"""
+import numpy as np
+import pytest
+
+import lsmf
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+SHEAR = np.array([[1.0, 0.3, -0.2], [0.1, 0.8, 0.25], [-0.15, 0.2, 1.1]])
+
+
+def rel(a, b):
+    return float(np.abs(a - b).max() / np.abs(b).max())
+
+
+def problem(dim, p, n, geometry):
+    mesh = lsmf.Mesh(dim, p, n, geometry="cook" if geometry == "cook" else "box")
+    if geometry == "sheared":
+        mesh.coords = np.ascontiguousarray(mesh.coords @ SHEAR[:dim, :dim].T)
+    rng = np.random.default_rng(3)
+    mu, lam = 1.0 + rng.random(mesh.n_cells), 2.0 + rng.random(mesh.n_cells)
+    u, _ = lsmf.smooth_displacement(mesh.coords, 0.02, 7)
+    cons = mesh.constrained_mask({0: list(range(dim)), 1: [0]})
+    return mesh, mu, lam, u, cons
+
+
+def oracle_op(mesh, mu, lam, u, cons, caching, formulation=1):
+    ref = oracle.OracleOperator(mesh.dim, mesh.degree, mesh.cell_nodes, mesh.coords, cons, caching=caching,
+                                formulation=formulation)
+    ref.set_material(mu, lam)
+    ref.set_linearization(u)
+    ref.cache()
+    return ref
+
+
+@pytest.mark.parametrize("geometry", ["sheared", "cook"])
+@pytest.mark.parametrize("dim,p,n", [(2, 1, [9, 8]), (2, 2, [8, 5]), (2, 4, [6, 3]), (3, 1, [5, 4, 3]),
+                                     (3, 2, [1, 1, 1]), (3, 2, [9, 2, 1]), (3, 2, [15, 3, 5]), (3, 4, [1, 1, 1]),
+                                     (3, 4, [5, 3, 2])],
+                         ids=lambda v: str(v).replace(" ", ""))
+def test_compact_products_match_oracle(dim, p, n, geometry, device):
+    import torch
+    print(f"[compact] dim={dim} p={p} n={n} {geometry}", flush=True)
+    mesh, mu, lam, u, cons = problem(dim, p, n, geometry)
+    ref = oracle_op(mesh, mu, lam, u, cons, "tensor4")
+    rng = np.random.default_rng(4)
+    v, w = (rng.standard_normal(mesh.n_dofs).astype(np.float32).astype(np.float64) for _ in range(2))
+    expect, plain, diag = ref.vmult(v), ref.vmult(v, plain=True), ref.diagonal()
+    for layout in ("auto", "cells"):
+        for prec, tol in (("fp64", 1e-12), ("fp32", 2e-5)):
+            op = lsmf.NeoHookOperator(mesh, precision=prec, caching="tensor4", constrained=cons, layout=layout)
+            op.set_material(mu, lam)
+            op.set_linearization(torch.tensor(u, device=device))
+            op.cache()
+            src = torch.tensor(v, device=device, dtype=op.dtype)
+            y = torch.full_like(src, np.nan)
+            op.vmult(y, src)
+            assert rel(y.cpu().double().numpy(), expect) < tol, (layout, prec)
+            y = torch.tensor(w, device=device, dtype=op.dtype)
+            op.vmult_add(y, src)
+            assert rel(y.cpu().double().numpy(), w + expect) < tol, (layout, prec)
+            y = torch.full_like(src, np.nan)
+            op.vmult(y, src, mask="plain")
+            assert rel(y.cpu().double().numpy(), plain) < tol, (layout, prec)
+            batch = torch.stack([src, 2 * src, -src])
+            out = torch.full_like(batch, np.nan)
+            op.vmult_batched(out, batch)
+            op.vmult(y, src)
+            assert torch.equal(out[0], y) and torch.equal(out[1], 2 * y) and torch.equal(out[2], -y)
+            op.compute_diagonal()
+            assert rel(op.diagonal().cpu().double().numpy(), diag) < tol, (layout, prec)
+
+
+def test_formulation_switch_changes_the_cached_values(device):
+    import torch
+    mesh, mu, lam, u, cons = problem(3, 2, [4, 3, 2], "sheared")
+    v = np.random.default_rng(4).standard_normal(mesh.n_dofs)
+    op = lsmf.NeoHookOperator(mesh, caching="tensor4", constrained=cons)
+    op.set_material(mu, lam)
+    op.set_linearization(torch.tensor(u, device=device))
+    src = torch.tensor(v, device=device)
+    y = torch.empty_like(src)
+    bytes_of = {}
+    for formulation in (1, 0, 1, 0):
+        lsmf._check(lsmf._lib.lsmf_set_formulation(op._h, formulation))
+        with pytest.raises(lsmf.LsmfError):
+            op.vmult(y, src)  # the cache is of the other formulation
+        op.cache()
+        op.vmult(y, src)
+        expect = oracle_op(mesh, mu, lam, u, cons, "tensor4", formulation).vmult(v)
+        assert rel(y.cpu().numpy(), expect) < 1e-12, formulation
+        assert bytes_of.setdefault(formulation, op.memory_consumption()) == op.memory_consumption()
