@@ -194,6 +194,7 @@ template <int DIM, int N, int WG_ = kWG> struct TileShape {
   static constexpr int TN = NX * NY * NZ;
   static_assert(TX * TY * TZ == CPW, "tile must hold the workgroup's cells");
   static_assert(TN <= WG, "one lane per tile node");
+  static constexpr int TW = (TN + 31) / 32;  // words of a tile's tpriv bits
 };
 constexpr uint32_t kNoNode = 0xFFFFFFFFu;  // tile node outside the mesh
 
@@ -1037,6 +1038,13 @@ template <typename Number> struct VmultParams {
   int curved;       // support points off the Q1 maps: Eulerian Q_p metric (scalar variants)
   const uint32_t *__restrict__ tnodes;  // tiled layout: [tile][TN] node codes
   const int32_t *__restrict__ tinfo;    // tiled layout: [tile][2] first cell, extents
+  const int32_t *__restrict__ tlist;    // coloured launches: the tiles by colour; nullptr: tile = block
+  // one launch over all tiles (nullptr: coloured launches): a tile writes the
+  // nodes that only it touches (bit set in tpriv, TW words per tile) and
+  // leaves its share of the others in tbuf [tile][TN][DIM] for k_tile_sum
+  const uint32_t *__restrict__ tpriv;
+  Number *__restrict__ tbuf;
+  int identity;  // with tbuf: constrained DoFs get the identity here and in k_tile_sum
   // node (hanging) constraints, cells layout only; hang == nullptr: none.
   // Each (cell, constrained node) pair is an instance: its cell reads the
   // weighted sum of the masters and leaves its result in hbuf, from where
@@ -1272,9 +1280,9 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
   size_t node = 0;
   // tiled layout: slot -> (sx, sy, sz) in the tile, lane t < TN -> tile node
   const int sx = slot % TS::TX, sy = (slot / TS::TX) % TS::TY, sz = slot / (TS::TX * TS::TY);
-  const int tile = P.cell_begin + L;
+  const int tile = TILE && P.tlist ? P.tlist[P.cell_begin + L] : P.cell_begin + L;
   uint32_t tcode = 0;
-  bool tvalid = false;
+  bool tvalid = false, tshared = false;  // tshared: the node's sum is k_tile_sum's
   size_t tnode = 0;
   T sv[DIM];
   T dv[DIM];
@@ -1289,11 +1297,16 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
     tcode = P.tnodes[(size_t)tile * TN + (t < TN ? t : 0)];
     tvalid = t < TN && tcode != kNoNode;
     tnode = tvalid ? (tcode & kNodeMask) : 0;
+    if (P.tbuf) {
+      const uint32_t *priv = P.tpriv + (size_t)tile * TS::TW;
+      tshared = !((priv[t < TN ? t / 32 : 0] >> (t % 32)) & 1u);
+    }
     if constexpr (VAR != V_RESIDUAL) load_node<DIM, T>(src + tnode * DIM, sv);
     // the node's destination values, read now rather than at the final
-    // read-modify-write: no other tile of this colour touches the node, so
-    // they do not change before this tile writes them
-    if (tvalid && (ADD || !(tcode & kFirstBit))) load_node<DIM, T>(dst + tnode * DIM, dv);
+    // read-modify-write: no other tile of this colour (of the launch: a
+    // private node) touches the node, so they do not change before this tile
+    // writes them
+    if (tvalid && (ADD ? !tshared : !P.tbuf && !(tcode & kFirstBit))) load_node<DIM, T>(dst + tnode * DIM, dv);
   } else {
     cell = P.cell_begin + L * CPW + slot;
     active = on && (cell < P.cell_end);
@@ -1601,12 +1614,18 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
       T nv[DIM];
 #pragma unroll
       for (int c = 0; c < DIM; ++c) nv[c] = tile_v[t * DIM + c] + acc[c];  // destination: 0 on first touch
-      if (!CONSTR || !((tcode >> kConsShift) & ((1u << DIM) - 1u))) {
+      if (tshared) {
+        store_node<DIM, T>(P.tbuf + ((size_t)tile * TN + t) * DIM, nv);
+      } else if (!CONSTR || !((tcode >> kConsShift) & ((1u << DIM) - 1u))) {
         store_node<DIM, T>(dst + tnode * DIM, nv);
       } else {
 #pragma unroll
-        for (int c = 0; c < DIM; ++c)
+        for (int c = 0; c < DIM; ++c) {
           if (!((tcode >> (kConsShift + c)) & 1u)) dst[tnode * DIM + c] = nv[c];
+          // the identity on a constrained DoF (coloured launches: k_constrained_identity)
+          else if (P.tbuf && P.identity)
+            dst[tnode * DIM + c] = (ADD ? tile_v[t * DIM + c] : T(0)) + src[tnode * DIM + c];
+        }
       }
     }
     return;
@@ -1634,6 +1653,83 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
     T *h = P.hbuf + (size_t)blockIdx.y * P.hstride + (size_t)hidx * DIM;
 #pragma unroll
     for (int c = 0; c < DIM; ++c) h[c] = out[c];
+  }
+}
+
+// ------------------------------------------------------------------------
+// Second half of a product done in one launch over all tiles: every node that
+// several tiles touch sums their shares from tbuf in colour order, the order
+// in which coloured launches add to it (same bits), and is written once.
+// Nodes are grouped by the number M of tiles that touch them (2, 4, 8); group
+// g holds nodes [begin[g], begin[g + 1]) and its slots k-th tile by k-th tile
+// (coalesced), slot = tile * TN + tile node.  One lane per node.
+//
+// Against 2^dim coloured launches: two launches instead of eight, all tiles
+// at once (a 32^3 Q2 mesh has 256 tiles per colour, one per CU).  Per 9x2x1
+// tile 51 of 285 nodes are private; the other 234 are written to and read
+// from tbuf where coloured launches read and write 141 and write 93 in place,
+// and neighbouring tiles run together, so source nodes come from L2.
+// ------------------------------------------------------------------------
+constexpr int kMaxGroups = 8;
+template <typename T> struct TileSumParams {
+  const uint32_t *__restrict__ node;  // node | constraint bits
+  const uint32_t *__restrict__ slot;
+  const T *__restrict__ buf;
+  const T *__restrict__ src;  // constrained rows (CONSTR)
+  T *__restrict__ dst;
+  int identity;
+  int n_groups;
+  int begin[kMaxGroups + 1];
+  int mult[kMaxGroups];
+  size_t first_slot[kMaxGroups];
+};
+
+template <int DIM, int M, typename T>
+__device__ __forceinline__ void sum_slots(const uint32_t *__restrict__ slot, size_t stride,
+                                          const T *__restrict__ buf, T (&acc)[DIM]) {
+  uint32_t id[M];
+#pragma unroll
+  for (int k = 0; k < M; ++k) id[k] = slot[k * stride];
+  T v[M][DIM];
+#pragma unroll
+  for (int k = 0; k < M; ++k) load_node<DIM, T>(buf + (size_t)id[k] * DIM, v[k]);
+#pragma unroll
+  for (int k = 0; k < M; ++k)
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) acc[c] += v[k][c];
+}
+
+template <int DIM, typename T, bool ADD, bool CONSTR>
+__global__ void __launch_bounds__(kWG) k_tile_sum(const TileSumParams<T> P) {
+  const int i = xcd_remap(blockIdx.x, gridDim.x) * kWG + (int)threadIdx.x;
+  int g = 0;
+  while (g < P.n_groups && i >= P.begin[g + 1]) ++g;
+  if (g >= P.n_groups) return;
+  const size_t stride = (size_t)(P.begin[g + 1] - P.begin[g]);
+  const uint32_t *slot = P.slot + P.first_slot[g] + (i - P.begin[g]);
+  const uint32_t code = P.node[i];
+  const size_t node = code & kNodeMask;
+  T acc[DIM];
+#pragma unroll
+  for (int c = 0; c < DIM; ++c) acc[c] = T(0);
+  if constexpr (ADD) load_node<DIM, T>(P.dst + node * DIM, acc);
+  T old[DIM];
+#pragma unroll
+  for (int c = 0; c < DIM; ++c) old[c] = acc[c];
+  const int m = P.mult[g];
+  if (m == 2) sum_slots<DIM, 2, T>(slot, stride, P.buf, acc);
+  else if (m == 4) sum_slots<DIM, 4, T>(slot, stride, P.buf, acc);
+  else if (m == 8) sum_slots<DIM, 8, T>(slot, stride, P.buf, acc);
+  else
+    for (int k = 0; k < m; ++k) sum_slots<DIM, 1, T>(slot + k * stride, stride, P.buf, acc);
+  if (!CONSTR || !((code >> kConsShift) & ((1u << DIM) - 1u))) {
+    store_node<DIM, T>(P.dst + node * DIM, acc);
+  } else {
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) {
+      if (!((code >> (kConsShift + c)) & 1u)) P.dst[node * DIM + c] = acc[c];
+      else if (P.identity) P.dst[node * DIM + c] = old[c] + P.src[node * DIM + c];
+    }
   }
 }
 
@@ -1894,7 +1990,7 @@ __global__ void __launch_bounds__(kWG) k_diagonal(const VmultParams<T> P) {
   const int i0 = r % N, i1 = (r / N) % N, i2 = (DIM == 3) ? r / (N * N) : 0;
   const int L = xcd_remap(blockIdx.x, gridDim.x);
   const bool on = slot < CPW;
-  const int tile = P.cell_begin + L;
+  const int tile = TILE && P.tlist ? P.tlist[P.cell_begin + L] : P.cell_begin + L;
   int ex = 0, ey = 0, ez = 0;
   for (int round = 0; round < ROUNDS; ++round) {
   const int ts = round * CPW + slot;  // this lane's cell within the tile

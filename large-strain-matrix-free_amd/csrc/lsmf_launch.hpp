@@ -54,6 +54,7 @@ template <int DIM, int N> struct Launch {
     P.curved = op->curved;
     P.tnodes = op->d_tile_nodes;
     P.tinfo = op->d_tile_info;
+    P.tlist = op->d_tile_list;
     P.hang = op->d_hang;
     P.hcons = op->d_hcons;
     P.hbuf = static_cast<T *>(op->d_hbuf);
@@ -116,6 +117,61 @@ template <int DIM, int N> struct Launch {
                        op->n_hang_masters);
   }
 
+  // all tiles in one launch, then the sums of the nodes they share (with
+  // CONSTR and identity also the constrained rows)
+  template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
+  static int run_tiles(const lsmf_op *op, T *dst, const T *src, int identity, hipStream_t s) {
+    VmultParams<T> P = params<T>(op, 0);
+    P.src = src;
+    P.dst = dst;
+    P.tlist = nullptr;
+    P.cell_begin = 0;
+    P.cell_end = op->tile_ptr.back();
+    P.tpriv = op->d_tile_priv;
+    P.tbuf = static_cast<T *>(op->d_tile_buf);
+    P.identity = identity;
+    if (op->prof) op->prof->before(s);
+    const int rc = launch_vmult<T, VAR, ADD, CONSTR, PH>(op, P, P.cell_end, 1, s);
+    if (rc) return rc;
+    const int n = op->sum_begin[op->n_sum_groups];
+    if (n > 0) {
+      TileSumParams<T> S{};
+      S.node = op->d_sum_node;
+      S.slot = op->d_sum_slot;
+      S.buf = P.tbuf;
+      S.src = src;
+      S.dst = dst;
+      S.identity = identity;
+      S.n_groups = op->n_sum_groups;
+      for (int g = 0; g < S.n_groups; ++g) {
+        S.begin[g] = op->sum_begin[g];
+        S.mult[g] = op->sum_mult[g];
+        S.first_slot[g] = op->sum_first_slot[g];
+      }
+      S.begin[S.n_groups] = n;
+      hipLaunchKernelGGL((k_tile_sum<DIM, T, ADD, CONSTR>), dim3((n + kWG - 1) / kWG), dim3(kWG), 0, s, S);
+    }
+    if (op->prof) op->prof->after(s);
+    return 0;
+  }
+
+  // the cell kernels of one product: one launch over all tiles where the
+  // stream may use the tile buffer, else one launch per colour.  *identity:
+  // in, the constrained rows are wanted; out, they are still to be done
+  // (rows of DoFs that no cell touches are done by the list either way)
+  template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
+  static int run_cells(const lsmf_op *op, T *dst, const T *src, bool *identity, hipStream_t s) {
+    if (op->d_tile_buf) {
+      const TileBufferLock lock(op, s);
+      if (lock) {
+        const int fold = identity && *identity && op->n_orphan == 0;
+        if (fold) *identity = false;
+        return run_tiles<T, VAR, ADD, CONSTR, PH>(op, dst, src, fold, s);
+      }
+    }
+    return run_colours<T, VAR, ADD, CONSTR, PH>(op, dst, src, s);
+  }
+
   // one launch per colour; the tiled layout launches one workgroup per tile
   template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
   static int run_colours(const lsmf_op *op, T *dst, const T *src, hipStream_t s) {
@@ -145,20 +201,21 @@ template <int DIM, int N> struct Launch {
     if (!add) zero_orphans(op, dst, s);
     int rc;
     if (constr) {
+      bool identity = op->n_cons > 0;
       if (ph == FULL) {
-        if (add) rc = run_colours<T, VAR, true, true, FULL>(op, dst, src, s);
-        else rc = run_colours<T, VAR, false, true, FULL>(op, dst, src, s);
+        if (add) rc = run_cells<T, VAR, true, true, FULL>(op, dst, src, &identity, s);
+        else rc = run_cells<T, VAR, false, true, FULL>(op, dst, src, &identity, s);
       } else if (ph == PH_SF) {
-        rc = run_colours<T, VAR, false, true, PH_SF>(op, dst, src, s);
+        rc = run_cells<T, VAR, false, true, PH_SF>(op, dst, src, &identity, s);
       } else {
-        rc = run_colours<T, VAR, false, true, 0u>(op, dst, src, s);
+        rc = run_cells<T, VAR, false, true, 0u>(op, dst, src, &identity, s);
       }
-      if (op->n_cons > 0)
+      if (identity)
         hipLaunchKernelGGL(k_constrained_identity<T>, dim3((op->n_cons + 255) / 256), dim3(256), 0, s, op->d_cons,
                            op->n_cons, src, dst, add ? 1 : 0);
     } else {
-      if (add) rc = run_colours<T, VAR, true, false, FULL>(op, dst, src, s);
-      else rc = run_colours<T, VAR, false, false, FULL>(op, dst, src, s);
+      if (add) rc = run_cells<T, VAR, true, false, FULL>(op, dst, src, nullptr, s);
+      else rc = run_cells<T, VAR, false, false, FULL>(op, dst, src, nullptr, s);
     }
     if (rc) return rc;
     return hipGetLastError() == hipSuccess ? 0 : LSMF_ERR_HIP;
@@ -360,7 +417,7 @@ template <int DIM, int N> struct Launch {
     constexpr unsigned FULL = PH_SF | PH_QD;
     zero_if_constrained(op, rhs, false, s);
     zero_orphans(op, rhs, s);
-    const int rc = run_colours<double, V_RESIDUAL, false, false, FULL>(op, rhs, nullptr, s);
+    const int rc = run_cells<double, V_RESIDUAL, false, false, FULL>(op, rhs, nullptr, nullptr, s);
     if (rc) return rc;
     return hipGetLastError() == hipSuccess ? 0 : LSMF_ERR_HIP;
   }
@@ -370,7 +427,7 @@ template <int DIM, int N> struct Launch {
     constexpr unsigned FULL = PH_SF | PH_QD;
     zero_if_constrained(op, du, false, s);
     zero_orphans(op, du, s);
-    const int rc = run_colours<double, V_ADJOINT, false, false, FULL>(op, du, w, s);
+    const int rc = run_cells<double, V_ADJOINT, false, false, FULL>(op, du, w, nullptr, s);
     if (rc) return rc;
     return hipGetLastError() == hipSuccess ? 0 : LSMF_ERR_HIP;
   }

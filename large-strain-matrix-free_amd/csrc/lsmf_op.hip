@@ -63,6 +63,31 @@ int cache_variant(const lsmf_op *op) {
   }
 }
 
+void bind_stream(lsmf_op *op, hipStream_t s) {
+  op->ws_bound = true;
+  op->ws_stream = s;
+  op->ws_capture = true;
+}
+
+TileBufferLock::TileBufferLock(const lsmf_op *op, hipStream_t s) {
+  if (!op->d_tile_buf || s == hipStreamPerThread) return;  // that handle is a stream per thread
+  if (!op->ws_capture) {
+    // a captured product may be replayed on any stream
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
+    if (st != hipStreamCaptureStatusNone) return;
+  }
+  std::unique_lock<std::mutex> lock(op->ws_mu);
+  if (!op->ws_bound) {
+    op->ws_bound = true;
+    op->ws_stream = s;
+  }
+  if (op->ws_stream == s) lock_ = std::move(lock);
+}
+
 namespace {
 template <int DIM> int fields_of(int variant) {
   switch (variant) {
@@ -106,7 +131,8 @@ template <typename T> int dalloc(T **p, size_t n, const char *what) {
 void free_op(lsmf_op *op) {
   void *ptrs[] = {op->d_idx,  op->d_coords,    op->d_tab,  op->d_tab64, op->d_mu64,     op->d_lambda64,
                   op->d_mu,   op->d_lambda,    op->d_cache, op->d_caff, op->d_diag, op->d_inv_diag, op->d_cons,
-                  op->d_bad,  op->d_perm,      op->d_tile_nodes, op->d_tile_info, op->d_orphan, op->d_hang, op->d_hptr,
+                  op->d_bad,  op->d_perm,      op->d_tile_nodes, op->d_tile_info, op->d_tile_tables,
+                  op->d_tile_buf, op->d_orphan, op->d_hang, op->d_hptr,
                   op->d_hmaster, op->d_hw, op->d_hcons, op->d_hg_node, op->d_hg_ptr, op->d_hg_inst, op->d_hg_w,
                   op->d_hbuf, op->d_dcell, op->d_deptr, op->d_dtptr, op->d_dta, op->d_dtw, op->d_dbuf,
                   op->d_dg_node, op->d_dg_ptr, op->d_dg_ent};
@@ -361,94 +387,166 @@ bool tile_dims(int dim, int N, int kind, TileDims &t) {
 }
 
 // Tiles of a logically structured mesh (cell grid cell_at, n cells per
-// direction), coloured by the parity of their position so that no two tiles
-// of one colour share a node.  Fills perm (tile order, the cells of a tile
-// consecutive in slot order), tile_ptr, the tile node table (node ids from
-// the cells' own node lists; first-touch bit: the node's first tile in
-// colour order) and tile info.  Returns kNotTileable when cells that share
-// a tile node position disagree about its node (the cells layout then
-// serves the mesh).
+// direction) in grid order, coloured by the parity of their position so that
+// no two tiles of one colour share a node.  Fills perm (tile order, the cells
+// of a tile consecutive in slot order), the tile node table (node ids from
+// the cells' own node lists; first-touch bit: the node's first tile in colour
+// order), tile info, the tiles by colour, and for products in one launch the
+// private-node bits and the shared nodes with their slots.  Returns
+// kNotTileable when cells that share a tile node position disagree about its
+// node (the cells layout then serves the mesh).
 constexpr int kNotTileable = 1;
+// Largest operator whose products run in one launch: above it the tiles'
+// shares of common nodes travel to HBM and back and cost more than the
+// coloured launches' starts and tails save.  One launch against 8 coloured
+// ones, 3D Q2 tensor4 FP64, us: 13 / 59 (16^3), 42 / 66 (32^3), 128 / 156
+// (48^3, 2.7 M DoF), 276 / 284 (64^3, 6.4 M), 485 / 461 (80^3), 2116 / 1814
+// (128^3); scalar 203 / 218 (48^3), 493 / 450 (64^3); Q4 tensor4 FP32 52 / 78
+// (24^3, 2.7 M), 117 / 118 (32^3, 6.4 M), 217 / 206 (40^3); 2D Q2 FP64 (4
+// colours) 50 / 58 (2.1 M), 190 / 173 (8.4 M).
+constexpr size_t kOneLaunchDofs = 4000000;
+struct TileTables {
+  std::vector<uint32_t> nodes, priv, sum_node, sum_slot;
+  std::vector<int32_t> info, list;
+};
 int build_tiles(lsmf_op *op, const lsmf_mesh_desc *mesh, const long long n[3], const std::vector<int32_t> &cell_at,
-                std::vector<uint32_t> &tnodes, std::vector<int32_t> &tinfo) {
+                TileTables &tt) {
   const int dim = op->dim, p = op->degree, N = p + 1, nqp = op->nqp;
   TileDims td;
   if (!tile_dims(dim, op->N, op->tile_kind, td)) return fail(LSMF_ERR_UNSUPPORTED, "tiles: no tile shape");
   const long long TXn = (n[0] + td.tx - 1) / td.tx, TYn = (n[1] + td.ty - 1) / td.ty,
                   TZn = (n[2] + td.tz - 1) / td.tz;
   const long long n_tiles = TXn * TYn * TZn;
-  const int n_col = 1 << dim;
-  std::vector<long long> order;
-  order.reserve(n_tiles);
+  const int n_col = 1 << dim, tw = (td.tn + 31) / 32;
+  std::vector<uint8_t> tcol(n_tiles);
+  for (long long b = 0; b < n_tiles; ++b)
+    tcol[b] = (uint8_t)((b % TXn & 1) | ((b / TXn % TYn & 1) << 1) | ((b / (TXn * TYn) & 1) << 2));
+  tt.list.clear();
+  tt.list.reserve(n_tiles);
   op->tile_ptr.assign(n_col + 1, 0);
   for (int col = 0; col < n_col; ++col) {
-    for (long long bz = 0; bz < TZn; ++bz)
-      for (long long by = 0; by < TYn; ++by)
-        for (long long bx = 0; bx < TXn; ++bx)
-          if (((bx & 1) | ((by & 1) << 1) | ((bz & 1) << 2)) == col) order.push_back(bx + TXn * (by + TYn * bz));
-    op->tile_ptr[col + 1] = (int)order.size();
+    for (long long b = 0; b < n_tiles; ++b)
+      if (tcol[b] == col) tt.list.push_back((int32_t)b);
+    op->tile_ptr[col + 1] = (int)tt.list.size();
   }
   op->perm.assign(op->n_cells, 0);
   op->inv_perm.assign(op->n_cells, 0);
-  tinfo.assign((size_t)n_tiles * 2, 0);
-  tnodes.assign((size_t)n_tiles * td.tn, kNoNode);
-  std::vector<int> min_col(mesh->n_nodes, 1 << 30), stamp(mesh->n_nodes, -1);
+  tt.info.assign((size_t)n_tiles * 2, 0);
+  tt.nodes.assign((size_t)n_tiles * td.tn, kNoNode);
+  std::vector<uint8_t> cols(mesh->n_nodes, 0);  // colours of the tiles that touch a node
+  // tile position l: (slot, local node) of the tile's cells that hold it
+  std::vector<std::pair<int, int>> at;
+  std::vector<int> at_ptr(1, 0);
+  for (int l = 0; l < td.tn; ++l) {
+    const int X = l % td.nx, Y = (l / td.nx) % td.ny, Z = l / (td.nx * td.ny);
+    for (int sz = 0; sz < td.tz; ++sz)
+      for (int sy = 0; sy < td.ty; ++sy)
+        for (int sx = 0; sx < td.tx; ++sx) {
+          const int x = X - sx * p, y = Y - sy * p, z = Z - sz * p;
+          if (x >= 0 && x <= p && y >= 0 && y <= p && z >= 0 && z <= p)
+            at.push_back({sx + td.tx * (sy + td.ty * sz), x + N * (y + N * z)});
+        }
+    at_ptr.push_back((int)at.size());
+  }
+  std::vector<const int32_t *> cell_nodes(td.tx * td.ty * td.tz);
   int pos = 0;
-  for (int col = 0; col < n_col; ++col)
-    for (int ti = op->tile_ptr[col]; ti < op->tile_ptr[col + 1]; ++ti) {
-      const long long b = order[ti];
-      const long long bx = b % TXn, by = (b / TXn) % TYn, bz = b / (TXn * TYn);
-      const int ex = (int)std::min<long long>(td.tx, n[0] - bx * td.tx);
-      const int ey = (int)std::min<long long>(td.ty, n[1] - by * td.ty);
-      const int ez = (int)std::min<long long>(td.tz, n[2] - bz * td.tz);
-      tinfo[(size_t)ti * 2] = pos;
-      tinfo[(size_t)ti * 2 + 1] = ex | (ey << 8) | (ez << 16);
-      auto tile_cell = [&](int sx, int sy, int sz) {
-        return cell_at[(bx * td.tx + sx) + n[0] * ((by * td.ty + sy) + n[1] * (bz * td.tz + sz))];
-      };
-      for (int sz = 0; sz < ez; ++sz)
-        for (int sy = 0; sy < ey; ++sy)
-          for (int sx = 0; sx < ex; ++sx) {
-            const int cell = tile_cell(sx, sy, sz);
-            op->perm[pos] = cell;
-            op->inv_perm[cell] = pos;
-            ++pos;
-          }
-      for (int l = 0; l < td.tn; ++l) {
-        const int X = l % td.nx, Y = (l / td.nx) % td.ny, Z = l / (td.nx * td.ny);
-        if (X > ex * p || Y > ey * p || Z > ez * p) continue;  // beyond a ragged tile
-        // the node from every cell of the tile that holds this position
-        // (the kernels sum those cells' contributions into it)
-        const int xs[2] = {X == 0 ? 0 : (X - 1) / p, std::min(X / p, ex - 1)};
-        const int ys[2] = {Y == 0 ? 0 : (Y - 1) / p, std::min(Y / p, ey - 1)};
-        const int zs[2] = {Z == 0 ? 0 : (Z - 1) / p, std::min(Z / p, ez - 1)};
-        long long node = -1;
-        for (int cz = zs[0]; cz <= zs[1]; ++cz)
-          for (int cy = ys[0]; cy <= ys[1]; ++cy)
-            for (int cx = xs[0]; cx <= xs[1]; ++cx) {
-              const int a = (X - cx * p) + N * ((Y - cy * p) + (dim == 3 ? N * (Z - cz * p) : 0));
-              const long long nd = mesh->cell_nodes[(size_t)tile_cell(cx, cy, cz) * nqp + a];
-              if (node >= 0 && nd != node) return kNotTileable;
-              node = nd;
-            }
-        if (stamp[node] == col) return kNotTileable;  // two tiles of one colour share a node
-        stamp[node] = col;
-        min_col[node] = std::min(min_col[node], col);
-        tnodes[(size_t)ti * td.tn + l] = (uint32_t)node;
+  for (long long b = 0; b < n_tiles; ++b) {
+    const long long bx = b % TXn, by = (b / TXn) % TYn, bz = b / (TXn * TYn);
+    const int ex = (int)std::min<long long>(td.tx, n[0] - bx * td.tx);
+    const int ey = (int)std::min<long long>(td.ty, n[1] - by * td.ty);
+    const int ez = (int)std::min<long long>(td.tz, n[2] - bz * td.tz);
+    tt.info[(size_t)b * 2] = pos;
+    tt.info[(size_t)b * 2 + 1] = ex | (ey << 8) | (ez << 16);
+    auto tile_cell = [&](int sx, int sy, int sz) {
+      return cell_at[(bx * td.tx + sx) + n[0] * ((by * td.ty + sy) + n[1] * (bz * td.tz + sz))];
+    };
+    std::fill(cell_nodes.begin(), cell_nodes.end(), nullptr);
+    for (int sz = 0; sz < ez; ++sz)
+      for (int sy = 0; sy < ey; ++sy)
+        for (int sx = 0; sx < ex; ++sx) {
+          const int cell = tile_cell(sx, sy, sz);
+          cell_nodes[sx + td.tx * (sy + td.ty * sz)] = mesh->cell_nodes + (size_t)cell * nqp;
+          op->perm[pos] = cell;
+          op->inv_perm[cell] = pos;
+          ++pos;
+        }
+    for (int l = 0; l < td.tn; ++l) {
+      // the node from every cell of the tile that holds this position (the
+      // kernels sum those cells' contributions into it); none: beyond a
+      // ragged tile
+      long long node = -1;
+      for (int k = at_ptr[l]; k < at_ptr[l + 1]; ++k) {
+        const int32_t *cn = cell_nodes[at[k].first];
+        if (!cn) continue;
+        const long long nd = cn[at[k].second];
+        if (node >= 0 && nd != node) return kNotTileable;
+        node = nd;
       }
+      if (node < 0) continue;
+      if ((cols[node] >> tcol[b]) & 1u) return kNotTileable;  // two tiles of one colour share a node
+      cols[node] |= (uint8_t)(1u << tcol[b]);
+      tt.nodes[(size_t)b * td.tn + l] = (uint32_t)node;
     }
+  }
   if (pos != op->n_cells) return fail(LSMF_ERR_INVALID_ARGUMENT, "tiles: cell count mismatch");
-  for (int col = 0; col < n_col; ++col)
-    for (int ti = op->tile_ptr[col]; ti < op->tile_ptr[col + 1]; ++ti)
+  auto cons_bits = [&](size_t node) {
+    uint32_t bits = 0;
+    if (mesh->constrained)
+      for (int comp = 0; comp < dim; ++comp)
+        if (mesh->constrained[node * dim + comp]) bits |= 1u << (kConsShift + comp);
+    return bits;
+  };
+  if (op->n_dofs > kOneLaunchDofs) {
+    for (long long b = 0; b < n_tiles; ++b)
       for (int l = 0; l < td.tn; ++l) {
-        uint32_t &code = tnodes[(size_t)ti * td.tn + l];
+        uint32_t &code = tt.nodes[(size_t)b * td.tn + l];
         if (code == kNoNode) continue;
         const uint32_t node = code;
-        if (mesh->constrained)
-          for (int comp = 0; comp < dim; ++comp)
-            if (mesh->constrained[(size_t)node * dim + comp]) code |= 1u << (kConsShift + comp);
-        if (min_col[node] == col) code |= kFirstBit;
+        code |= cons_bits(node);
+        if (!(cols[node] & ((1u << tcol[b]) - 1u))) code |= kFirstBit;
       }
+    return LSMF_OK;
+  }
+  // shared nodes by the number of tiles that touch them, in node order
+  std::vector<uint32_t> where(mesh->n_nodes, 0);  // position within its group
+  size_t count[9] = {};
+  for (int node = 0; node < mesh->n_nodes; ++node) {
+    const int m = __builtin_popcount(cols[node]);
+    where[node] = (uint32_t)count[m]++;
+  }
+  int group[9] = {};
+  size_t n_shared = 0, n_slots = 0;
+  op->n_sum_groups = 0;
+  for (int m = 2; m <= n_col; ++m) {
+    if (count[m] == 0) continue;
+    const int g = group[m] = op->n_sum_groups++;
+    op->sum_begin[g] = (int)n_shared;
+    op->sum_mult[g] = m;
+    op->sum_first_slot[g] = n_slots;
+    n_shared += count[m];
+    n_slots += (size_t)m * count[m];
+  }
+  op->sum_begin[op->n_sum_groups] = (int)n_shared;
+  tt.sum_node.resize(n_shared);
+  tt.sum_slot.resize(n_slots);
+  tt.priv.assign((size_t)n_tiles * tw, 0);
+  for (long long b = 0; b < n_tiles; ++b)
+    for (int l = 0; l < td.tn; ++l) {
+      uint32_t &code = tt.nodes[(size_t)b * td.tn + l];
+      if (code == kNoNode) continue;
+      const uint32_t node = code, c = cols[node], below = c & ((1u << tcol[b]) - 1u);
+      code |= cons_bits(node);
+      const int m = __builtin_popcount(c);
+      if (m == 1) {
+        tt.priv[(size_t)b * tw + l / 32] |= 1u << (l % 32);
+      } else {
+        // this tile's place among the node's tiles, in colour order
+        const int g = group[m], k = __builtin_popcount(below);
+        if (k == 0) tt.sum_node[op->sum_begin[g] + where[node]] = code;
+        tt.sum_slot[op->sum_first_slot[g] + (size_t)k * count[m] + where[node]] = (uint32_t)(b * td.tn + l);
+      }
+      if (!below) code |= kFirstBit;
+    }
   return LSMF_OK;
 }
 
@@ -607,73 +705,12 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
   };
   std::vector<int> wbuf;
 
-  // --- colouring (given, checked below, or greedy first fit)
-  std::vector<int> colour(nc, 0);
-  if (mesh->cell_colour) {
-    for (int c = 0; c < nc; ++c) {
-      colour[c] = mesh->cell_colour[c];
-      if (colour[c] < 0 || colour[c] > 63) {
-        delete op;
-        return fail(LSMF_ERR_INVALID_ARGUMENT, "lsmf_op_create: colour out of [0, 63]");
-      }
-    }
-  } else {
-    std::vector<uint64_t> used(mesh->n_nodes, 0);
-    for (int c = 0; c < nc; ++c) {
-      write_nodes(c, wbuf);
-      uint64_t m = 0;
-      for (int n : wbuf) m |= used[n];
-      int col = 0;
-      while (col < 64 && (m >> col) & 1ull) ++col;
-      if (col == 64) {
-        delete op;
-        return fail(LSMF_ERR_INVALID_ARGUMENT, "lsmf_op_create: greedy colouring needs more than 64 colours");
-      }
-      colour[c] = col;
-      for (int n : wbuf) used[n] |= (1ull << col);
-    }
-  }
-  std::vector<int> min_col;
-  int n_col = 0;
-  for (int c = 0; c < nc; ++c) n_col = std::max(n_col, colour[c] + 1);
-  op->colour_ptr.assign(n_col + 1, 0);
-  for (int c = 0; c < nc; ++c) op->colour_ptr[colour[c] + 1]++;
-  for (int k = 0; k < n_col; ++k) op->colour_ptr[k + 1] += op->colour_ptr[k];
-  op->perm.assign(nc, 0);
-  op->inv_perm.assign(nc, 0);
-  {
-    std::vector<int> fill(op->colour_ptr.begin(), op->colour_ptr.end() - 1);
-    for (int c = 0; c < nc; ++c) {
-      const int pos = fill[colour[c]]++;
-      op->perm[pos] = c;
-      op->inv_perm[c] = pos;
-    }
-  }
-  // colour conflict check: no node written by two cells of one colour; min
-  // colour per node
-  std::vector<int> stamp(mesh->n_nodes, -1), stamp_cell(mesh->n_nodes, -1);
-  min_col.assign(mesh->n_nodes, 1 << 30);
-  for (int k = 0; k < n_col; ++k)
-    for (int pos = op->colour_ptr[k]; pos < op->colour_ptr[k + 1]; ++pos) {
-      const int c = op->perm[pos];
-      write_nodes(c, wbuf);
-      for (int nd : wbuf) {
-        if (stamp[nd] == k && stamp_cell[nd] != c) {
-          delete op;
-          return fail(LSMF_ERR_INVALID_ARGUMENT, "lsmf_op_create: two cells of one colour share a node");
-        }
-        stamp[nd] = k;
-        stamp_cell[nd] = c;
-        min_col[nd] = std::min(min_col[nd], k);
-      }
-    }
   op->curved = p > 1 && support_points_curved(mesh, dim, p, nqp);
   op->affine = cells_affine(mesh, dim, p, nqp);
   op->n_fields = n_cache_fields(op);
-  // --- cell order of the tiled layout (structured meshes) replaces the
-  // colour order; the per-cell index table then carries no first-touch bits
-  std::vector<uint32_t> tnodes;
-  std::vector<int32_t> tinfo;
+  // --- cell order of the tiled layout (structured meshes), else by colour;
+  // the per-cell index table of tiles carries no first-touch bits
+  TileTables tt;
   long long sn[3] = {1, 1, 1};
   std::vector<int32_t> cell_at;
   op->tiled = opt->layout == LSMF_LAYOUT_AUTO && nnc == 0 && cell_grid(mesh, dim, p, nqp, sn, cell_at);
@@ -684,19 +721,72 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
                       ? kTileWide
                       : 1;
   if (op->tiled) {
-    const std::vector<int> perm0 = op->perm, inv0 = op->inv_perm;
-    const int rc = build_tiles(op, mesh, sn, cell_at, tnodes, tinfo);
-    if (rc == kNotTileable) {  // the colour order of the cells layout stays
+    const int rc = build_tiles(op, mesh, sn, cell_at, tt);
+    if (rc == kNotTileable) {  // the cells layout
       op->tiled = false;
       op->tile_kind = 0;
-      op->perm = perm0;
-      op->inv_perm = inv0;
       op->tile_ptr.clear();
-      tnodes.clear();
-      tinfo.clear();
+      op->n_sum_groups = 0;
+      tt = TileTables();
     } else if (rc) {
       delete op;
       return rc;
+    }
+  }
+  // --- colouring (given and checked, or greedy first fit): no node is written
+  // by two cells of one colour; used[n] = colours of the cells that write n.
+  // Tiles need none, but a given one is checked for them too.
+  const bool colouring = !op->tiled || mesh->cell_colour;
+  std::vector<int> colour(colouring ? nc : 0, 0);
+  std::vector<uint64_t> used(mesh->n_nodes, 0);
+  for (int c = 0; c < nc; ++c) {
+    write_nodes(c, wbuf);
+    if (!colouring) {
+      for (int n : wbuf) used[n] = 1;
+      continue;
+    }
+    uint64_t m = 0;
+    for (int n : wbuf) m |= used[n];
+    int col = 0;
+    if (mesh->cell_colour) {
+      col = mesh->cell_colour[c];
+      if (col < 0 || col > 63) {
+        delete op;
+        return fail(LSMF_ERR_INVALID_ARGUMENT, "lsmf_op_create: colour out of [0, 63]");
+      }
+      if ((m >> col) & 1ull) {
+        delete op;
+        return fail(LSMF_ERR_INVALID_ARGUMENT, "lsmf_op_create: two cells of one colour share a node");
+      }
+    } else {
+      while (col < 64 && (m >> col) & 1ull) ++col;
+      if (col == 64) {
+        delete op;
+        return fail(LSMF_ERR_INVALID_ARGUMENT, "lsmf_op_create: greedy colouring needs more than 64 colours");
+      }
+    }
+    colour[c] = col;
+    for (int n : wbuf) used[n] |= (1ull << col);
+  }
+  std::vector<int> min_col;
+  if (!op->tiled) {
+    min_col.assign(mesh->n_nodes, 1 << 30);
+    for (int n = 0; n < mesh->n_nodes; ++n)
+      if (used[n]) min_col[n] = __builtin_ctzll(used[n]);
+    int n_col = 0;
+    for (int c = 0; c < nc; ++c) n_col = std::max(n_col, colour[c] + 1);
+    op->colour_ptr.assign(n_col + 1, 0);
+    for (int c = 0; c < nc; ++c) op->colour_ptr[colour[c] + 1]++;
+    for (int k = 0; k < n_col; ++k) op->colour_ptr[k + 1] += op->colour_ptr[k];
+    op->perm.assign(nc, 0);
+    op->inv_perm.assign(nc, 0);
+    {
+      std::vector<int> fill(op->colour_ptr.begin(), op->colour_ptr.end() - 1);
+      for (int c = 0; c < nc; ++c) {
+        const int pos = fill[colour[c]]++;
+        op->perm[pos] = c;
+        op->inv_perm[c] = pos;
+      }
     }
   }
   // --- index table (sorted cells): node | constraint bits | first-touch bit
@@ -724,13 +814,9 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
   // DoFs of nodes that no cell references: their rows are zero, and the
   // first-touch stores never write them
   std::vector<int32_t> orphan;
-  {
-    std::vector<uint8_t> used(mesh->n_nodes, 0);
-    for (size_t i = 0; i < (size_t)nc * nqp; ++i) used[mesh->cell_nodes[i]] = 1;
-    for (int nd = 0; nd < mesh->n_nodes; ++nd)
-      if (!used[nd])
-        for (int c = 0; c < dim; ++c) orphan.push_back(nd * dim + c);
-  }
+  for (int nd = 0; nd < mesh->n_nodes; ++nd)
+    if (!used[nd])
+      for (int c = 0; c < dim; ++c) orphan.push_back(nd * dim + c);
   op->n_orphan = (int)orphan.size();
 
   // --- node-constraint tables: instances and their masters (products), and
@@ -865,6 +951,10 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
   for (int i = 0; i < 2 * N * N; ++i) op->h_sf[i] = tab[i];
   for (int k = 0; k < (N + 1) / 2; ++k) op->h_qw[k] = t1.qw[k];
 
+  // the tile tables in one piece: tiles by colour, private bits, shared nodes, slots
+  std::vector<uint32_t> tile_tables(tt.list.begin(), tt.list.end());
+  for (const auto *v : {&tt.priv, &tt.sum_node, &tt.sum_slot}) tile_tables.insert(tile_tables.end(), v->begin(), v->end());
+
   const size_t es = elem_size(op);
   int rc = 0;
   if ((rc = dalloc(&op->d_idx, idx.size(), "index table")) ||
@@ -883,8 +973,9 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
       (rc = dalloc(&op->d_cons, cons.size(), "constrained list")) || (rc = dalloc(&op->d_bad, 1, "counter")) ||
       (rc = dalloc(&op->d_orphan, orphan.size(), "unreferenced DoFs")) ||
       (rc = dalloc(&op->d_perm, (size_t)nc, "cell permutation")) ||
-      (rc = dalloc(&op->d_tile_nodes, tnodes.size(), "tile nodes")) ||
-      (rc = dalloc(&op->d_tile_info, tinfo.size(), "tile info")) ||
+      (rc = dalloc(&op->d_tile_nodes, tt.nodes.size(), "tile nodes")) ||
+      (rc = dalloc(&op->d_tile_info, tt.info.size(), "tile info")) ||
+      (rc = dalloc(&op->d_tile_tables, tile_tables.size(), "tile tables")) ||
       (nnc > 0 && ((rc = dalloc(&op->d_hang, hang_tab.size(), "constraint table")) ||
                    (rc = dalloc(&op->d_hptr, hptr.size(), "constraint offsets")) ||
                    (rc = dalloc(&op->d_hmaster, hmaster.size(), "constraint masters")) ||
@@ -915,6 +1006,17 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
     delete op;
     return rc;
   }
+  if (!tt.priv.empty()) {
+    // without this memory the coloured launches serve every product
+    const size_t bytes = tt.nodes.size() * dim * es;
+    if (hipMalloc(&op->d_tile_buf, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      op->d_tile_buf = nullptr;
+    } else {
+      op->bytes_sum = bytes;
+    }
+  }
+  op->bytes_sum += tile_tables.size() * sizeof(uint32_t);
   op->bytes_idx = idx.size() * sizeof(uint32_t);
   op->bytes_cache = cache_bytes(op);
   hipError_t e = hipSuccess;
@@ -935,10 +1037,17 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
   if (e == hipSuccess && !orphan.empty())
     e = hipMemcpy(op->d_orphan, orphan.data(), orphan.size() * sizeof(int32_t), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(op->d_perm, op->perm.data(), (size_t)nc * sizeof(int32_t), hipMemcpyHostToDevice);
-  if (e == hipSuccess && !tnodes.empty())
-    e = hipMemcpy(op->d_tile_nodes, tnodes.data(), tnodes.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
-  if (e == hipSuccess && !tinfo.empty())
-    e = hipMemcpy(op->d_tile_info, tinfo.data(), tinfo.size() * sizeof(int32_t), hipMemcpyHostToDevice);
+  if (e == hipSuccess && !tt.nodes.empty())
+    e = hipMemcpy(op->d_tile_nodes, tt.nodes.data(), tt.nodes.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
+  if (e == hipSuccess && !tt.info.empty())
+    e = hipMemcpy(op->d_tile_info, tt.info.data(), tt.info.size() * sizeof(int32_t), hipMemcpyHostToDevice);
+  if (e == hipSuccess && !tile_tables.empty()) {
+    e = hipMemcpy(op->d_tile_tables, tile_tables.data(), tile_tables.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
+    op->d_tile_list = reinterpret_cast<const int32_t *>(op->d_tile_tables);
+    op->d_tile_priv = op->d_tile_tables + tt.list.size();
+    op->d_sum_node = op->d_tile_priv + tt.priv.size();
+    op->d_sum_slot = op->d_sum_node + tt.sum_node.size();
+  }
   if (e == hipSuccess && nnc > 0) {
     e = hipMemcpy(op->d_hang, hang_tab.data(), hang_tab.size() * sizeof(int32_t), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(op->d_hptr, hptr.data(), hptr.size() * sizeof(int32_t), hipMemcpyHostToDevice);
@@ -985,7 +1094,7 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
       up(op->d_dtw, wf.data(), wf.size() * sizeof(float));
     }
   }
-  op->bytes_idx += tnodes.size() * sizeof(uint32_t) + tinfo.size() * sizeof(int32_t);
+  op->bytes_idx += tt.nodes.size() * sizeof(uint32_t) + tt.info.size() * sizeof(int32_t);
   if (e != hipSuccess) {
     free_op(op);
     delete op;
@@ -1180,7 +1289,7 @@ size_t lsmf_op_size(const lsmf_op *op) { return op ? op->n_dofs : 0; }
 size_t lsmf_memory_consumption(const lsmf_op *op) {
   if (!op) return 0;
   const size_t es = elem_size(op);
-  size_t b = op->bytes_cache + op->bytes_idx + 2 * (size_t)op->n_cells * es;
+  size_t b = op->bytes_cache + op->bytes_idx + op->bytes_sum + 2 * (size_t)op->n_cells * es;
   if (op->caching == LSMF_CACHING_SCALAR || op->caching == LSMF_CACHING_SCALAR_REFERENTIAL)
     b += op->n_dofs * es + (size_t)op->n_nodes * op->dim * sizeof(double);
   return b;

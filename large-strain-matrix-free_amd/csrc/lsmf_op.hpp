@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -83,14 +84,34 @@ struct lsmf_op {
   int *d_bad = nullptr;
   int32_t *d_perm = nullptr;        // sorted position -> mesh cell
   double *adj_dmu = nullptr, *adj_dlambda = nullptr;  // outputs of the running residual VJP
-  // tiled layout (structured meshes): tiles sorted by colour, tiles of colour
-  // k are [tile_ptr[k], tile_ptr[k+1]); each tile's cells are consecutive
-  // sorted cells
+  // tiled layout (structured meshes): tiles in grid order (x fastest); each
+  // tile's cells are consecutive sorted cells.  Tiles of colour k are entries
+  // [tile_ptr[k], tile_ptr[k+1]) of d_tile_list
   bool tiled = false;
   int tile_kind = 0;  // TILE argument of the cell kernels: 0 cells, 1 tiles, 2 wide tiles
   std::vector<int> tile_ptr;
   uint32_t *d_tile_nodes = nullptr;  // [n_tiles][TN] node | constraint bits | first-touch bit, or kNoNode
   int32_t *d_tile_info = nullptr;    // [n_tiles][2] first sorted cell, extents ex | ey << 8 | ez << 16
+  uint32_t *d_tile_tables = nullptr;  // the memory of the next four tables
+  const int32_t *d_tile_list = nullptr;  // tiles by colour
+  // products in one launch over all tiles (k_vmult with tbuf, k_tile_sum):
+  // private-node bits, the shared nodes and their slots, and the tiles' shares
+  // of them (d_tile_buf: nullptr when its memory could not be had)
+  const uint32_t *d_tile_priv = nullptr, *d_sum_node = nullptr, *d_sum_slot = nullptr;
+  void *d_tile_buf = nullptr;
+  int n_sum_groups = 0;
+  int sum_begin[9] = {}, sum_mult[8] = {};
+  size_t sum_first_slot[8] = {};
+  size_t bytes_sum = 0;
+  // d_tile_buf serves one stream: the first that asks for it, or the one the
+  // operator's owner binds (bind_stream); calls on any other stream, and
+  // captured ones unless the owner allows them, take the coloured launches,
+  // which share nothing.  The mutex keeps the two launches of a product
+  // together when threads share the stream.
+  mutable std::mutex ws_mu;
+  mutable bool ws_bound = false;
+  mutable hipStream_t ws_stream = nullptr;
+  bool ws_capture = false;
   // node (hanging) constraints: cells layout, all-add scatter after a zero
   // pass.  Instances
   // (cell, constrained node) leave their results in d_hbuf; the masters
@@ -120,6 +141,20 @@ struct lsmf_op {
 namespace lsmf {
 
 size_t elem_size(const lsmf_op *op);
+
+// The owner of an operator that runs it on one stream only, its graphs
+// included, gives it d_tile_buf on that stream, captured or not.
+void bind_stream(lsmf_op *op, hipStream_t s);
+
+// Holds d_tile_buf for the launches of one call on stream s, if it may.
+class TileBufferLock {
+ public:
+  TileBufferLock(const lsmf_op *op, hipStream_t s);
+  explicit operator bool() const { return lock_.owns_lock(); }
+
+ private:
+  std::unique_lock<std::mutex> lock_;
+};
 
 // launch entry points of one (dim, N) instantiation unit
 struct LaunchTable {

@@ -19,6 +19,8 @@
 
 namespace lsmf {
 
+void bind_stream(lsmf_op *op, hipStream_t s);  // lsmf_op.hpp
+
 struct HipError : std::runtime_error {
   int code;
   HipError(int c, const std::string &m) : std::runtime_error(m), code(c) {}
@@ -87,6 +89,7 @@ template <typename number> class NeoHookOperatorHIP {
     lsmf_op_options o{n_q_1d, sizeof(number) == 8 ? LSMF_FP64 : LSMF_FP32, caching};
     abi_check(lsmf_op_create(&mesh, &o, &op_), "NeoHookOperator::initialize");
     stream_ = s;
+    bind_stream(op_, s);  // this object's calls, graphs included, run on s
   }
   void set_formulation(int formulation) { abi_check(lsmf_set_formulation(op_, formulation), "set_formulation"); }
   void set_material(const double *mu, const double *lambda) {
