@@ -717,6 +717,30 @@ __device__ __forceinline__ void flux_times_kt(const T (&Q)[DIM][DIM], const T (&
     }
 }
 
+// W = K H K^T for symmetric H, W in Voigt order
+template <int DIM, typename T>
+__device__ __forceinline__ void symmetric_form(const T (&K)[DIM][DIM], const T *H, T *W) {
+  constexpr int NV = Voigt<DIM>::NV;
+  T KH[DIM][DIM];
+#pragma unroll
+  for (int d = 0; d < DIM; ++d)
+#pragma unroll
+    for (int j = 0; j < DIM; ++j) {
+      T s = K[d][0] * H[voigt_index<DIM>(0, j)];
+#pragma unroll
+      for (int i = 1; i < DIM; ++i) s = fma(K[d][i], H[voigt_index<DIM>(i, j)], s);
+      KH[d][j] = s;
+    }
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int d = voigt_first<DIM>(v), e = voigt_second<DIM>(v);
+    T s = KH[d][0] * K[e][0];
+#pragma unroll
+    for (int j = 1; j < DIM; ++j) s = fma(KH[d][j], K[e][j], s);
+    W[v] = s;
+  }
+}
+
 // tensor4: Q = g T + M : sym(g)   (cached T, M already carry JxW)
 template <int DIM, typename T>
 __device__ __forceinline__ void qp_tensor4(const T (&G)[DIM][DIM], const T *cch, T (&Phi)[DIM][DIM]) {
@@ -1950,11 +1974,12 @@ template <int DIM, int N, typename T, int VAR> __global__ void __launch_bounds__
 //                 = sum_q gamma.T.gamma + c1/2 (|gamma|^2 + gamma_c^2)
 //                          + c2 gamma_c^2               (tensor2 / scalar)
 // where s~ is the Voigt vector of sym(e_c (x) gamma) with doubled shears.
+// Cells layout: point by point, which also serves the weighted basis
+// functions of cells with constrained nodes; tiles: k_diagonal_tiles.
 // ------------------------------------------------------------------------
-template <int DIM, int N, typename T, int VAR, int TILE>
+template <int DIM, int N, typename T, int VAR>
 __global__ void __launch_bounds__(kWG) k_diagonal(const VmultParams<T> P) {
   using CS = CellShape<DIM, N>;
-  using TS = TileShape<DIM, N, tile_threads<TILE>()>;  // the layout's tiles (this kernel: 256 threads)
   constexpr int NQP = CS::NQP, CPW = CS::CPW, NB = CS::NB, NC = CS::NC;
   constexpr int NV = Voigt<DIM>::NV;
   // the scalar variant evaluates the tensor4 fields per point (either
@@ -1970,17 +1995,8 @@ __global__ void __launch_bounds__(kWG) k_diagonal(const VmultParams<T> P) {
   // the kinematic prologue's scratch (SF ping-pong, corners) is dead once the
   // per-point fields are written, so it shares the fields' region
   constexpr int QDN = CPW * NF * NQP > SFN + XN ? CPW * NF * NQP : SFN + XN;
-  // a tile of TC cells is done in ROUNDS rounds of CPW cells (3D Q4 tiles
-  // hold four cells, twice this kernel's); the per-lane results of all the
-  // tile's cells then live in their own region, with one round in the
-  // fields' region once those are dead
-  constexpr int TC = TILE ? TS::CPW : CPW;
-  constexpr int ROUNDS = (TC + CPW - 1) / CPW;
-  constexpr int RESN = ROUNDS > 1 ? TC * NQP * DIM : 0;  // TC cells' results
-  static_assert(ROUNDS > 1 || CPW * NQP * DIM <= QDN, "tile results fit the fields' region");
-  __shared__ T lds[QDN + TABN + RESN];
+  __shared__ T lds[QDN + TABN];
   T *qd_all = lds;
-  T *res = ROUNDS > 1 ? lds + QDN + TABN : lds;
   T *tab = lds + QDN;
   T *sf_all = lds;
   T *X_all = sf_all + SFN;
@@ -1990,22 +2006,8 @@ __global__ void __launch_bounds__(kWG) k_diagonal(const VmultParams<T> P) {
   const int i0 = r % N, i1 = (r / N) % N, i2 = (DIM == 3) ? r / (N * N) : 0;
   const int L = xcd_remap(blockIdx.x, gridDim.x);
   const bool on = slot < CPW;
-  const int tile = TILE && P.tlist ? P.tlist[P.cell_begin + L] : P.cell_begin + L;
-  int ex = 0, ey = 0, ez = 0;
-  for (int round = 0; round < ROUNDS; ++round) {
-  const int ts = round * CPW + slot;  // this lane's cell within the tile
-  int cell;
-  bool active;
-  if constexpr (TILE) {
-    const int first = P.tinfo[2 * (size_t)tile], ext = P.tinfo[2 * (size_t)tile + 1];
-    ex = ext & 0xff, ey = (ext >> 8) & 0xff, ez = ext >> 16;
-    const int sx = ts % TS::TX, sy = (ts / TS::TX) % TS::TY, sz = ts / (TS::TX * TS::TY);
-    active = on && ts < TC && sx < ex && sy < ey && sz < ez;
-    cell = first + sx + ex * (sy + ey * sz);
-  } else {
-    cell = P.cell_begin + L * CPW + slot;
-    active = on && (cell < P.cell_end);
-  }
+  const int cell = P.cell_begin + L * CPW + slot;
+  const bool active = on && (cell < P.cell_end);
   const int sl = slot < CPW ? slot : 0;
   T *qd = qd_all + sl * NF * NQP;
   uint32_t code = 0;
@@ -2057,7 +2059,7 @@ __global__ void __launch_bounds__(kWG) k_diagonal(const VmultParams<T> P) {
     }
   }
   lds_barrier();
-  if (!TILE && !active) return;  // the tiled layout's lanes all reach the sum below
+  if (!active) return;
   const T *S = tab, *D = tab + N * N;
   // reference gradient of the basis function of local node a at point q
   auto grad_ref = [&](int a, int q, T (&g)[DIM]) {
@@ -2141,34 +2143,32 @@ __global__ void __launch_bounds__(kWG) k_diagonal(const VmultParams<T> P) {
       for (int c = 0; c < DIM; ++c) acc[c] += geo + T(0.5) * c1 * (g2 + gam[c] * gam[c]) + c2 * gam[c] * gam[c];
     }
   };
-  if constexpr (!TILE) {
-    const int hc = P.dcell ? P.dcell[cell] : -1;
-    if (hc >= 0) {
-      // a cell with constrained nodes: per entry (a node the cell couples)
-      // the basis function is the weighted sum of local ones; results wait
-      // in dbuf for the gather that follows the colours
-      for (int e = P.deptr[hc] + r; e < P.deptr[hc + 1]; e += NQP) {
-        T acc[DIM];
+  const int hc = P.dcell ? P.dcell[cell] : -1;
+  if (hc >= 0) {
+    // a cell with constrained nodes: per entry (a node the cell couples)
+    // the basis function is the weighted sum of local ones; results wait
+    // in dbuf for the gather that follows the colours
+    for (int e = P.deptr[hc] + r; e < P.deptr[hc + 1]; e += NQP) {
+      T acc[DIM];
 #pragma unroll
-        for (int c = 0; c < DIM; ++c) acc[c] = T(0);
-        for (int q = 0; q < NQP; ++q) {
-          T gph[DIM];
+      for (int c = 0; c < DIM; ++c) acc[c] = T(0);
+      for (int q = 0; q < NQP; ++q) {
+        T gph[DIM];
 #pragma unroll
-          for (int d = 0; d < DIM; ++d) gph[d] = T(0);
-          for (int k = P.dtptr[e]; k < P.dtptr[e + 1]; ++k) {
-            T g[DIM];
-            grad_ref(P.dta[k], q, g);
-            const T w = P.dtw[k];
+        for (int d = 0; d < DIM; ++d) gph[d] = T(0);
+        for (int k = P.dtptr[e]; k < P.dtptr[e + 1]; ++k) {
+          T g[DIM];
+          grad_ref(P.dta[k], q, g);
+          const T w = P.dtw[k];
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) gph[d] = fma(w, g[d], gph[d]);
-          }
-          point(q, gph, acc);
+          for (int d = 0; d < DIM; ++d) gph[d] = fma(w, g[d], gph[d]);
         }
-#pragma unroll
-        for (int c = 0; c < DIM; ++c) P.dbuf[(size_t)e * DIM + c] = acc[c];
+        point(q, gph, acc);
       }
-      return;
+#pragma unroll
+      for (int c = 0; c < DIM; ++c) P.dbuf[(size_t)e * DIM + c] = acc[c];
     }
+    return;
   }
   T acc[DIM];
 #pragma unroll
@@ -2178,53 +2178,269 @@ __global__ void __launch_bounds__(kWG) k_diagonal(const VmultParams<T> P) {
     grad_ref(r, q, gph);
     point(q, gph, acc);
   }
-  if constexpr (TILE) {
-    lds_barrier();  // every lane is done with the per-point fields
-    if (on)
+  const size_t node = code & kNodeMask;
 #pragma unroll
-      for (int c = 0; c < DIM; ++c)
-        if (ts < TC) res[(ts * NQP + r) * DIM + c] = active ? acc[c] : T(0);
-    lds_barrier();
+  for (int c = 0; c < DIM; ++c) {
+    if ((code >> (kConsShift + c)) & 1u) continue;
+    T *d = P.dst + node * DIM + c;
+    if (code & kFirstBit) *d = acc[c];
+    else *d += acc[c];
+  }
+}
+
+// ------------------------------------------------------------------------
+// exact diagonal on tiles, sum-factorized.  For every variant the entry of
+// local DoF (a, c) is a quadratic form of the reference gradient h of phi_a,
+//   A_(a,c),(a,c) = sum_q h^T W^c(q) h,
+//   compact          W^c = A + (c + 2 lambda) dw k k^T,  k = column c of K
+//   tensor2          W^c = K (T + c1/2 I) K^T + (c1/2 + c2) k k^T
+//   tensor4, scalar  W^c = K H K^T,  H_ij = T_ij + M_(ci)(cj)
+//   tensor4_ns       W^c = K H K^T,  H_ij = A_(ci)(cj)  (K = J_ref^-1)
+// and h_d h_e at q is a product over the directions f of the squared 1D
+// tables S S, S D or D D, so the DIM (DIM + 1) / 2 fields of W^c integrate in
+// three 1D passes: 15 N multiply-adds per point and component in 3D where the
+// sum over (basis function, point) pairs took about 30 N^3.
+// One lane per 1D line of all fields of a component; bound by the FP64 / LDS
+// work of the passes (the cache is read once).  All tiles: 48^3 Q2 FP64 432 ->
+// 135 us, 32^3 Q4 FP32 930 -> 140 us; FP32 error against 64 bits 2.0e-7 ->
+// 1.5e-7, FP64 unchanged.
+// ------------------------------------------------------------------------
+template <int DIM, int N, typename T, int VAR, int TILE>
+__global__ void __launch_bounds__(tile_threads<TILE>()) k_diagonal_tiles(const VmultParams<T> P) {
+  constexpr int WG = tile_threads<TILE>();
+  using TS = TileShape<DIM, N, WG>;
+  constexpr int NQP = ipow(N, DIM), CPW = TS::CPW, TN = TS::TN, NV = Voigt<DIM>::NV, NL = NQP / N;
+  constexpr int D2 = DIM * DIM, NC = 1 << DIM;
+  constexpr bool KIN = VAR == V_SCALAR;
+  // per cell: NV fields of each component (V_SCALAR first needs its
+  // kinematics' sum-factorization buffers there)
+  constexpr int ARR = KIN && DIM == 2 ? 2 * D2 : DIM * NV;
+  constexpr int SLOT = ARR * NQP;
+  constexpr int TABN = 4 * N * N + 2 * N;
+  __shared__ T lds[CPW * SLOT];
+  __shared__ T tab[TABN];
+  __shared__ T sq[3 * N * N];  // S S, S D, D D by [a][q]
+  __shared__ T X_all[KIN ? CPW * NC * DIM : 1];
+  const int t = threadIdx.x;
+  for (int k = t; k < TABN; k += WG) tab[k] = P.tab[k];
+  for (int k = t; k < N * N; k += WG) {
+    const T s = P.tab[2 * N * N + k], d = P.tab[3 * N * N + k];
+    sq[k] = s * s;
+    sq[N * N + k] = s * d;
+    sq[2 * N * N + k] = d * d;
+  }
+  const int slot = t / NQP, r = t - slot * NQP;
+  const int i0 = r % N, i1 = (r / N) % N, i2 = (DIM == 3) ? r / (N * N) : 0;
+  const bool on = slot < CPW;
+  const int sl = on ? slot : 0;
+  const int L = xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = P.tlist ? P.tlist[P.cell_begin + L] : P.cell_begin + L;
+  const int first = P.tinfo[2 * (size_t)tile], ext = P.tinfo[2 * (size_t)tile + 1];
+  const int ex = ext & 0xff, ey = (ext >> 8) & 0xff, ez = ext >> 16;
+  const int sx = slot % TS::TX, sy = (slot / TS::TX) % TS::TY, sz = slot / (TS::TX * TS::TY);
+  const bool active = on && sx < ex && sy < ey && sz < ez;
+  const int cell = active ? first + sx + ex * (sy + ey * sz) : first;
+  const size_t cq = (size_t)cell * NQP + (on ? r : 0);
+  T *A = lds + sl * SLOT;
+
+  // K and per component the symmetric H with W^c = K H K^T, or W^c itself
+  T K[DIM][DIM], base[NV], M[VAR == V_TENSOR4 || KIN ? NV * (NV + 1) / 2 : VAR == V_TENSOR4_NS ? D2 * (D2 + 1) / 2 : 1];
+  T kk = T(0);
+  if constexpr (KIN) {
+    uint32_t code = 0;
+    if (active) code = P.idx[cq];
+    lds_barrier();  // tab
+    T F[DIM][DIM], Jri[DIM][DIM], detJr, Gu[DIM][DIM], GX[DIM][DIM];
+    T *B = A + D2 * NQP;
+    T *Xc = X_all + sl * NC * DIM;
+    kinematics_prologue<DIM, N, T>(P, tab, A, B, Xc, on, active, code, r, i0, i1, i2, F, Jri, detJr, Gu);
+    if (P.curved)
+      geometry_gradient<DIM, N, T, false>(P.coords, P.sf, tab, lds, A, B, on, active, code, t, slot, r, i0, i1, i2,
+                                          GX);
+    const T m = P.mu[cell], l = P.lambda[cell];
+    T Fi[DIM][DIM];
+    const T J = inverse<DIM>(F, Fi);
+    const T *qw = tab + 4 * N * N + N;
+    const T w = (DIM == 3) ? qw[i0] * qw[i1] * qw[i2] : qw[i0] * qw[i1];
+    T dw = detJr * w;
+    if (P.curved)
+      eulerian_metric<DIM, T>(GX, Gu, J, w, K, dw);
+    else
+      grad_times<DIM>(Jri, Fi, K);
+    tensor4_fields<DIM, T>(F, J, m, l, dw, P.formulation, base, M);
   } else {
-    const size_t node = code & kNodeMask;
+    constexpr int NFC = CacheFields<DIM, VAR>::value;
+    T v[NFC];
+    load_cache<T, NFC>(P.cache, cq, P.fs, v);
 #pragma unroll
-    for (int c = 0; c < DIM; ++c) {
-      if ((code >> (kConsShift + c)) & 1u) continue;
-      T *d = P.dst + node * DIM + c;
-      if (code & kFirstBit) *d = acc[c];
-      else *d += acc[c];
+    for (int d = 0; d < DIM; ++d)
+#pragma unroll
+      for (int j = 0; j < DIM; ++j) K[d][j] = v[d * DIM + j];
+    if constexpr (VAR == V_COMPACT) {
+      kk = v[D2] + v[D2 + 1];
+#pragma unroll
+      for (int k = 0; k < NV; ++k) base[k] = v[D2 + 2 + k];
+    } else if constexpr (VAR == V_COMPACT_AFFINE) {
+      double w = weight_1d<N>(P.qw, i0) * weight_1d<N>(P.qw, i1);
+      if constexpr (DIM == 3) w *= weight_1d<N>(P.qw, i2);
+      const double *ca = P.caff + (size_t)cell * kAffineStride;
+      kk = v[D2] + T(ca[0] * w);
+#pragma unroll
+      for (int k = 0; k < NV; ++k) base[k] = T(ca[1 + k] * w);
+    } else if constexpr (VAR == V_TENSOR2) {
+      const T c1 = v[D2 + NV], c2 = v[D2 + NV + 1];
+      kk = T(0.5) * c1 + c2;
+      T Tv[NV];
+#pragma unroll
+      for (int k = 0; k < NV; ++k) Tv[k] = v[D2 + k] + (k < DIM ? T(0.5) * c1 : T(0));
+      symmetric_form<DIM>(K, Tv, base);
+    } else {
+      constexpr int NM = sizeof(M) / sizeof(M[0]);
+#pragma unroll
+      for (int k = 0; k < NV; ++k) base[k] = VAR == V_TENSOR4 ? v[D2 + k] : T(0);
+#pragma unroll
+      for (int k = 0; k < NM; ++k) M[k] = v[NFC - NM + k];
     }
   }
-  }  // rounds
-  if constexpr (TILE) {
-    for (int nd = t; nd < TS::TN; nd += kWG) {
-      const uint32_t tcode = P.tnodes[(size_t)tile * TS::TN + nd];
-      if (tcode != kNoNode) {
-        const int X = nd % TS::NX, Y = (nd / TS::NX) % TS::NY, Z = nd / (TS::NX * TS::NY);
-        constexpr int PP = N - 1;
-        T sum[DIM];
+  if (on) {
 #pragma unroll
-        for (int c = 0; c < DIM; ++c) sum[c] = T(0);
-        const int zlo = Z == 0 ? 0 : (Z - 1) / PP, zhi = min(Z / PP, ez - 1);
-        const int ylo = Y == 0 ? 0 : (Y - 1) / PP, yhi = min(Y / PP, ey - 1);
-        const int xlo = X == 0 ? 0 : (X - 1) / PP, xhi = min(X / PP, ex - 1);
-        for (int cz = zlo; cz <= zhi; ++cz)
-          for (int cy = ylo; cy <= yhi; ++cy)
-            for (int cx = xlo; cx <= xhi; ++cx) {
-              const int rr = (X - cx * PP) + N * ((Y - cy * PP) + N * (Z - cz * PP));
-              const int lane = (cx + TS::TX * (cy + TS::TY * cz)) * NQP + rr;
+    for (int c = 0; c < DIM; ++c) {
+      T W[NV];
+      if constexpr (VAR == V_TENSOR4 || VAR == V_TENSOR4_NS || KIN) {
+        T H[NV];
 #pragma unroll
-              for (int c = 0; c < DIM; ++c) sum[c] += res[lane * DIM + c];
-            }
-        const size_t tnode = tcode & kNodeMask;
-#pragma unroll
-        for (int c = 0; c < DIM; ++c) {
-          if ((tcode >> (kConsShift + c)) & 1u) continue;
-          T *d = P.dst + tnode * DIM + c;
-          if (tcode & kFirstBit) *d = sum[c];
-          else *d += sum[c];
+        for (int v = 0; v < NV; ++v) {
+          const int i = voigt_first<DIM>(v), j = voigt_second<DIM>(v);
+          H[v] = base[v] + (VAR == V_TENSOR4_NS ? M[sym_index<D2>(c * DIM + i, c * DIM + j)]
+                                                : M[sym_index<NV>(voigt_index<DIM>(c, i), voigt_index<DIM>(c, j))]);
         }
+        symmetric_form<DIM>(K, H, W);
+      } else {
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+          W[v] = fma(kk * K[voigt_first<DIM>(v)][c], K[voigt_second<DIM>(v)][c], base[v]);
       }
+      // the off-diagonal entries count twice
+#pragma unroll
+      for (int v = 0; v < NV; ++v) A[(c * NV + v) * NQP + r] = active ? (v < DIM ? W[v] : T(2) * W[v]) : T(0);
+    }
+  }
+  lds_barrier();
+
+  // y[a] (+)= sum_q tab[a][q] x[q]
+  const T *SS = sq, *SD = sq + N * N, *DD = sq + 2 * N * N;
+  auto apply = [](const T *m, const T (&x)[N], T (&y)[N], bool add) {
+#pragma unroll
+    for (int a = 0; a < N; ++a) {
+      T s = add ? fma(m[a * N], x[0], y[a]) : m[a * N] * x[0];
+#pragma unroll
+      for (int q = 1; q < N; ++q) s = fma(m[a * N + q], x[q], s);
+      y[a] = s;
+    }
+  };
+  constexpr int TASKS = CPW * DIM * NL;
+  auto field = [&](int task, int &l) {  // fields of (cell, component), line l
+    const int sc = task / NL;
+    l = task - sc * NL;
+    return lds + (sc / DIM) * SLOT + (sc % DIM) * NV * NQP;
+  };
+  if constexpr (DIM == 3) {
+    // z, in place: field (d, e) with D D, S D or S S as z occurs in it
+#pragma unroll 1
+    for (int task = t; task < TASKS; task += WG) {
+      int l;
+      T *p = field(task, l) + l;
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        T x[N], y[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) x[k] = p[v * NQP + k * NL];
+        apply(v == 2 ? DD : v >= 4 ? SD : SS, x, y, false);
+#pragma unroll
+        for (int k = 0; k < N; ++k) p[v * NQP + k * NL] = y[k];
+      }
+    }
+    lds_barrier();
+  }
+  // y: what x multiplies by D D, S S and S D into arrays 0, 1, 2
+#pragma unroll 1
+  for (int task = t; task < TASKS; task += WG) {
+    int l;
+    T *p = field(task, l) + (l % N) + (DIM == 3 ? N * N * (l / N) : 0);
+    T x[N], y[3][N];
+    auto line = [&](int v) {
+#pragma unroll
+      for (int k = 0; k < N; ++k) x[k] = p[v * NQP + k * N];
+    };
+    line(0);
+    apply(SS, x, y[0], false);
+    line(1);
+    apply(DD, x, y[1], false);
+    if constexpr (DIM == 3) {
+      line(2);
+      apply(SS, x, y[1], true);
+      line(5);
+      apply(SD, x, y[1], true);
+      line(3);
+      apply(SD, x, y[2], false);
+      line(4);
+      apply(SS, x, y[2], true);
+    } else {
+      line(2);
+      apply(SD, x, y[2], false);
+    }
+#pragma unroll
+    for (int v = 0; v < 3; ++v)
+#pragma unroll
+      for (int k = 0; k < N; ++k) p[v * NQP + k * N] = y[v][k];
+  }
+  lds_barrier();
+  // x: the entries into array 0
+#pragma unroll 1
+  for (int task = t; task < TASKS; task += WG) {
+    int l;
+    T *p = field(task, l) + l * N;
+    T x[N], y[N];
+#pragma unroll
+    for (int v = 0; v < 3; ++v) {
+#pragma unroll
+      for (int k = 0; k < N; ++k) x[k] = p[v * NQP + k];
+      apply(v == 0 ? DD : v == 1 ? SS : SD, x, y, v > 0);
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) p[k] = y[k];
+  }
+  lds_barrier();
+  for (int nd = t; nd < TN; nd += WG) {
+    const uint32_t tcode = P.tnodes[(size_t)tile * TN + nd];
+    if (tcode == kNoNode) continue;
+    const int X = nd % TS::NX, Y = (nd / TS::NX) % TS::NY, Z = nd / (TS::NX * TS::NY);
+    constexpr int PP = N - 1;
+    T sum[DIM];
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) sum[c] = T(0);
+    const int zlo = Z == 0 ? 0 : (Z - 1) / PP, zhi = min(Z / PP, ez - 1);
+    const int ylo = Y == 0 ? 0 : (Y - 1) / PP, yhi = min(Y / PP, ey - 1);
+    const int xlo = X == 0 ? 0 : (X - 1) / PP, xhi = min(X / PP, ex - 1);
+    for (int cz = zlo; cz <= zhi; ++cz)
+      for (int cy = ylo; cy <= yhi; ++cy)
+        for (int cx = xlo; cx <= xhi; ++cx) {
+          const int rr = (X - cx * PP) + N * ((Y - cy * PP) + N * (Z - cz * PP));
+          const int s = cx + TS::TX * (cy + TS::TY * cz);
+#pragma unroll
+          for (int c = 0; c < DIM; ++c) sum[c] += lds[s * SLOT + c * NV * NQP + rr];
+        }
+    if (P.tbuf && !((P.tpriv[(size_t)tile * TS::TW + nd / 32] >> (nd % 32)) & 1u)) {
+      store_node<DIM, T>(P.tbuf + ((size_t)tile * TN + nd) * DIM, sum);
+      continue;
+    }
+    const size_t tnode = tcode & kNodeMask;
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) {
+      if ((tcode >> (kConsShift + c)) & 1u) continue;
+      T *d = P.dst + tnode * DIM + c;
+      if (P.tbuf || (tcode & kFirstBit)) *d = sum[c];
+      else *d += sum[c];
     }
   }
 }

@@ -117,40 +117,51 @@ template <int DIM, int N> struct Launch {
                        op->n_hang_masters);
   }
 
-  // all tiles in one launch, then the sums of the nodes they share (with
-  // CONSTR and identity also the constrained rows)
-  template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
-  static int run_tiles(const lsmf_op *op, T *dst, const T *src, int identity, hipStream_t s) {
+  // parameters of one launch over all tiles
+  template <typename T> static VmultParams<T> tile_params(const lsmf_op *op) {
     VmultParams<T> P = params<T>(op, 0);
-    P.src = src;
-    P.dst = dst;
     P.tlist = nullptr;
     P.cell_begin = 0;
     P.cell_end = op->tile_ptr.back();
     P.tpriv = op->d_tile_priv;
     P.tbuf = static_cast<T *>(op->d_tile_buf);
+    return P;
+  }
+
+  // the sums of the nodes that several tiles share, after such a launch
+  template <typename T, bool ADD, bool CONSTR>
+  static void tile_sum(const lsmf_op *op, T *dst, const T *src, int identity, hipStream_t s) {
+    const int n = op->sum_begin[op->n_sum_groups];
+    if (n == 0) return;
+    TileSumParams<T> S{};
+    S.node = op->d_sum_node;
+    S.slot = op->d_sum_slot;
+    S.buf = static_cast<const T *>(op->d_tile_buf);
+    S.src = src;
+    S.dst = dst;
+    S.identity = identity;
+    S.n_groups = op->n_sum_groups;
+    for (int g = 0; g < S.n_groups; ++g) {
+      S.begin[g] = op->sum_begin[g];
+      S.mult[g] = op->sum_mult[g];
+      S.first_slot[g] = op->sum_first_slot[g];
+    }
+    S.begin[S.n_groups] = n;
+    hipLaunchKernelGGL((k_tile_sum<DIM, T, ADD, CONSTR>), dim3((n + kWG - 1) / kWG), dim3(kWG), 0, s, S);
+  }
+
+  // all tiles in one launch, then the sums of the nodes they share (with
+  // CONSTR and identity also the constrained rows)
+  template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
+  static int run_tiles(const lsmf_op *op, T *dst, const T *src, int identity, hipStream_t s) {
+    VmultParams<T> P = tile_params<T>(op);
+    P.src = src;
+    P.dst = dst;
     P.identity = identity;
     if (op->prof) op->prof->before(s);
     const int rc = launch_vmult<T, VAR, ADD, CONSTR, PH>(op, P, P.cell_end, 1, s);
     if (rc) return rc;
-    const int n = op->sum_begin[op->n_sum_groups];
-    if (n > 0) {
-      TileSumParams<T> S{};
-      S.node = op->d_sum_node;
-      S.slot = op->d_sum_slot;
-      S.buf = P.tbuf;
-      S.src = src;
-      S.dst = dst;
-      S.identity = identity;
-      S.n_groups = op->n_sum_groups;
-      for (int g = 0; g < S.n_groups; ++g) {
-        S.begin[g] = op->sum_begin[g];
-        S.mult[g] = op->sum_mult[g];
-        S.first_slot[g] = op->sum_first_slot[g];
-      }
-      S.begin[S.n_groups] = n;
-      hipLaunchKernelGGL((k_tile_sum<DIM, T, ADD, CONSTR>), dim3((n + kWG - 1) / kWG), dim3(kWG), 0, s, S);
-    }
+    tile_sum<T, ADD, CONSTR>(op, dst, src, identity, s);
     if (op->prof) op->prof->after(s);
     return 0;
   }
@@ -355,26 +366,38 @@ template <int DIM, int N> struct Launch {
     if (op->n_node_cons > 0)
       hipLaunchKernelGGL(k_zero<T>, dim3((unsigned)((op->n_dofs + 255) / 256)), dim3(256), 0, s,
                          static_cast<T *>(op->d_diag), op->n_dofs);
-    const int nc = n_colours(op);
-    for (int k = 0; k < nc; ++k) {
-      VmultParams<T> P = params<T>(op, k);
+    auto cells = [&](VmultParams<T> P, int n) {
       P.dst = static_cast<T *>(op->d_diag);
       // scalar_referential shares the scalar kernel but integrates on the Q1
       // vertex map on any mesh (include/mf_nh_operator.h:1255-1400)
       if (op->caching == LSMF_CACHING_SCALAR_REFERENTIAL) P.curved = 0;
-      const int n = P.cell_end - P.cell_begin;
-      if (n <= 0) continue;
+      if (n <= 0) return 0;
       if (op->tile_kind == kTileWide) {
         if constexpr (wide_ok<VAR>())
-          hipLaunchKernelGGL((k_diagonal<DIM, N, T, VAR, kTileWide>), dim3(n), dim3(kWG), 0, s, P);
+          hipLaunchKernelGGL((k_diagonal_tiles<DIM, N, T, VAR, kTileWide>), dim3(n),
+                             dim3(tile_threads<kTileWide>()), 0, s, P);
         else
-          return LSMF_ERR_UNSUPPORTED;
+          return (int)LSMF_ERR_UNSUPPORTED;
       } else if (op->tile_kind == 1) {
-        hipLaunchKernelGGL((k_diagonal<DIM, N, T, VAR, 1>), dim3(n), dim3(kWG), 0, s, P);
+        hipLaunchKernelGGL((k_diagonal_tiles<DIM, N, T, VAR, 1>), dim3(n), dim3(kWG), 0, s, P);
       } else {
-        hipLaunchKernelGGL((k_diagonal<DIM, N, T, VAR, 0>), dim3(grid_for(n)), dim3(kWG), 0, s, P);
+        hipLaunchKernelGGL((k_diagonal<DIM, N, T, VAR>), dim3(grid_for(n)), dim3(kWG), 0, s, P);
+      }
+      return 0;
+    };
+    int rc = 0;
+    const TileBufferLock lock(op, s);
+    if (lock) {
+      const VmultParams<T> P = tile_params<T>(op);
+      rc = cells(P, P.cell_end);
+      if (!rc) tile_sum<T, false, true>(op, static_cast<T *>(op->d_diag), nullptr, 0, s);
+    } else {
+      for (int k = 0; k < n_colours(op) && !rc; ++k) {
+        const VmultParams<T> P = params<T>(op, k);
+        rc = cells(P, P.cell_end - P.cell_begin);
       }
     }
+    if (rc) return rc;
     T *diag = static_cast<T *>(op->d_diag);
     if (op->n_diag_nodes > 0)
       hipLaunchKernelGGL((k_hang_gather<DIM, T, true>), dim3((op->n_diag_nodes + 255) / 256), dim3(256), 0, s, diag,
