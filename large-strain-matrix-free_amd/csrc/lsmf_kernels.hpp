@@ -66,6 +66,7 @@ enum Variant {
   V_SCALAR_REF = 4,
   V_COMPACT = 5,  // tensor2 / tensor4 operators in compact form
   V_COMPACT_AFFINE = 6,
+  V_COMPACT_U = 7,  // affine cells, K from the displacement (k_vmult_planes)
   V_RESIDUAL = 100,
   V_ADJOINT = 101
 };
@@ -104,7 +105,8 @@ template <int NV> __host__ __device__ constexpr int sym_index(int v, int w) {
 //   scalar      c
 //   scalar_ref  c, u at the point (DIM)
 //   compact     K (D2), c dw, 2 lambda dw, A dw (NV); affine cells: K, c dw
-//               (A and 2 lambda det(J_ref) per cell, P.caff)
+//               (A and 2 lambda det(J_ref) per cell, P.caff), or c dw alone
+//               where the product takes K from the displacement
 template <int DIM, int VAR> struct CacheFields {
   static constexpr int NV = Voigt<DIM>::NV;
   static constexpr int D2 = DIM * DIM;
@@ -115,6 +117,7 @@ template <int DIM, int VAR> struct CacheFields {
                                : VAR == V_SCALAR     ? 1
                                : VAR == V_COMPACT    ? D2 + 2 + NV
                                : VAR == V_COMPACT_AFFINE ? D2 + 1
+                               : VAR == V_COMPACT_U ? 1
                                                      : 0;
 };
 
@@ -158,10 +161,10 @@ template <typename T, int NF> __device__ __forceinline__ void load_cache(const T
   }
 }
 
-// values per cell of the affine compact form: 2 lambda det(J_ref), then A (NV);
+// values per cell of the affine compact forms: 2 lambda det(J_ref), A (NV), J_ref (DIM^2);
 // FP64 also for FP32 operators, so that a point's values, the product with its
 // weight, are rounded once, as the stored ones are
-constexpr int kAffineStride = 8;
+constexpr int kAffineStride = 16;
 
 // 1D tables: S, D, St, Dt (N*N each), Gauss points and weights (N each),
 // then the collocation derivative on the Gauss points (N*N, used by
@@ -438,6 +441,8 @@ template <int DIM, int N, typename T> struct SF {
 // and the middle column C[r] = M[r][H], rows r < R = H + N % 2: about half
 // the multiply-adds and half the constants of the plain products.
 // Packed per matrix: E[R][H], O[R][H], C[R] (PK values).
+// For odd N the middle support point is the middle Gauss point, so S's middle
+// row is a unit vector, and for N = 3 D's is (-1, 0, 1): neither is multiplied.
 // ------------------------------------------------------------------------
 template <int N, typename T> struct EvenOdd {
   static constexpr int H = N / 2, ODD = N % 2, R = H + ODD, PK = R * (2 * H + 1);
@@ -472,9 +477,10 @@ template <int N, typename T> struct EvenOdd {
       y[N - 1 - q] = SIG > 0 ? ev - od : od - ev;
     }
     if constexpr (ODD) {
-      T v = SIG > 0 ? C(pk, H) * s.m : T(0);
+      T v = SIG > 0 ? s.m : N == 3 ? -s.o[0] : T(0);
+      if constexpr (SIG < 0 && N > 3)
 #pragma unroll
-      for (int k = 0; k < H; ++k) v = SIG > 0 ? fma(E(pk, H, k), s.e[k], v) : fma(O(pk, H, k), s.o[k], v);
+        for (int k = 0; k < H; ++k) v = fma(O(pk, H, k), s.o[k], v);
       y[H] = v;
     }
   }
@@ -484,8 +490,8 @@ template <int N, typename T> struct EvenOdd {
     for (int a = 0; a < H; ++a) {
       T u, w;
       if constexpr (SIG > 0) {
-        u = ODD ? E(pk, H, a) * s.m : T(0);  // even part
-        w = T(0);                            // odd part
+        u = T(0);  // even part
+        w = T(0);  // odd part
 #pragma unroll
         for (int q = 0; q < H; ++q) {
           u = fma(E(pk, q, a), s.e[q], u);
@@ -493,7 +499,7 @@ template <int N, typename T> struct EvenOdd {
         }
       } else {
         u = T(0);
-        w = ODD ? O(pk, H, a) * s.m : T(0);
+        w = !ODD ? T(0) : N == 3 ? -s.m : O(pk, H, a) * s.m;
 #pragma unroll
         for (int q = 0; q < H; ++q) {
           u = fma(E(pk, q, a), s.o[q], u);
@@ -504,7 +510,7 @@ template <int N, typename T> struct EvenOdd {
       y[N - 1 - a] = u - w;
     }
     if constexpr (ODD) {
-      T v = SIG > 0 ? C(pk, H) * s.m : T(0);
+      T v = SIG > 0 ? s.m : T(0);
 #pragma unroll
       for (int q = 0; q < H; ++q) v = fma(C(pk, q), SIG > 0 ? s.e[q] : s.o[q], v);
       y[H] = v;
@@ -871,14 +877,14 @@ __device__ __forceinline__ void qp_compact(const T (&G)[DIM][DIM], const T *K, T
   const T lt = ldw * tr;
 #pragma unroll
   for (int d = 0; d < DIM; ++d) {
-    T Y[DIM];  // row d of c dw X
+    T Y[DIM];  // row d of c dw X + lt I
 #pragma unroll
-    for (int e = 0; e < DIM; ++e) Y[e] = cdw * X[d][e];
+    for (int e = 0; e < DIM; ++e) Y[e] = e == d ? fma(cdw, X[d][e], lt) : cdw * X[d][e];
 #pragma unroll
     for (int c = 0; c < DIM; ++c) {
-      T s = lt * K[d * DIM + c];
+      T s = Y[0] * K[c];
 #pragma unroll
-      for (int e = 0; e < DIM; ++e) s = fma(Y[e], K[e * DIM + c], s);
+      for (int e = 1; e < DIM; ++e) s = fma(Y[e], K[e * DIM + c], s);
 #pragma unroll
       for (int e = 0; e < DIM; ++e) s = fma(G[c][e], A[voigt_index<DIM>(e, d)], s);
       Phi[c][d] = s;
@@ -1681,6 +1687,345 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
 }
 
 // ------------------------------------------------------------------------
+// Fused product of the compact forms on wide 3D tiles: planes and columns.
+//
+// k_vmult's line-per-lane passes go through LDS after every 1D operator: about
+// 100 LDS accesses per point and nine workgroup barriers, which bound the
+// compact forms (their cached stream is short).  Here a lane first takes a
+// plane of one component (N x N values at one z) and does x and y in
+// registers, then a column of N points (all components, three arrays each)
+// and does z, the tangent of its points and z transposed in registers, then
+// its plane again: 45 LDS accesses per point.  The lanes of a cell sit in one
+// wave, whose LDS accesses are in order, so only the tile's gather and the
+// final sums need workgroup barriers.
+// 128^3 Q2 FP32 1052 -> 916 us, 48^3 79 -> 63 us: bound by memory (4.2 TB/s).
+// FP64 with the cached stream only 1814 -> 1786 us, bound by memory too (7.7
+// GB); V_COMPACT_U recomputes K = (J_ref + Grad_xi u)^-1, 4.4 GB: 1705 us, and
+// with the padded slots 1620 us (LDS bank conflicts 135 -> 22 of 525 kcycles),
+// 1555 us without the unit rows of the 1D matrices.  What is left is issue:
+// VALU and LDS each busy about half the time, nine waves per CU.
+// ------------------------------------------------------------------------
+template <int N, typename T> struct PlaneShape {
+  // Q2: ten lanes (nine used) and a padded slot per cell, so that planes
+  // (lanes 9 values apart) and columns (neighbours) spread over all banks
+  static constexpr int LPC = N == 3 ? 10 : N * N;  // lanes per cell
+  static constexpr int CPV = 64 / LPC;             // cells per wave
+  static constexpr int CPW = TileShape<3, N, tile_threads<kTileWide>()>::CPW;
+  static constexpr int WAVES = (CPW + CPV - 1) / CPV;
+  static constexpr int WG = 64 * WAVES;
+  static constexpr int SLOT = N == 3 ? (sizeof(T) == 8 ? 250 : 266) : 9 * N * N * N;
+};
+// LDS order within a wave: the accesses of its lanes are in order in
+// hardware, this keeps the compiler to it
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int N, typename T> struct SFPlane {
+  static constexpr int NL = N * N, NQP = N * N * N;
+  using EO = EvenOdd<N, T>;
+  // plane x[y][x] of component c at height z -> arrays c (value), 3 + c (d/dx)
+  // and 6 + c (d/dy) of the cell's slot
+  static __device__ __forceinline__ void evaluate_plane(const T *sf, T *p, const T (&x)[N][N]) {
+    const T *S = sf, *D = sf + EO::PK;
+    T v[N][N], d[N][N];
+#pragma unroll
+    for (int y = 0; y < N; ++y) {
+      const typename EO::Split s = EO::split(x[y]);
+      EO::template fwd<1>(S, s, v[y]);
+      EO::template fwd<-1>(D, s, d[y]);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      T a[N], b[N], o[N];
+#pragma unroll
+      for (int y = 0; y < N; ++y) {
+        a[y] = v[y][i];
+        b[y] = d[y][i];
+      }
+      const typename EO::Split sa = EO::split(a), sb = EO::split(b);
+      auto put = [&](int e) {
+#pragma unroll
+        for (int y = 0; y < N; ++y) p[e * 3 * NQP + y * N + i] = o[y];
+      };
+      EO::template fwd<1>(S, sa, o);
+      put(0);
+      EO::template fwd<1>(S, sb, o);
+      put(1);
+      EO::template fwd<-1>(D, sa, o);
+      put(2);
+    }
+  }
+  // column at p (stride NL): gradient of component c at its N points
+  static __device__ __forceinline__ void evaluate_column(const T *sf, const T *p, T (&g)[3][N]) {
+    const T *S = sf, *D = sf + EO::PK;
+    T e[3][N];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int k = 0; k < N; ++k) e[a][k] = p[a * 3 * NQP + k * NL];
+    EO::template fwd<1>(S, EO::split(e[1]), g[0]);
+    EO::template fwd<1>(S, EO::split(e[2]), g[1]);
+    EO::template fwd<-1>(D, EO::split(e[0]), g[2]);
+  }
+  // z transposed of the fluxes f[d][k] of one component
+  static __device__ __forceinline__ void integrate_column(const T *sf, T *p, const T (&f)[3][N]) {
+    const T *S = sf, *D = sf + EO::PK;
+    T y[N];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      if (d < 2) EO::template tr<1>(S, EO::split(f[d]), y);
+      else EO::template tr<-1>(D, EO::split(f[d]), y);
+#pragma unroll
+      for (int k = 0; k < N; ++k) p[d * 3 * NQP + k * NL] = y[k];
+    }
+  }
+  // y and x transposed: the plane's results into array c
+  static __device__ __forceinline__ void integrate_plane(const T *sf, T *p) {
+    const T *S = sf, *D = sf + EO::PK;
+    T v[N][N], d[N][N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      T e[3][N], o[N], q[N];
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int y = 0; y < N; ++y) e[a][y] = p[a * 3 * NQP + y * N + i];
+      EO::template tr<1>(S, EO::split(e[2]), o);
+      EO::template tr<-1>(D, EO::split(e[1]), q);
+#pragma unroll
+      for (int y = 0; y < N; ++y) v[y][i] = o[y] + q[y];
+      EO::template tr<1>(S, EO::split(e[0]), o);
+#pragma unroll
+      for (int y = 0; y < N; ++y) d[y][i] = o[y];
+    }
+#pragma unroll
+    for (int y = 0; y < N; ++y) {
+      T o[N], q[N];
+      EO::template tr<1>(S, EO::split(v[y]), o);
+      EO::template tr<-1>(D, EO::split(d[y]), q);
+#pragma unroll
+      for (int i = 0; i < N; ++i) p[y * N + i] = o[i] + q[i];
+    }
+  }
+};
+
+// waves per SIMD
+template <int N, typename T> constexpr int planes_min_waves() { return sizeof(T) == 8 ? (N == 3 ? 3 : 2) : 4; }
+
+template <int N, typename T, int VAR, bool ADD, bool CONSTR>
+__global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T>())) k_vmult_planes(const VmultParams<T> P) {
+  static_assert(VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U);
+  constexpr bool AFFINE = VAR != V_COMPACT, RECOMP = VAR == V_COMPACT_U;
+  using PS = PlaneShape<N, T>;
+  using TS = TileShape<3, N, tile_threads<kTileWide>()>;
+  using SF3 = SFPlane<N, T>;
+  constexpr int NQP = N * N * N, NL = N * N, TN = TS::TN, WG = PS::WG, PP = N - 1;
+  constexpr int NF = CacheFields<3, VAR>::value;
+  constexpr int ROUNDS = (TN + WG - 1) / WG;
+  constexpr int NCA = RECOMP ? 16 : 7;  // constants per cell
+  constexpr int CA = AFFINE ? PS::CPW * NCA : 1;
+  constexpr int CROUNDS = (CA + WG - 1) / WG;
+  __shared__ T lds[PS::CPW * PS::SLOT];
+  __shared__ T tile_v[TN * 3];
+  __shared__ double caff_all[CA];
+  __shared__ T tile_u[RECOMP ? TN * 3 : 1];
+  const T *__restrict__ src = P.src + (size_t)blockIdx.y * P.vstride;
+  T *__restrict__ dst = P.dst + (size_t)blockIdx.y * P.vstride;
+  const int t = threadIdx.x, wave = t / 64, lane = t % 64;
+  const int L = xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = P.tlist ? P.tlist[P.cell_begin + L] : P.cell_begin + L;
+  const int first = P.tinfo[2 * (size_t)tile], ext = P.tinfo[2 * (size_t)tile + 1];
+  const int ex = ext & 0xff, ey = (ext >> 8) & 0xff, ez = ext >> 16;
+  // lane -> cell of the wave and its plane / column
+  const int wc = lane / PS::LPC, j = lane - wc * PS::LPC;
+  const int slot = wave * PS::CPV + wc;  // cell of the tile
+  const bool has = wc < PS::CPV && slot < ex * ey * ez;
+  const bool col = has && j < NL, pln = has && j < 3 * N;
+  const int cell = has ? first + slot : first;
+
+  // the tile's nodes: codes and source values, then what the final write
+  // adds to (see k_vmult); issued before the cached stream
+  uint32_t tcode[ROUNDS];
+  T sv[ROUNDS][3], dv[ROUNDS][3], uv[ROUNDS][3];
+  bool tshared[ROUNDS];
+#pragma unroll
+  for (int k = 0; k < ROUNDS; ++k) {
+    const int n = t + k * WG;
+    tcode[k] = n < TN ? P.tnodes[(size_t)tile * TN + n] : kNoNode;
+    tshared[k] = false;
+    if (P.tbuf) tshared[k] = !((P.tpriv[(size_t)tile * TS::TW + (n < TN ? n / 32 : 0)] >> (n % 32)) & 1u);
+  }
+#pragma unroll
+  for (int k = 0; k < ROUNDS; ++k) {
+    const bool valid = tcode[k] != kNoNode;
+    const size_t node = valid ? tcode[k] & kNodeMask : 0;
+    if constexpr (RECOMP) load_node<3, T>(P.u + node * 3, uv[k]);
+    load_node<3, T>(src + node * 3, sv[k]);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) dv[k][c] = T(0);
+    if (valid && (ADD ? !tshared[k] : !P.tbuf && !(tcode[k] & kFirstBit))) load_node<3, T>(dst + node * 3, dv[k]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // the cells' constants (consecutive cells) wait in LDS
+  const int n_ca = ex * ey * ez * NCA;
+  double ca[CROUNDS];
+  if constexpr (AFFINE)
+#pragma unroll
+    for (int k = 0; k < CROUNDS; ++k) {
+      const int i = t + k * WG < n_ca ? t + k * WG : 0;
+      ca[k] = P.caff[(size_t)(first + i / NCA) * kAffineStride + i % NCA];
+    }
+  __builtin_amdgcn_sched_barrier(0);
+  T cch[N][NF];
+  const size_t cq = (size_t)cell * NQP + (col ? j : 0);
+#pragma unroll
+  for (int k = 0; k < N; ++k) load_cache<T, NF>(P.cache, cq + k * NL, P.fs, cch[k]);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (AFFINE)
+#pragma unroll
+    for (int k = 0; k < CROUNDS; ++k)
+      if (t + k * WG < CA) caff_all[t + k * WG] = ca[k];
+#pragma unroll
+  for (int k = 0; k < ROUNDS; ++k) {
+    const int n = t + k * WG;
+    if (n < TN)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const bool zero = tcode[k] == kNoNode || (CONSTR && ((tcode[k] >> (kConsShift + c)) & 1u));
+        tile_v[n * 3 + c] = zero ? T(0) : sv[k][c];
+        if constexpr (RECOMP) tile_u[n * 3 + c] = uv[k][c];
+      }
+  }
+  lds_barrier();
+  T *A = lds + (has ? slot : 0) * PS::SLOT;
+  const int pc = j / N, pz = j - pc * N;  // plane: component, height
+  T *plane = A + pc * NQP + pz * NL;
+  const int sx = slot % ex, sy = (slot / ex) % ey, sz = slot / (ex * ey);
+  const int origin = ((sx * PP) + TS::NX * ((sy * PP) + TS::NY * (sz * PP + pz))) * 3 + pc;
+  auto gather = [&](const T *v, T (&x)[N][N]) {
+#pragma unroll
+    for (int y = 0; y < N; ++y)
+#pragma unroll
+      for (int i = 0; i < N; ++i) x[y][i] = v[origin + (y * TS::NX + i) * 3];
+  };
+  const double *cell_c = caff_all + (AFFINE && has ? slot * NCA : 0);
+  T K[RECOMP ? N : 1][9];
+  if constexpr (RECOMP) {
+    // K = (J_ref + Grad_xi u)^-1 at the column's points
+    if (pln) {
+      T x[N][N];
+      gather(tile_u, x);
+      SF3::evaluate_plane(P.sf, plane, x);
+    }
+    wave_lds_fence();
+    if (col) {
+      T G[3][3][N];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) SF3::evaluate_column(P.sf, A + c * NQP + j, G[c]);
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        T Jc[3][3], Ki[3][3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) Jc[i][d] = T(cell_c[7 + 3 * i + d]) + G[i][d][k];
+        inverse<3>(Jc, Ki);
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+          for (int c = 0; c < 3; ++c) K[k][3 * d + c] = Ki[d][c];
+      }
+    }
+    wave_lds_fence();
+  }
+  {
+    T x[N][N];
+    if (pln) gather(tile_v, x);
+    lds_barrier();
+    // every lane has gathered: the tile's destination values take the source
+    // values' place
+#pragma unroll
+    for (int k = 0; k < ROUNDS; ++k)
+      if (t + k * WG < TN)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) tile_v[(t + k * WG) * 3 + c] = dv[k][c];
+    if (pln) SF3::evaluate_plane(P.sf, plane, x);
+  }
+  wave_lds_fence();
+  if (col) {
+    T G[3][3][N];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) SF3::evaluate_column(P.sf, A + c * NQP + j, G[c]);
+    const double wxy = AFFINE ? weight_1d<N>(P.qw, j % N) * weight_1d<N>(P.qw, j / N) : 0.0;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      T g[3][3], Phi[3][3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) g[c][d] = G[c][d][k];
+      if constexpr (VAR == V_COMPACT) {
+        qp_compact<3, T>(g, cch[k], cch[k][9], cch[k][10], cch[k] + 11, Phi);
+      } else {
+        const double w = wxy * P.qw[k < N - 1 - k ? k : N - 1 - k];
+        T aw[7];
+#pragma unroll
+        for (int q = 0; q < 7; ++q) aw[q] = T(cell_c[q] * w);
+        if constexpr (RECOMP) qp_compact<3, T>(g, K[k], cch[k][0], aw[0], aw + 1, Phi);
+        else qp_compact<3, T>(g, cch[k], cch[k][9], aw[0], aw + 1, Phi);
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) G[c][d][k] = Phi[c][d];
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) SF3::integrate_column(P.sf, A + c * NQP + j, G[c]);
+  }
+  wave_lds_fence();
+  if (pln) SF3::integrate_plane(P.sf, plane);
+  lds_barrier();
+  // sum the cells' results per tile node (fixed order), one write per node
+#pragma unroll
+  for (int k = 0; k < ROUNDS; ++k) {
+    const int n = t + k * WG;
+    if (tcode[k] == kNoNode) continue;
+    const int X = n % TS::NX, Y = (n / TS::NX) % TS::NY, Z = n / (TS::NX * TS::NY);
+    T acc[3] = {T(0), T(0), T(0)};
+    const int zlo = Z == 0 ? 0 : (Z - 1) / PP, zhi = min(Z / PP, ez - 1);
+    const int ylo = Y == 0 ? 0 : (Y - 1) / PP, yhi = min(Y / PP, ey - 1);
+    const int xlo = X == 0 ? 0 : (X - 1) / PP, xhi = min(X / PP, ex - 1);
+    for (int cz = zlo; cz <= zhi; ++cz)
+      for (int cy = ylo; cy <= yhi; ++cy)
+        for (int cx = xlo; cx <= xhi; ++cx) {
+          const int rr = (X - cx * PP) + N * ((Y - cy * PP) + N * (Z - cz * PP));
+          const int s = cx + ex * (cy + ey * cz);
+#pragma unroll
+          for (int c = 0; c < 3; ++c) acc[c] += lds[s * PS::SLOT + c * NQP + rr];
+        }
+    T nv[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) nv[c] = tile_v[n * 3 + c] + acc[c];
+    const size_t node = tcode[k] & kNodeMask;
+    if (tshared[k]) {
+      store_node<3, T>(P.tbuf + ((size_t)tile * TN + n) * 3, nv);
+    } else if (!CONSTR || !((tcode[k] >> kConsShift) & 7u)) {
+      store_node<3, T>(dst + node * 3, nv);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        if (!((tcode[k] >> (kConsShift + c)) & 1u)) dst[node * 3 + c] = nv[c];
+        else if (P.tbuf && P.identity)
+          dst[node * 3 + c] = (ADD ? tile_v[n * 3 + c] : T(0)) + src[node * 3 + c];
+      }
+    }
+  }
+}
+
+// ------------------------------------------------------------------------
 // Second half of a product done in one launch over all tiles: every node that
 // several tiles touch sums their shares from tbuf in colour order, the order
 // in which coloured launches add to it (same bits), and is written once.
@@ -1846,7 +2191,8 @@ template <int DIM, int N, typename T, int VAR> __global__ void __launch_bounds__
   KP.u = P.u;
   KP.coords = P.coords;
   double F[DIM][DIM], Jri[DIM][DIM], detJr, Gu[DIM][DIM], GX[DIM][DIM];
-  kinematics_prologue<DIM, N, double, false, CPW, kWG, VAR == V_COMPACT_AFFINE>(KP, tab, A, B, Xc, on, active, code, r, i0, i1, i2, F, Jri, detJr, Gu);
+  kinematics_prologue<DIM, N, double, false, CPW, kWG, VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U>(
+      KP, tab, A, B, Xc, on, active, code, r, i0, i1, i2, F, Jri, detJr, Gu);
   // the spatial caches carry the current metric: Eulerian Q_p on curved meshes
   constexpr bool SPATIAL = (VAR == V_TENSOR2 || VAR == V_TENSOR4);
   if (SPATIAL && P.curved)
@@ -1926,14 +2272,15 @@ template <int DIM, int N, typename T, int VAR> __global__ void __launch_bounds__
     for (int v = 0; v < NV; ++v) put(D2 + v, Tv[v]);
 #pragma unroll
     for (int k = 0; k < NV * (NV + 1) / 2; ++k) put(D2 + NV + k, M[k]);
-  } else if constexpr (VAR == V_COMPACT || VAR == V_COMPACT_AFFINE) {
-    // K and c dw per point; A = mu dw R R^T and 2 lambda dw per point, or
+  } else if constexpr (VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U) {
+    // K (unless it is recomputed) and c dw per point; A = mu dw R R^T and 2 lambda dw per point, or
     // without the quadrature weight once per cell where R is one per cell
+    if constexpr (VAR != V_COMPACT_U)
 #pragma unroll
     for (int d = 0; d < DIM; ++d)
 #pragma unroll
       for (int j = 0; j < DIM; ++j) put(d * DIM + j, K[d][j]);
-    put(D2, cs * dw);
+    put(VAR == V_COMPACT_U ? 0 : D2, cs * dw);
     const double aw = VAR == V_COMPACT ? dw : detJr;
     double *ca = P.caff + (size_t)cell * kAffineStride;
     if (VAR == V_COMPACT) put(D2 + 1, 2.0 * l * aw);
@@ -1946,6 +2293,14 @@ template <int DIM, int N, typename T, int VAR> __global__ void __launch_bounds__
       for (int k = 0; k < DIM; ++k) s += Jri[i][k] * Jri[j][k];
       if (VAR == V_COMPACT) put(D2 + 2 + v, m * s * aw);
       else if (r == 0) ca[1 + v] = m * s * aw;
+    }
+    if (VAR == V_COMPACT_U && r == 0) {
+      double Jr[DIM][DIM];
+      affine_jacobian<DIM>(Xc, Jr);
+#pragma unroll
+      for (int i = 0; i < DIM; ++i)
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) ca[1 + NV + DIM * i + d] = Jr[i][d];
     }
   } else {  // tensor2 (include/mf_nh_operator.h:535-547)
 #pragma unroll
@@ -2211,16 +2566,16 @@ __global__ void __launch_bounds__(tile_threads<TILE>()) k_diagonal_tiles(const V
   using TS = TileShape<DIM, N, WG>;
   constexpr int NQP = ipow(N, DIM), CPW = TS::CPW, TN = TS::TN, NV = Voigt<DIM>::NV, NL = NQP / N;
   constexpr int D2 = DIM * DIM, NC = 1 << DIM;
-  constexpr bool KIN = VAR == V_SCALAR;
-  // per cell: NV fields of each component (V_SCALAR first needs its
-  // kinematics' sum-factorization buffers there)
+  constexpr bool KIN = VAR == V_SCALAR, RECOMP = VAR == V_COMPACT_U;
+  // per cell: NV fields of each component (V_SCALAR and V_COMPACT_U first
+  // need their kinematics' sum-factorization buffers there)
   constexpr int ARR = KIN && DIM == 2 ? 2 * D2 : DIM * NV;
   constexpr int SLOT = ARR * NQP;
   constexpr int TABN = 4 * N * N + 2 * N;
   __shared__ T lds[CPW * SLOT];
   __shared__ T tab[TABN];
   __shared__ T sq[3 * N * N];  // S S, S D, D D by [a][q]
-  __shared__ T X_all[KIN ? CPW * NC * DIM : 1];
+  __shared__ T X_all[KIN || RECOMP ? CPW * NC * DIM : 1];
   const int t = threadIdx.x;
   for (int k = t; k < TABN; k += WG) tab[k] = P.tab[k];
   for (int k = t; k < N * N; k += WG) {
@@ -2246,14 +2601,16 @@ __global__ void __launch_bounds__(tile_threads<TILE>()) k_diagonal_tiles(const V
   // K and per component the symmetric H with W^c = K H K^T, or W^c itself
   T K[DIM][DIM], base[NV], M[VAR == V_TENSOR4 || KIN ? NV * (NV + 1) / 2 : VAR == V_TENSOR4_NS ? D2 * (D2 + 1) / 2 : 1];
   T kk = T(0);
-  if constexpr (KIN) {
-    uint32_t code = 0;
+  T F[DIM][DIM], Jri[DIM][DIM], detJr, Gu[DIM][DIM], GX[DIM][DIM];
+  T *B = A + D2 * NQP;
+  uint32_t code = 0;
+  if constexpr (KIN || RECOMP) {
     if (active) code = P.idx[cq];
     lds_barrier();  // tab
-    T F[DIM][DIM], Jri[DIM][DIM], detJr, Gu[DIM][DIM], GX[DIM][DIM];
-    T *B = A + D2 * NQP;
     T *Xc = X_all + sl * NC * DIM;
     kinematics_prologue<DIM, N, T>(P, tab, A, B, Xc, on, active, code, r, i0, i1, i2, F, Jri, detJr, Gu);
+  }
+  if constexpr (KIN) {
     if (P.curved)
       geometry_gradient<DIM, N, T, false>(P.coords, P.sf, tab, lds, A, B, on, active, code, t, slot, r, i0, i1, i2,
                                           GX);
@@ -2272,19 +2629,29 @@ __global__ void __launch_bounds__(tile_threads<TILE>()) k_diagonal_tiles(const V
     constexpr int NFC = CacheFields<DIM, VAR>::value;
     T v[NFC];
     load_cache<T, NFC>(P.cache, cq, P.fs, v);
+    if constexpr (RECOMP) {
+      const double *jr = P.caff + (size_t)cell * kAffineStride + 1 + NV;
+      T Jc[DIM][DIM];
 #pragma unroll
-    for (int d = 0; d < DIM; ++d)
+      for (int i = 0; i < DIM; ++i)
 #pragma unroll
-      for (int j = 0; j < DIM; ++j) K[d][j] = v[d * DIM + j];
+        for (int d = 0; d < DIM; ++d) Jc[i][d] = T(jr[DIM * i + d]) + Gu[i][d];
+      inverse<DIM>(Jc, K);
+    } else {
+#pragma unroll
+      for (int d = 0; d < DIM; ++d)
+#pragma unroll
+        for (int j = 0; j < DIM; ++j) K[d][j] = v[d * DIM + j];
+    }
     if constexpr (VAR == V_COMPACT) {
       kk = v[D2] + v[D2 + 1];
 #pragma unroll
       for (int k = 0; k < NV; ++k) base[k] = v[D2 + 2 + k];
-    } else if constexpr (VAR == V_COMPACT_AFFINE) {
+    } else if constexpr (VAR == V_COMPACT_AFFINE || RECOMP) {
       double w = weight_1d<N>(P.qw, i0) * weight_1d<N>(P.qw, i1);
       if constexpr (DIM == 3) w *= weight_1d<N>(P.qw, i2);
       const double *ca = P.caff + (size_t)cell * kAffineStride;
-      kk = v[D2] + T(ca[0] * w);
+      kk = v[NFC - 1] + T(ca[0] * w);
 #pragma unroll
       for (int k = 0; k < NV; ++k) base[k] = T(ca[1 + k] * w);
     } else if constexpr (VAR == V_TENSOR2) {

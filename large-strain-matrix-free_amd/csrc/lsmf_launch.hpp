@@ -16,19 +16,30 @@ template <int DIM, int N> struct Launch {
   template <int VAR> static constexpr bool wide_ok() {
     return DIM == 3 && (N == 5 || N == 3) &&
            (VAR == V_TENSOR2 || VAR == V_TENSOR4 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE ||
-            VAR == V_RESIDUAL || VAR == V_ADJOINT);
+            VAR == V_COMPACT_U || VAR == V_RESIDUAL || VAR == V_ADJOINT);
   }
+
+  // products of the compact forms on wide tiles
+  template <int VAR> static constexpr bool planes_ok() {
+    return DIM == 3 && N == 3 && (VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U);
+  }
+  // K from the displacement: that kernel only (cache_variant)
+  static constexpr bool recompute_ok() { return DIM == 3 && N == 3; }
 
   // one colour's fused cell kernel: n tiles (tiled layouts) or n cells, nv
   // vectors (grid y)
   template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
   static int launch_vmult(const lsmf_op *op, const VmultParams<T> &P, int n, unsigned nv, hipStream_t s) {
     if (op->tile_kind == kTileWide) {
-      if constexpr (wide_ok<VAR>())
+      if constexpr (planes_ok<VAR>() && PH == (PH_SF | PH_QD))
+        hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR>), dim3(n, nv), dim3((PlaneShape<N, T>::WG)), 0, s, P);
+      else if constexpr (wide_ok<VAR>())
         hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide>), dim3(n, nv),
                            dim3(tile_threads<kTileWide>()), 0, s, P);
       else
         return LSMF_ERR_UNSUPPORTED;
+    } else if constexpr (VAR == V_COMPACT_U) {
+      return LSMF_ERR_UNSUPPORTED;
     } else if (op->tile_kind == 1) {
       hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, 1>), dim3(n, nv), dim3(kWG), 0, s, P);
     } else {
@@ -37,13 +48,13 @@ template <int DIM, int N> struct Launch {
     return 0;
   }
 
-  template <typename T> static VmultParams<T> params(const lsmf_op *op, int k) {
+  template <typename T, int VAR> static VmultParams<T> params(const lsmf_op *op, int k) {
     VmultParams<T> P{};
     P.idx = op->d_idx;
     P.cache = static_cast<const T *>(op->d_cache);
     P.fs = op->field_stride;
     P.tab = static_cast<const T *>(op->d_tab);
-    P.u = static_cast<const T *>(op->d_u);
+    P.u = static_cast<const T *>(VAR == V_COMPACT_U ? op->d_uc : op->d_u);
     P.coords = op->d_coords;
     P.mu = static_cast<const T *>(op->d_mu);
     P.lambda = static_cast<const T *>(op->d_lambda);
@@ -118,8 +129,8 @@ template <int DIM, int N> struct Launch {
   }
 
   // parameters of one launch over all tiles
-  template <typename T> static VmultParams<T> tile_params(const lsmf_op *op) {
-    VmultParams<T> P = params<T>(op, 0);
+  template <typename T, int VAR> static VmultParams<T> tile_params(const lsmf_op *op) {
+    VmultParams<T> P = params<T, VAR>(op, 0);
     P.tlist = nullptr;
     P.cell_begin = 0;
     P.cell_end = op->tile_ptr.back();
@@ -154,7 +165,7 @@ template <int DIM, int N> struct Launch {
   // CONSTR and identity also the constrained rows)
   template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
   static int run_tiles(const lsmf_op *op, T *dst, const T *src, int identity, hipStream_t s) {
-    VmultParams<T> P = tile_params<T>(op);
+    VmultParams<T> P = tile_params<T, VAR>(op);
     P.src = src;
     P.dst = dst;
     P.identity = identity;
@@ -188,7 +199,7 @@ template <int DIM, int N> struct Launch {
   static int run_colours(const lsmf_op *op, T *dst, const T *src, hipStream_t s) {
     const int nc = n_colours(op);
     for (int k = 0; k < nc; ++k) {
-      VmultParams<T> P = params<T>(op, k);
+      VmultParams<T> P = params<T, VAR>(op, k);
       P.src = src;
       P.dst = dst;
       const int n = P.cell_end - P.cell_begin;
@@ -252,7 +263,7 @@ template <int DIM, int N> struct Launch {
         hipLaunchKernelGGL(k_zero_list_batch<T>, dim3((op->n_orphan + 255) / 256, nv), dim3(256), 0, s,
                            op->d_orphan, op->n_orphan, d, n);
       for (int k = 0; k < nc; ++k) {
-        VmultParams<T> P = params<T>(op, k);
+        VmultParams<T> P = params<T, VAR>(op, k);
         P.src = x;
         P.dst = d;
         P.vstride = n;
@@ -277,6 +288,9 @@ template <int DIM, int N> struct Launch {
     switch (cache_variant(op)) {
       case V_COMPACT: LSMF_BATCH(V_COMPACT);
       case V_COMPACT_AFFINE: LSMF_BATCH(V_COMPACT_AFFINE);
+      case V_COMPACT_U:
+        if constexpr (recompute_ok()) return vmult_batched_t<double, V_COMPACT_U>(op, (double *)dst, (const double *)src, nvec, s);
+        return LSMF_ERR_UNSUPPORTED;
       case V_TENSOR4: LSMF_BATCH(V_TENSOR4);
       case V_TENSOR2: LSMF_BATCH(V_TENSOR2);
       case V_SCALAR: LSMF_BATCH(V_SCALAR);
@@ -295,6 +309,9 @@ template <int DIM, int N> struct Launch {
       case V_COMPACT:
         return f64 ? vmult_t<double, V_COMPACT>(op, dst, src, add, constr, ph, s)
                    : vmult_t<float, V_COMPACT>(op, dst, src, add, constr, ph, s);
+      case V_COMPACT_U:
+        if constexpr (recompute_ok()) return vmult_t<double, V_COMPACT_U>(op, dst, src, add, constr, ph, s);
+        return LSMF_ERR_UNSUPPORTED;
       case V_COMPACT_AFFINE:
         return f64 ? vmult_t<double, V_COMPACT_AFFINE>(op, dst, src, add, constr, ph, s)
                    : vmult_t<float, V_COMPACT_AFFINE>(op, dst, src, add, constr, ph, s);
@@ -342,6 +359,15 @@ template <int DIM, int N> struct Launch {
     switch (cache_variant(op)) {
       case V_COMPACT:
         return f64 ? cache_t<double, V_COMPACT>(op, bad, s) : cache_t<float, V_COMPACT>(op, bad, s);
+      case V_COMPACT_U:
+        if constexpr (recompute_ok()) {
+          // the products read this copy: the next linearisation state may be
+          // set while they run
+          if (hipMemcpyAsync(op->d_uc, op->d_u64, op->n_dofs * sizeof(double), hipMemcpyDeviceToDevice, s) != hipSuccess)
+            return LSMF_ERR_HIP;
+          return cache_t<double, V_COMPACT_U>(op, bad, s);
+        }
+        return LSMF_ERR_UNSUPPORTED;
       case V_COMPACT_AFFINE:
         return f64 ? cache_t<double, V_COMPACT_AFFINE>(op, bad, s) : cache_t<float, V_COMPACT_AFFINE>(op, bad, s);
       case V_TENSOR4:
@@ -378,6 +404,8 @@ template <int DIM, int N> struct Launch {
                              dim3(tile_threads<kTileWide>()), 0, s, P);
         else
           return (int)LSMF_ERR_UNSUPPORTED;
+      } else if constexpr (VAR == V_COMPACT_U) {
+        return (int)LSMF_ERR_UNSUPPORTED;
       } else if (op->tile_kind == 1) {
         hipLaunchKernelGGL((k_diagonal_tiles<DIM, N, T, VAR, 1>), dim3(n), dim3(kWG), 0, s, P);
       } else {
@@ -388,12 +416,12 @@ template <int DIM, int N> struct Launch {
     int rc = 0;
     const TileBufferLock lock(op, s);
     if (lock) {
-      const VmultParams<T> P = tile_params<T>(op);
+      const VmultParams<T> P = tile_params<T, VAR>(op);
       rc = cells(P, P.cell_end);
       if (!rc) tile_sum<T, false, true>(op, static_cast<T *>(op->d_diag), nullptr, 0, s);
     } else {
       for (int k = 0; k < n_colours(op) && !rc; ++k) {
-        const VmultParams<T> P = params<T>(op, k);
+        const VmultParams<T> P = params<T, VAR>(op, k);
         rc = cells(P, P.cell_end - P.cell_begin);
       }
     }
@@ -419,6 +447,9 @@ template <int DIM, int N> struct Launch {
     switch (cache_variant(op)) {
       case V_COMPACT:
         return f64 ? diagonal_t<double, V_COMPACT>(op, s) : diagonal_t<float, V_COMPACT>(op, s);
+      case V_COMPACT_U:
+        if constexpr (recompute_ok()) return diagonal_t<double, V_COMPACT_U>(op, s);
+        return LSMF_ERR_UNSUPPORTED;
       case V_COMPACT_AFFINE:
         return f64 ? diagonal_t<double, V_COMPACT_AFFINE>(op, s) : diagonal_t<float, V_COMPACT_AFFINE>(op, s);
       case V_TENSOR4:

@@ -49,11 +49,20 @@ size_t elem_size(const lsmf_op *op) { return op->precision == LSMF_FP64 ? sizeof
 // where it exists: formulation 1 with the Q1 metric.  Curved meshes (Eulerian
 // Q_p metric: K F is no longer J_ref^-1) and formulation 0 keep the stored
 // tensors.
+// K from the displacement instead of from memory (one cached value per point
+// instead of ten): FP64 operators on wide Q2 tiles of affine cells, 128^3
+// 1786 -> 1705 us, 64^3 287 -> 281, 32^3 43.5 -> 44.7 before that kernel's
+// slots were padded.  FP32 operators keep K, which is rounded once from FP64;
+// from an FP32 displacement it would lose the digits of |u| / h.
+static bool recompute_k(const lsmf_op *op) {
+  return op->affine && op->precision == LSMF_FP64 && op->dim == 3 && op->N == 3 && op->tile_kind == kTileWide;
+}
 int cache_variant(const lsmf_op *op) {
   const bool compact = op->formulation == 1 && !op->curved;
   switch (op->caching) {
     case LSMF_CACHING_TENSOR4:
     case LSMF_CACHING_TENSOR2:
+      if (compact && recompute_k(op)) return V_COMPACT_U;
       if (compact) return op->affine ? V_COMPACT_AFFINE : V_COMPACT;
       return op->caching == LSMF_CACHING_TENSOR4 ? V_TENSOR4 : V_TENSOR2;
     case LSMF_CACHING_TENSOR4_NS: return V_TENSOR4_NS;
@@ -93,6 +102,7 @@ template <int DIM> int fields_of(int variant) {
   switch (variant) {
     case V_COMPACT: return CacheFields<DIM, V_COMPACT>::value;
     case V_COMPACT_AFFINE: return CacheFields<DIM, V_COMPACT_AFFINE>::value;
+    case V_COMPACT_U: return CacheFields<DIM, V_COMPACT_U>::value;
     case V_TENSOR4: return CacheFields<DIM, V_TENSOR4>::value;
     case V_TENSOR2: return CacheFields<DIM, V_TENSOR2>::value;
     case V_TENSOR4_NS: return CacheFields<DIM, V_TENSOR4_NS>::value;
@@ -129,7 +139,7 @@ template <typename T> int dalloc(T **p, size_t n, const char *what) {
 }
 
 void free_op(lsmf_op *op) {
-  void *ptrs[] = {op->d_idx,  op->d_coords,    op->d_tab,  op->d_tab64, op->d_mu64,     op->d_lambda64,
+  void *ptrs[] = {op->d_uc,   op->d_idx,  op->d_coords,    op->d_tab,  op->d_tab64, op->d_mu64,     op->d_lambda64,
                   op->d_mu,   op->d_lambda,    op->d_cache, op->d_caff, op->d_diag, op->d_inv_diag, op->d_cons,
                   op->d_bad,  op->d_perm,      op->d_tile_nodes, op->d_tile_info, op->d_tile_tables,
                   op->d_tile_buf, op->d_orphan, op->d_hang, op->d_hptr,
@@ -560,11 +570,15 @@ __global__ void k_convert_f64_f32(const double *__restrict__ a, float *__restric
 
 namespace lsmf {
 namespace {
+bool cell_constants(const lsmf_op *op) {
+  return cache_variant(op) == V_COMPACT_AFFINE || cache_variant(op) == V_COMPACT_U;
+}
 // bytes of the cached values a product reads
 size_t cache_bytes(const lsmf_op *op) {
   const size_t es = elem_size(op);
   return (size_t)op->n_fields * op->field_stride * es +
-         (cache_variant(op) == V_COMPACT_AFFINE ? (size_t)op->n_cells * kAffineStride * sizeof(double) : 0);
+         (cell_constants(op) ? (size_t)op->n_cells * kAffineStride * sizeof(double) : 0) +
+         (cache_variant(op) == V_COMPACT_U ? op->n_dofs * es : 0);
 }
 
 // cache(): zero the det F <= 0 counter bad_dev, run the cache kernel, read
@@ -707,7 +721,6 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
 
   op->curved = p > 1 && support_points_curved(mesh, dim, p, nqp);
   op->affine = cells_affine(mesh, dim, p, nqp);
-  op->n_fields = n_cache_fields(op);
   // --- cell order of the tiled layout (structured meshes), else by colour;
   // the per-cell index table of tiles carries no first-touch bits
   TileTables tt;
@@ -733,6 +746,7 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
       return rc;
     }
   }
+  op->n_fields = n_cache_fields(op);
   // --- colouring (given and checked, or greedy first fit): no node is written
   // by two cells of one colour; used[n] = colours of the cells that write n.
   // Tiles need none, but a given one is checked for them too.
@@ -966,7 +980,8 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
       (rc = dalloc((char **)&op->d_lambda, (size_t)nc * es, "lambda")) ||
       (rc = dalloc(&op->d_u64, op->n_dofs, "displacement")) ||
       (rc = dalloc((char **)&op->d_cache, (size_t)op->n_fields * op->field_stride * es, "cache")) ||
-      (cache_variant(op) == V_COMPACT_AFFINE &&
+      (cache_variant(op) == V_COMPACT_U && (rc = dalloc((char **)&op->d_uc, op->n_dofs * es, "cached displacement"))) ||
+      (cell_constants(op) &&
        (rc = dalloc(&op->d_caff, (size_t)nc * kAffineStride, "cell constants"))) ||
       (rc = dalloc((char **)&op->d_diag, op->n_dofs * es, "diagonal")) ||
       (rc = dalloc((char **)&op->d_inv_diag, op->n_dofs * es, "inverse diagonal")) ||

@@ -97,3 +97,31 @@ def test_formulation_switch_changes_the_cached_values(device):
         expect = oracle_op(mesh, mu, lam, u, cons, "tensor4", formulation).vmult(v)
         assert rel(y.cpu().numpy(), expect) < 1e-12, formulation
         assert bytes_of.setdefault(formulation, op.memory_consumption()) == op.memory_consumption()
+
+
+def test_products_keep_the_cached_state(device):
+    """a product after cache() uses the state that was cached: the next
+    linearisation state may be set (on another stream) while it runs, and no
+    product runs between set_linearization and cache()"""
+    import torch
+    mesh, mu, lam, u, cons = problem(3, 2, [19, 9, 9], "sheared")
+    x = torch.tensor(np.random.default_rng(1).standard_normal(mesh.n_dofs), device=device)
+    op = lsmf.NeoHookOperator(mesh, caching="tensor4", constrained=cons)
+    op.set_material(mu, lam)
+    op.set_linearization(torch.tensor(u, device=device))
+    op.cache()
+    expect = oracle_op(mesh, mu, lam, u, cons, "tensor4").vmult(x.cpu().numpy())
+    other, ys = torch.cuda.Stream(), [torch.empty_like(x) for _ in range(20)]
+    zero = torch.zeros_like(x)
+    torch.cuda.synchronize()
+    for y in ys:
+        op.vmult(y, x)
+    op.set_linearization(zero, stream=other.cuda_stream)
+    torch.cuda.synchronize()
+    for y in ys:
+        assert rel(y.cpu().numpy(), expect) < 1e-12
+    with pytest.raises(lsmf.LsmfError):
+        op.vmult(ys[0], x)
+    op.cache()
+    op.vmult(ys[0], x)
+    assert rel(ys[0].cpu().numpy(), oracle_op(mesh, mu, lam, 0 * u, cons, "tensor4").vmult(x.cpu().numpy())) < 1e-12

@@ -1,7 +1,7 @@
 """Products in one launch over all tiles (the operator's first stream) against
 the coloured launches (any other stream, captured calls, batched products):
 the same sums in the same order, so the same bits, for set, add, plain and
-phase-masked products, the residual and its VJP, at meshes of one cell, less
+phase-masked products, the diagonal, the residual and its VJP, at meshes of one cell, less
 than one tile, ragged and several tiles per direction.
 """
 import threading
@@ -45,6 +45,8 @@ def test_same_bits_as_coloured_launches(dim, p, n, caching, precision, device):
             y = start.clone() if kw.get("add") else torch.full_like(x, float("nan"))
             op.vmult(y, x, stream=stream, **kw)
             out.append(y)
+        op.compute_diagonal(stream=stream)
+        out.append(op.diagonal())
         if precision == "fp64":
             r, du = torch.full_like(x, float("nan")), torch.full_like(x, float("nan"))
             dmu = torch.empty(op.n_cells, dtype=x.dtype, device=device)
