@@ -2164,6 +2164,7 @@ struct CacheParams {
   int formulation;
   int curved;  // Eulerian Q_p metric for the spatial caches (tensor2, tensor4)
   int *bad;
+  double sf[2 * 15];  // even-odd 1D matrices, see VmultParams
 };
 
 template <int DIM, int N, typename T, int VAR> __global__ void __launch_bounds__(kWG) k_cache(const CacheParams P) {
@@ -2171,8 +2172,12 @@ template <int DIM, int N, typename T, int VAR> __global__ void __launch_bounds__
   constexpr int NQP = CS::NQP, CPW = CS::CPW, NB = CS::NB, NC = CS::NC;
   constexpr int NV = Voigt<DIM>::NV;
   constexpr int TABN = 4 * N * N + 2 * N;
-  __shared__ double lds[CPW * 2 * NB * NQP + TABN + CPW * NC * DIM];
-  double *tab = lds + CPW * 2 * NB * NQP;
+  // 3D: line-per-lane sums in place (SFLine), half the LDS of the 2D ping-pong
+  // pair: 32^3 Q4 FP32 187 -> 103 us, 48^3 Q2 FP64 92 -> 77
+  constexpr bool LINE = DIM == 3;
+  constexpr int SLOTW = (LINE ? 1 : 2) * NB * NQP;
+  __shared__ double lds[CPW * SLOTW + TABN + CPW * NC * DIM];
+  double *tab = lds + CPW * SLOTW;
   const int t = threadIdx.x;
   if (t < TABN) tab[t] = P.tab[t];
   const int slot = t / NQP, r = t - slot * NQP;
@@ -2181,8 +2186,8 @@ template <int DIM, int N, typename T, int VAR> __global__ void __launch_bounds__
   constexpr int D2 = DIM * DIM;
   const bool on = slot < CPW;
   const bool active = on && (cell < P.n_cells);
-  double *A = lds + (slot < CPW ? slot : 0) * 2 * NB * NQP;
-  double *B = A + NB * NQP;
+  double *A = lds + (slot < CPW ? slot : 0) * SLOTW;
+  double *B = LINE ? A : A + NB * NQP;  // 2D only
   double *Xc = tab + TABN + (slot < CPW ? slot : 0) * NC * DIM;
   uint32_t code = 0;
   if (active) code = P.idx[(size_t)cell * NQP + r];
@@ -2190,14 +2195,15 @@ template <int DIM, int N, typename T, int VAR> __global__ void __launch_bounds__
   KP.formulation = P.formulation;
   KP.u = P.u;
   KP.coords = P.coords;
+  for (int k = 0; k < 2 * 15; ++k) KP.sf[k] = P.sf[k];
   double F[DIM][DIM], Jri[DIM][DIM], detJr, Gu[DIM][DIM], GX[DIM][DIM];
-  kinematics_prologue<DIM, N, double, false, CPW, kWG, VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U>(
-      KP, tab, A, B, Xc, on, active, code, r, i0, i1, i2, F, Jri, detJr, Gu);
+  kinematics_prologue<DIM, N, double, LINE, CPW, kWG, VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U>(
+      KP, tab, A, B, Xc, on, active, code, r, i0, i1, i2, F, Jri, detJr, Gu, lds, t, slot);
   // the spatial caches carry the current metric: Eulerian Q_p on curved meshes
   constexpr bool SPATIAL = (VAR == V_TENSOR2 || VAR == V_TENSOR4);
   if (SPATIAL && P.curved)
-    geometry_gradient<DIM, N, double, false>(P.coords, nullptr, tab, lds, A, B, on, active, code, t, slot, r, i0, i1,
-                                             i2, GX);
+    geometry_gradient<DIM, N, double, LINE>(P.coords, P.sf, tab, lds, A, B, on, active, code, t, slot, r, i0, i1, i2,
+                                            GX);
   double uq[DIM];
   if constexpr (VAR == V_SCALAR_REF) {
     // u at this Gauss point: the tensor-product interpolation of the nodal
@@ -2571,6 +2577,7 @@ __global__ void __launch_bounds__(tile_threads<TILE>()) k_diagonal_tiles(const V
   // need their kinematics' sum-factorization buffers there)
   constexpr int ARR = KIN && DIM == 2 ? 2 * D2 : DIM * NV;
   constexpr int SLOT = ARR * NQP;
+  static_assert(DIM == 2 || CPW * SFLine<N, T>::SLOT <= CPW * SLOT, "kinematics fit the fields' region");
   constexpr int TABN = 4 * N * N + 2 * N;
   __shared__ T lds[CPW * SLOT];
   __shared__ T tab[TABN];
@@ -2602,18 +2609,21 @@ __global__ void __launch_bounds__(tile_threads<TILE>()) k_diagonal_tiles(const V
   T K[DIM][DIM], base[NV], M[VAR == V_TENSOR4 || KIN ? NV * (NV + 1) / 2 : VAR == V_TENSOR4_NS ? D2 * (D2 + 1) / 2 : 1];
   T kk = T(0);
   T F[DIM][DIM], Jri[DIM][DIM], detJr, Gu[DIM][DIM], GX[DIM][DIM];
-  T *B = A + D2 * NQP;
+  // 3D: line-per-lane sums, slots of their own stride in the same region
+  constexpr bool LINE = DIM == 3;
+  T *KA = LINE ? lds + sl * D2 * NQP : A, *B = A + D2 * NQP;
   uint32_t code = 0;
   if constexpr (KIN || RECOMP) {
     if (active) code = P.idx[cq];
     lds_barrier();  // tab
     T *Xc = X_all + sl * NC * DIM;
-    kinematics_prologue<DIM, N, T>(P, tab, A, B, Xc, on, active, code, r, i0, i1, i2, F, Jri, detJr, Gu);
+    kinematics_prologue<DIM, N, T, LINE, CPW, WG>(P, tab, KA, B, Xc, on, active, code, r, i0, i1, i2, F, Jri, detJr,
+                                                  Gu, lds, t, slot);
   }
   if constexpr (KIN) {
     if (P.curved)
-      geometry_gradient<DIM, N, T, false>(P.coords, P.sf, tab, lds, A, B, on, active, code, t, slot, r, i0, i1, i2,
-                                          GX);
+      geometry_gradient<DIM, N, T, LINE, CPW, WG>(P.coords, P.sf, tab, lds, KA, B, on, active, code, t, slot, r, i0,
+                                                  i1, i2, GX);
     const T m = P.mu[cell], l = P.lambda[cell];
     T Fi[DIM][DIM];
     const T J = inverse<DIM>(F, Fi);

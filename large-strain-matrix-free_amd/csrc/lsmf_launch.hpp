@@ -48,6 +48,22 @@ template <int DIM, int N> struct Launch {
     return 0;
   }
 
+  // even-odd forms of S (rows r < R) and D, from the plain tables
+  template <typename T> static void pack_sf(const lsmf_op *op, T *sf) {
+    using EO = EvenOdd<N, T>;
+    for (int m = 0; m < 2; ++m) {
+      const double *M = op->h_sf + m * N * N;
+      T *pk = sf + m * EO::PK;
+      for (int r = 0; r < EO::R; ++r) {
+        for (int k = 0; k < EO::H; ++k) {
+          pk[r * EO::H + k] = T(0.5 * (M[r * N + k] + M[r * N + N - 1 - k]));
+          pk[EO::R * EO::H + r * EO::H + k] = T(0.5 * (M[r * N + k] - M[r * N + N - 1 - k]));
+        }
+        pk[2 * EO::R * EO::H + r] = EO::ODD ? T(M[r * N + EO::H]) : T(0);
+      }
+    }
+  }
+
   template <typename T, int VAR> static VmultParams<T> params(const lsmf_op *op, int k) {
     VmultParams<T> P{};
     P.idx = op->d_idx;
@@ -84,20 +100,8 @@ template <int DIM, int N> struct Launch {
     P.perm = op->d_perm;
     P.caff = op->d_caff;
     for (int k = 0; k < 3; ++k) P.qw[k] = op->h_qw[k];
-    using EO = EvenOdd<N, T>;
-    static_assert(sizeof(P.sf) / sizeof(P.sf[0]) >= 2 * EO::PK, "1D matrices do not fit the kernel arguments");
-    // even-odd forms of S (rows r < R) and D, from the plain tables
-    for (int m = 0; m < 2; ++m) {
-      const double *M = op->h_sf + m * N * N;
-      T *pk = P.sf + m * EO::PK;
-      for (int r = 0; r < EO::R; ++r) {
-        for (int k = 0; k < EO::H; ++k) {
-          pk[r * EO::H + k] = T(0.5 * (M[r * N + k] + M[r * N + N - 1 - k]));
-          pk[EO::R * EO::H + r * EO::H + k] = T(0.5 * (M[r * N + k] - M[r * N + N - 1 - k]));
-        }
-        pk[2 * EO::R * EO::H + r] = EO::ODD ? T(M[r * N + EO::H]) : T(0);
-      }
-    }
+    static_assert(sizeof(P.sf) / sizeof(P.sf[0]) >= 2 * EvenOdd<N, T>::PK, "1D matrices do not fit the kernel arguments");
+    pack_sf<T>(op, P.sf);
     return P;
   }
 
@@ -350,6 +354,7 @@ template <int DIM, int N> struct Launch {
     P.formulation = op->formulation;
     P.curved = op->curved;
     P.bad = bad;
+    pack_sf<double>(op, P.sf);
     hipLaunchKernelGGL((k_cache<DIM, N, T, VAR>), dim3(grid_for(op->n_cells)), dim3(kWG), 0, s, P);
     return hipGetLastError() == hipSuccess ? 0 : LSMF_ERR_HIP;
   }
