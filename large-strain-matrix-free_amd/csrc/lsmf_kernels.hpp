@@ -1051,13 +1051,59 @@ template <int DIM, int N> __device__ __forceinline__ int node_corner(int i0, int
   return (i0 ? 1 : 0) + (i1 ? 2 : 0) + ((DIM == 3 && i2) ? 4 : 0);
 }
 
+// What a launch over all tiles does with A x of a node instead of storing it:
+// the smoother's vector updates (deal.II's PreconditionChebyshev recurrence),
+// so that they cost no launch and A x no trip to memory.  x is the product's
+// source too: a node is updated by its only tile after the tile has read it,
+// or by k_tile_sum after all tiles have.
+enum EpilogueKind {
+  EP_STORE = 0,
+  EP_RESIDUAL = 1,    // dst = b - A x
+  EP_CHEB_FIRST = 2,  // d = f2 invd (b - A x), x += d
+  EP_CHEB = 3         // d = f1 d + f2 invd (b - A x), x += d
+};
+template <typename T> struct Epilogue {
+  int kind;
+  const T *b, *invd;
+  T *d, *x;
+  T f1, f2;
+};
+template <int DIM, typename T> __device__ __forceinline__ void store_node(T *p, const T (&v)[DIM]);
+template <int DIM, typename T>
+__device__ __forceinline__ void apply_epilogue(const Epilogue<T> &ep, T *dst, const T *src, size_t node, uint32_t code,
+                                               T (&ax)[DIM]) {
+  const size_t at = node * DIM;
+  T x[DIM], b[DIM], iv[DIM], d[DIM];
+  load_node<DIM, T>(src + at, x);
+  load_node<DIM, T>(ep.b + at, b);
+#pragma unroll
+  for (int c = 0; c < DIM; ++c)
+    if ((code >> (kConsShift + c)) & 1u) ax[c] = x[c];  // the constrained rows' identity
+  if (ep.kind == EP_RESIDUAL) {
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) b[c] -= ax[c];
+    store_node<DIM, T>(dst + at, b);
+    return;
+  }
+  load_node<DIM, T>(ep.invd + at, iv);
+  if (ep.kind == EP_CHEB) load_node<DIM, T>(ep.d + at, d);
+#pragma unroll
+  for (int c = 0; c < DIM; ++c) {
+    const T di = ep.f2 * iv[c] * (b[c] - ax[c]);
+    d[c] = ep.kind == EP_CHEB ? ep.f1 * d[c] + di : di;
+    x[c] += d[c];
+  }
+  store_node<DIM, T>(ep.d + at, d);
+  store_node<DIM, T>(ep.x + at, x);
+}
+
 template <typename Number> struct VmultParams {
   const uint32_t *__restrict__ idx;   // [cells][NQP] sorted cells
   const Number *__restrict__ cache;   // SoA caches
   size_t fs;                          // field stride = n_cells * NQP
   const Number *__restrict__ tab;     // S, D, St, Dt, qp, qw (Number)
-  const Number *__restrict__ src;
-  Number *__restrict__ dst;
+  const Number *src;
+  Number *dst;
   size_t vstride;                     // batched products: distance between vectors (0: one vector)
   const Number *__restrict__ u;       // scalar / residual: displacement
   const double *__restrict__ coords;  // scalar / residual: node coordinates
@@ -1075,6 +1121,7 @@ template <typename Number> struct VmultParams {
   const uint32_t *__restrict__ tpriv;
   Number *__restrict__ tbuf;
   int identity;  // with tbuf: constrained DoFs get the identity here and in k_tile_sum
+  Epilogue<Number> ep;  // with tbuf, identity and CONSTR
   // node (hanging) constraints, cells layout only; hang == nullptr: none.
   // Each (cell, constrained node) pair is an instance: its cell reads the
   // weighted sum of the masters and leaves its result in hbuf, from where
@@ -1284,8 +1331,8 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
 
   // batched products (all columns of a small matrix in one launch): vector
   // blockIdx.y lives at offset blockIdx.y * vstride of src and dst
-  const T *__restrict__ src = P.src + (size_t)blockIdx.y * P.vstride;
-  T *__restrict__ dst = P.dst + (size_t)blockIdx.y * P.vstride;
+  const T *src = P.src + (size_t)blockIdx.y * P.vstride;  // an epilogue updates it in place
+  T *dst = P.dst + (size_t)blockIdx.y * P.vstride;
   const int t = threadIdx.x;
   if (t < TABN) tab[t] = P.tab[t];
   const int slot = t / NQP;
@@ -1646,6 +1693,8 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
       for (int c = 0; c < DIM; ++c) nv[c] = tile_v[t * DIM + c] + acc[c];  // destination: 0 on first touch
       if (tshared) {
         store_node<DIM, T>(P.tbuf + ((size_t)tile * TN + t) * DIM, nv);
+      } else if (CONSTR && !ADD && P.ep.kind != EP_STORE) {
+        apply_epilogue<DIM, T>(P.ep, dst, src, tnode, tcode, nv);
       } else if (!CONSTR || !((tcode >> kConsShift) & ((1u << DIM) - 1u))) {
         store_node<DIM, T>(dst + tnode * DIM, nv);
       } else {
@@ -1832,8 +1881,8 @@ __global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T
   __shared__ T tile_v[TN * 3];
   __shared__ double caff_all[CA];
   __shared__ T tile_u[RECOMP ? TN * 3 : 1];
-  const T *__restrict__ src = P.src + (size_t)blockIdx.y * P.vstride;
-  T *__restrict__ dst = P.dst + (size_t)blockIdx.y * P.vstride;
+  const T *src = P.src + (size_t)blockIdx.y * P.vstride;  // an epilogue updates it in place
+  T *dst = P.dst + (size_t)blockIdx.y * P.vstride;
   const int t = threadIdx.x, wave = t / 64, lane = t % 64;
   const int L = xcd_remap(blockIdx.x, gridDim.x);
   const int tile = P.tlist ? P.tlist[P.cell_begin + L] : P.cell_begin + L;
@@ -2012,6 +2061,8 @@ __global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T
     const size_t node = tcode[k] & kNodeMask;
     if (tshared[k]) {
       store_node<3, T>(P.tbuf + ((size_t)tile * TN + n) * 3, nv);
+    } else if (CONSTR && !ADD && P.ep.kind != EP_STORE) {
+      apply_epilogue<3, T>(P.ep, dst, src, node, tcode[k], nv);
     } else if (!CONSTR || !((tcode[k] >> kConsShift) & 7u)) {
       store_node<3, T>(dst + node * 3, nv);
     } else {
@@ -2044,9 +2095,10 @@ template <typename T> struct TileSumParams {
   const uint32_t *__restrict__ node;  // node | constraint bits
   const uint32_t *__restrict__ slot;
   const T *__restrict__ buf;
-  const T *__restrict__ src;  // constrained rows (CONSTR)
-  T *__restrict__ dst;
+  const T *src;  // constrained rows (CONSTR)
+  T *dst;
   int identity;
+  Epilogue<T> ep;
   int n_groups;
   int begin[kMaxGroups + 1];
   int mult[kMaxGroups];
@@ -2091,6 +2143,11 @@ __global__ void __launch_bounds__(kWG) k_tile_sum(const TileSumParams<T> P) {
   else if (m == 8) sum_slots<DIM, 8, T>(slot, stride, P.buf, acc);
   else
     for (int k = 0; k < m; ++k) sum_slots<DIM, 1, T>(slot + k * stride, stride, P.buf, acc);
+  if constexpr (CONSTR && !ADD)
+    if (P.ep.kind != EP_STORE) {
+      apply_epilogue<DIM, T>(P.ep, P.dst, P.src, node, code, acc);
+      return;
+    }
   if (!CONSTR || !((code >> kConsShift) & ((1u << DIM) - 1u))) {
     store_node<DIM, T>(P.dst + node * DIM, acc);
   } else {

@@ -145,7 +145,8 @@ template <int DIM, int N> struct Launch {
 
   // the sums of the nodes that several tiles share, after such a launch
   template <typename T, bool ADD, bool CONSTR>
-  static void tile_sum(const lsmf_op *op, T *dst, const T *src, int identity, hipStream_t s) {
+  static void tile_sum(const lsmf_op *op, T *dst, const T *src, int identity, hipStream_t s,
+                       const Epilogue<T> &ep = Epilogue<T>()) {
     const int n = op->sum_begin[op->n_sum_groups];
     if (n == 0) return;
     TileSumParams<T> S{};
@@ -155,6 +156,7 @@ template <int DIM, int N> struct Launch {
     S.src = src;
     S.dst = dst;
     S.identity = identity;
+    S.ep = ep;
     S.n_groups = op->n_sum_groups;
     for (int g = 0; g < S.n_groups; ++g) {
       S.begin[g] = op->sum_begin[g];
@@ -168,15 +170,17 @@ template <int DIM, int N> struct Launch {
   // all tiles in one launch, then the sums of the nodes they share (with
   // CONSTR and identity also the constrained rows)
   template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
-  static int run_tiles(const lsmf_op *op, T *dst, const T *src, int identity, hipStream_t s) {
+  static int run_tiles(const lsmf_op *op, T *dst, const T *src, int identity, hipStream_t s,
+                       const Epilogue<T> &ep = Epilogue<T>()) {
     VmultParams<T> P = tile_params<T, VAR>(op);
+    P.ep = ep;
     P.src = src;
     P.dst = dst;
     P.identity = identity;
     if (op->prof) op->prof->before(s);
     const int rc = launch_vmult<T, VAR, ADD, CONSTR, PH>(op, P, P.cell_end, 1, s);
     if (rc) return rc;
-    tile_sum<T, ADD, CONSTR>(op, dst, src, identity, s);
+    tile_sum<T, ADD, CONSTR>(op, dst, src, identity, s, ep);
     if (op->prof) op->prof->after(s);
     return 0;
   }
@@ -245,6 +249,45 @@ template <int DIM, int N> struct Launch {
     }
     if (rc) return rc;
     return hipGetLastError() == hipSuccess ? 0 : LSMF_ERR_HIP;
+  }
+
+  // a product with an epilogue, where it can run in one launch over all tiles
+  // (*done; else nothing was launched)
+  template <typename T, int VAR>
+  static int smooth_t(const lsmf_op *op, const SmoothArgs &a, bool *done, hipStream_t s) {
+    *done = false;
+    if (op->n_orphan > 0) return 0;
+    const TileBufferLock lock(op, s);
+    if (!lock) return 0;
+    *done = true;
+    T *x = static_cast<T *>(a.x);
+    const Epilogue<T> ep{a.kind, static_cast<const T *>(a.b), static_cast<const T *>(a.invd), static_cast<T *>(a.d), x,
+                         T(a.f1), T(a.f2)};
+    T *dst = a.kind == EP_RESIDUAL ? static_cast<T *>(a.dst) : x;
+    const int rc = run_tiles<T, VAR, false, true, PH_SF | PH_QD>(op, dst, x, 1, s, ep);
+    if (rc) return rc;
+    return hipGetLastError() == hipSuccess ? 0 : LSMF_ERR_HIP;
+  }
+  static int smooth(const lsmf_op *op, const SmoothArgs &a, bool *done, hipStream_t s) {
+    const bool f64 = op->precision == LSMF_FP64;
+    *done = false;
+    switch (cache_variant(op)) {
+      case V_COMPACT_U:
+        if constexpr (recompute_ok()) return smooth_t<double, V_COMPACT_U>(op, a, done, s);
+        return 0;
+      case V_COMPACT_AFFINE:
+        return f64 ? smooth_t<double, V_COMPACT_AFFINE>(op, a, done, s)
+                   : smooth_t<float, V_COMPACT_AFFINE>(op, a, done, s);
+      case V_COMPACT:
+        return f64 ? smooth_t<double, V_COMPACT>(op, a, done, s) : smooth_t<float, V_COMPACT>(op, a, done, s);
+      case V_TENSOR4:
+        return f64 ? smooth_t<double, V_TENSOR4>(op, a, done, s) : smooth_t<float, V_TENSOR4>(op, a, done, s);
+      case V_TENSOR2:
+        return f64 ? smooth_t<double, V_TENSOR2>(op, a, done, s) : smooth_t<float, V_TENSOR2>(op, a, done, s);
+      case V_SCALAR:
+        return f64 ? smooth_t<double, V_SCALAR>(op, a, done, s) : smooth_t<float, V_SCALAR>(op, a, done, s);
+      default: return 0;
+    }
   }
 
   // nvec products in set mode with constraints, vector b at b * n_dofs:
@@ -492,7 +535,7 @@ template <int DIM, int N> struct Launch {
   }
 
   static const LaunchTable *table() {
-    static const LaunchTable t{&vmult, &vmult_batched, &cache, &diagonal, &residual, &residual_vjp};
+    static const LaunchTable t{&vmult, &vmult_batched, &smooth, &cache, &diagonal, &residual, &residual_vjp};
     return &t;
   }
 };

@@ -72,6 +72,13 @@ int cache_variant(const lsmf_op *op) {
   }
 }
 
+int smooth(lsmf_op *op, const SmoothArgs &a, bool *done, hipStream_t s) {
+  *done = false;
+  if (!op->cached) return fail(LSMF_ERR_NOT_CACHED, "smooth: call cache() first");
+  const int rc = launch_table(op->dim, op->N)->smooth(op, a, done, s);
+  return rc ? fail(rc, "smooth: kernel launch failed") : LSMF_OK;
+}
+
 void bind_stream(lsmf_op *op, hipStream_t s) {
   op->ws_bound = true;
   op->ws_stream = s;

@@ -157,10 +157,24 @@ class TileBufferLock {
   std::unique_lock<std::mutex> lock_;
 };
 
+// A product A x with a vector update in the operator's precision (EpilogueKind
+// of lsmf_kernels.hpp): kind 1: dst = b - A x; kinds 2, 3: the Chebyshev step on
+// x and d.  *done false: not available for this operator (too large, another
+// stream's), nothing was launched.
+struct SmoothArgs {
+  int kind;
+  void *dst, *x;
+  const void *b, *invd;
+  void *d;
+  double f1, f2;
+};
+int smooth(lsmf_op *op, const SmoothArgs &a, bool *done, hipStream_t s);
+
 // launch entry points of one (dim, N) instantiation unit
 struct LaunchTable {
   int (*vmult)(const lsmf_op *, void *dst, const void *src, bool add, bool constr, unsigned ph, hipStream_t);
   int (*vmult_batched)(const lsmf_op *, void *dst, const void *src, int nvec, hipStream_t);
+  int (*smooth)(const lsmf_op *, const SmoothArgs &, bool *done, hipStream_t);
   int (*cache)(const lsmf_op *, int *bad, hipStream_t);  // bad: det F <= 0 counter (zeroed by the caller)
   int (*diagonal)(const lsmf_op *, hipStream_t);
   int (*residual)(const lsmf_op *, double *rhs, hipStream_t);

@@ -31,6 +31,8 @@
 #include "lsmf.h"
 #include "lsmf_error.hpp"
 #include "lsmf_fe.hpp"
+#include "lsmf_kernels.hpp"
+#include "lsmf_op.hpp"
 #include "lsmf_solver.hpp"
 #include "lsmf_vec.hpp"
 
@@ -595,6 +597,13 @@ template <typename T> class GMG : public GMGBase {
   }
 
 
+  // a product with its vector update in the product's launches; false: do both
+  bool fused(Level<T> &v, const SmoothArgs &a) {
+    bool done = false;
+    abi_check(smooth(v.op->handle(), a, &done, s_), "smooth");
+    return done;
+  }
+
   // Chebyshev smoother / coarse solver on level v: x from zero (vmult) or
   // from its current value (step)
   void chebyshev(Level<T> &v, T *x, const T *b, bool x_zero) {
@@ -603,17 +612,20 @@ template <typename T> class GMG : public GMGBase {
     if (x_zero) {
       launch_cheb_first<T>(s_, x, v.d.p, b, (const T *)nullptr, invd, 1.0 / v.theta, 1, n);
     } else {
-      v.op->vmult(v.t.p, x);
-      launch_cheb_first<T>(s_, x, v.d.p, b, (const T *)v.t.p, invd, 1.0 / v.theta, 0, n);
+      if (!fused(v, {EP_CHEB_FIRST, nullptr, x, b, invd, v.d.p, 0.0, 1.0 / v.theta})) {
+        v.op->vmult(v.t.p, x);
+        launch_cheb_first<T>(s_, x, v.d.p, b, (const T *)v.t.p, invd, 1.0 / v.theta, 0, n);
+      }
     }
     if (v.degree < 2 || std::fabs(v.delta) < 1e-40) return;
     double rhok = v.delta / v.theta;
     const double sigma = v.theta / v.delta;
     for (int k = 0; k < v.degree - 1; ++k) {
-      v.op->vmult(v.t.p, x);
       const double rhokp = 1.0 / (2.0 * sigma - rhok);
       const double f1 = rhokp * rhok, f2 = 2.0 * rhokp / v.delta;
       rhok = rhokp;
+      if (fused(v, {EP_CHEB, nullptr, x, b, invd, v.d.p, f1, f2})) continue;
+      v.op->vmult(v.t.p, x);
       launch_cheb_update<T>(s_, x, v.d.p, b, (const T *)v.t.p, invd, f1, f2, n);
     }
   }
@@ -633,8 +645,10 @@ template <typename T> class GMG : public GMGBase {
       return;
     }
     chebyshev(v, v.sol.p, v.rhs.p, true);  // pre-smoothing from zero
-    v.op->vmult(v.t.p, v.sol.p);
-    launch_residual<T>(s_, v.t.p, (const T *)v.rhs.p, n);
+    if (!fused(v, {EP_RESIDUAL, v.t.p, v.sol.p, v.rhs.p, nullptr, nullptr, 0.0, 0.0})) {
+      v.op->vmult(v.t.p, v.sol.p);
+      launch_residual<T>(s_, v.t.p, (const T *)v.rhs.p, n);
+    }
     Level<T> &c = lv_[l - 1];
     restrict_(l, c.rhs.p, v.t.p);
     vcycle(l - 1);

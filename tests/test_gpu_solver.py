@@ -594,3 +594,43 @@ def test_condition_number_estimate(device):
     assert 1.0 <= est3 <= exact * (1 + 1e-10)
     est0, _ = solve(0)
     assert est0 == 0.0
+
+
+@pytest.mark.parametrize("dim,p,coarse,levels,precision", [(3, 2, [1, 1, 1], 3, "fp32"), (3, 2, [3, 1, 2], 3, "fp64"),
+                                                           (3, 4, [1, 1, 1], 3, "fp64"), (2, 2, [3, 2, 1], 4, "fp64"),
+                                                           (3, 1, [2, 2, 2], 3, "fp64")])
+def test_vcycle_replay_and_eager_agree(dim, p, coarse, levels, precision, device):
+    """V-cycles whose smoothing steps run inside the products' launches: the
+    captured graph's replays, between products of the fine operator on another
+    stream, and the eager V-cycle give the same bits; a second state changes
+    them, and returning to the first gives the first result"""
+    import torch
+    print(f"[fused smoother] dim={dim} p={p} {coarse} {levels} {precision}", flush=True)
+    n_cells = int(np.prod([c << (levels - 1) for c in coarse[:dim]]))
+    rng = np.random.default_rng(2)
+    mu, lam = 1.0 + rng.random(n_cells), 2.0 + rng.random(n_cells)
+    results = []
+    for graph in (1, 0):
+        o = lsmf.solver_options(dim=dim, degree=p, n_q_1d=p + 1, n_cells_coarse=coarse, n_levels=levels,
+                                caching="tensor4", mg_caching="tensor4", mg_precision=precision, smoother_degree=4,
+                                coarse_solver="direct", use_graph=graph,
+                                dirichlet={0: (list(range(dim)), [0.0] * dim), 1: ([0], [0.01])})
+        s = lsmf.Solver(o, mu, lam)
+        n = s.n_dofs()
+        r = torch.tensor(np.random.default_rng(3).standard_normal(n), device=device)
+        first = None
+        for state in (0.0, 1e-3, 0.0):
+            s.set_state(state * np.random.default_rng(4).standard_normal(n) * 0.01)
+            z = [torch.full_like(r, float("nan")) for _ in range(3)]
+            for out in z:
+                s.precondition(out, r)
+            torch.cuda.synchronize()
+            assert torch.equal(z[0], z[1]) and torch.equal(z[0], z[2]) and bool(torch.isfinite(z[0]).all())
+            if first is None:
+                first = z[0].clone()
+            elif state == 0.0:
+                assert torch.equal(z[0], first)
+            else:
+                assert not torch.equal(z[0], first)
+        results.append(first)
+    assert torch.equal(results[0], results[1])
