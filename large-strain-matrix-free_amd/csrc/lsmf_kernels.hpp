@@ -262,7 +262,7 @@ template <int DIM, typename T> __device__ __forceinline__ T det(const T (&A)[DIM
            A[0][2] * (A[1][0] * A[2][1] - A[1][1] * A[2][0]);
 }
 // B = A^-1, returns det(A)
-template <int DIM, typename T> __device__ __forceinline__ T inverse(const T (&A)[DIM][DIM], T (&B)[DIM][DIM]) {
+template <int DIM, typename T> __host__ __device__ __forceinline__ T inverse(const T (&A)[DIM][DIM], T (&B)[DIM][DIM]) {
   if constexpr (DIM == 2) {
     const T d = A[0][0] * A[1][1] - A[0][1] * A[1][0];
     const T id = T(1) / d;
@@ -1027,7 +1027,7 @@ __device__ __forceinline__ void q1_jacobian(const TC *X, const T *qp, int i0, in
 // of neighbouring vertices keep the digits that q1_jacobian's weighted sums of
 // all eight lose (J ~ h from terms ~ |X|).
 template <int DIM, typename T, typename TC>
-__device__ __forceinline__ void affine_jacobian(const TC *X, T (&J)[DIM][DIM]) {
+__host__ __device__ __forceinline__ void affine_jacobian(const TC *X, T (&J)[DIM][DIM]) {
 #pragma unroll
   for (int i = 0; i < DIM; ++i)
 #pragma unroll
@@ -1149,6 +1149,8 @@ template <typename Number> struct VmultParams {
   double *__restrict__ dlambda;
   const int32_t *__restrict__ perm;
   const double *__restrict__ caff;  // affine compact form: [sorted cell][kAffineStride]
+  // affine cells' geometry, the same layout: det(J_ref), det(J_ref) J_ref^-1 J_ref^-T, J_ref
+  const double *__restrict__ cgeo;
   double qw[3];                     // 1D quadrature weights, the first half (symmetric)
   // even-odd forms of the 1D matrices S and D (EvenOdd<N>::PK values each,
   // N <= 5) for the line-per-lane sum factorization: uniform across lanes,
@@ -1753,6 +1755,10 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
 // with the padded slots 1620 us (LDS bank conflicts 135 -> 22 of 525 kcycles),
 // 1555 us without the unit rows of the 1D matrices.  What is left is issue:
 // VALU and LDS each busy about half the time, nine waves per CU.
+//
+// The residual (one evaluation, of u) and its VJP (u, then w) on affine cells
+// take the same way: 48^3 147 -> 82 us and 206 -> 146 us, relative error of the
+// pair against 64 bits 1.8e-14 -> 1.3e-14.
 // ------------------------------------------------------------------------
 template <int N, typename T> struct PlaneShape {
   // Q2: ten lanes (nine used) and a padded slot per cell, so that planes
@@ -1861,18 +1867,23 @@ template <int N, typename T> struct SFPlane {
   }
 };
 
-// waves per SIMD
-template <int N, typename T> constexpr int planes_min_waves() { return sizeof(T) == 8 ? (N == 3 ? 3 : 2) : 4; }
+// Waves per SIMD: three FP64 workgroups of three waves fill a CU's LDS; the VJP
+// keeps K, ln J and two gradients and spills at 168 VGPRs (48^3: 164 us against
+// 146 with 240).
+template <int N, typename T, int VAR> constexpr int planes_min_waves() {
+  return VAR == V_ADJOINT ? 2 : sizeof(T) == 8 ? 3 : 4;
+}
 
 template <int N, typename T, int VAR, bool ADD, bool CONSTR>
-__global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T>())) k_vmult_planes(const VmultParams<T> P) {
-  static_assert(VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U);
-  constexpr bool AFFINE = VAR != V_COMPACT, RECOMP = VAR == V_COMPACT_U;
+__global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T, VAR>())) k_vmult_planes(const VmultParams<T> P) {
+  constexpr bool RES = VAR == V_RESIDUAL, ADJ = VAR == V_ADJOINT;  // affine cells, nothing cached
+  static_assert(VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U || RES || ADJ);
+  constexpr bool AFFINE = VAR != V_COMPACT, RECOMP = VAR == V_COMPACT_U || RES || ADJ;
   using PS = PlaneShape<N, T>;
   using TS = TileShape<3, N, tile_threads<kTileWide>()>;
   using SF3 = SFPlane<N, T>;
   constexpr int NQP = N * N * N, NL = N * N, TN = TS::TN, WG = PS::WG, PP = N - 1;
-  constexpr int NF = CacheFields<3, VAR>::value;
+  constexpr int NF = CacheFields<3, VAR>::value;  // 0: RES, ADJ
   constexpr int ROUNDS = (TN + WG - 1) / WG;
   constexpr int NCA = RECOMP ? 16 : 7;  // constants per cell
   constexpr int CA = AFFINE ? PS::CPW * NCA : 1;
@@ -1881,6 +1892,7 @@ __global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T
   __shared__ T tile_v[TN * 3];
   __shared__ double caff_all[CA];
   __shared__ T tile_u[RECOMP ? TN * 3 : 1];
+  __shared__ T red[ADJ ? PS::CPW * 2 * NL : 1];  // columns' shares of dmu, dlambda
   const T *src = P.src + (size_t)blockIdx.y * P.vstride;  // an epilogue updates it in place
   T *dst = P.dst + (size_t)blockIdx.y * P.vstride;
   const int t = threadIdx.x, wave = t / 64, lane = t % 64;
@@ -1912,7 +1924,7 @@ __global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T
     const bool valid = tcode[k] != kNoNode;
     const size_t node = valid ? tcode[k] & kNodeMask : 0;
     if constexpr (RECOMP) load_node<3, T>(P.u + node * 3, uv[k]);
-    load_node<3, T>(src + node * 3, sv[k]);
+    if constexpr (!RES) load_node<3, T>(src + node * 3, sv[k]);
 #pragma unroll
     for (int c = 0; c < 3; ++c) dv[k][c] = T(0);
     if (valid && (ADD ? !tshared[k] : !P.tbuf && !(tcode[k] & kFirstBit))) load_node<3, T>(dst + node * 3, dv[k]);
@@ -1925,13 +1937,19 @@ __global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T
 #pragma unroll
     for (int k = 0; k < CROUNDS; ++k) {
       const int i = t + k * WG < n_ca ? t + k * WG : 0;
-      ca[k] = P.caff[(size_t)(first + i / NCA) * kAffineStride + i % NCA];
+      ca[k] = (RES || ADJ ? P.cgeo : P.caff)[(size_t)(first + i / NCA) * kAffineStride + i % NCA];
     }
   __builtin_amdgcn_sched_barrier(0);
-  T cch[N][NF];
+  T cch[N][NF > 0 ? NF : 1];
   const size_t cq = (size_t)cell * NQP + (col ? j : 0);
+  if constexpr (NF > 0)
 #pragma unroll
-  for (int k = 0; k < N; ++k) load_cache<T, NF>(P.cache, cq + k * NL, P.fs, cch[k]);
+    for (int k = 0; k < N; ++k) load_cache<T, NF>(P.cache, cq + k * NL, P.fs, cch[k]);
+  T mu = T(0), lambda = T(0);
+  if constexpr (RES || ADJ) {
+    mu = P.mu[cell];
+    lambda = P.lambda[cell];
+  }
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (AFFINE)
 #pragma unroll
@@ -1944,7 +1962,7 @@ __global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         const bool zero = tcode[k] == kNoNode || (CONSTR && ((tcode[k] >> (kConsShift + c)) & 1u));
-        tile_v[n * 3 + c] = zero ? T(0) : sv[k][c];
+        tile_v[n * 3 + c] = RES ? dv[k][c] : zero ? T(0) : sv[k][c];
         if constexpr (RECOMP) tile_u[n * 3 + c] = uv[k][c];
       }
   }
@@ -1962,6 +1980,8 @@ __global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T
   };
   const double *cell_c = caff_all + (AFFINE && has ? slot * NCA : 0);
   T K[RECOMP ? N : 1][9];
+  const double wxy = AFFINE ? weight_1d<N>(P.qw, j % N) * weight_1d<N>(P.qw, (j / N) % N) : 0.0;
+  auto point_weight = [&](int k) { return wxy * P.qw[k < N - 1 - k ? k : N - 1 - k]; };
   if constexpr (RECOMP) {
     // K = (J_ref + Grad_xi u)^-1 at the column's points
     if (pln) {
@@ -1981,61 +2001,121 @@ __global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T
         for (int i = 0; i < 3; ++i)
 #pragma unroll
           for (int d = 0; d < 3; ++d) Jc[i][d] = T(cell_c[7 + 3 * i + d]) + G[i][d][k];
-        inverse<3>(Jc, Ki);
+        const T dc = inverse<3>(Jc, Ki);
+        if constexpr (RES) {
+          // -(tau F^-T) J_ref^-T dw = -(Jc A - c dw K^T), A = mu dw R R^T
+          // (mu F F^T K^T = mu F R^T and F = Jc R)
+          const T w = T(point_weight(k)), dw = cell_c[0] * w, mw = mu * w;
+          const T cdw = (mu - T(2) * lambda * T(log(double(dc / cell_c[0])))) * dw;
 #pragma unroll
-        for (int d = 0; d < 3; ++d)
+          for (int i = 0; i < 3; ++i)
 #pragma unroll
-          for (int c = 0; c < 3; ++c) K[k][3 * d + c] = Ki[d][c];
+            for (int d = 0; d < 3; ++d) {
+              T s = T(0);
+#pragma unroll
+              for (int e = 0; e < 3; ++e) s = fma(Jc[i][e], cell_c[1 + voigt_index<3>(e, d)], s);
+              G[i][d][k] = fma(cdw, Ki[d][i], -mw * s);
+            }
+        } else {
+          if constexpr (ADJ) cch[k][0] = T(log(double(dc / cell_c[0])));
+#pragma unroll
+          for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) K[k][3 * d + c] = Ki[d][c];
+        }
       }
+      if constexpr (RES)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) SF3::integrate_column(P.sf, A + c * NQP + j, G[c]);
     }
     wave_lds_fence();
   }
-  {
-    T x[N][N];
-    if (pln) gather(tile_v, x);
-    lds_barrier();
-    // every lane has gathered: the tile's destination values take the source
-    // values' place
+  if constexpr (!RES) {
+    {
+      T x[N][N];
+      if (pln) gather(tile_v, x);
+      lds_barrier();
+      // every lane has gathered: the tile's destination values take the source
+      // values' place
 #pragma unroll
-    for (int k = 0; k < ROUNDS; ++k)
-      if (t + k * WG < TN)
+      for (int k = 0; k < ROUNDS; ++k)
+        if (t + k * WG < TN)
 #pragma unroll
-        for (int c = 0; c < 3; ++c) tile_v[(t + k * WG) * 3 + c] = dv[k][c];
-    if (pln) SF3::evaluate_plane(P.sf, plane, x);
-  }
-  wave_lds_fence();
-  if (col) {
-    T G[3][3][N];
+          for (int c = 0; c < 3; ++c) tile_v[(t + k * WG) * 3 + c] = dv[k][c];
+      if (pln) SF3::evaluate_plane(P.sf, plane, x);
+    }
+    wave_lds_fence();
+    if (col) {
+      T G[3][3][N], dmu = T(0), dlam = T(0);
 #pragma unroll
-    for (int c = 0; c < 3; ++c) SF3::evaluate_column(P.sf, A + c * NQP + j, G[c]);
-    const double wxy = AFFINE ? weight_1d<N>(P.qw, j % N) * weight_1d<N>(P.qw, j / N) : 0.0;
+      for (int c = 0; c < 3; ++c) SF3::evaluate_column(P.sf, A + c * NQP + j, G[c]);
 #pragma unroll
-    for (int k = 0; k < N; ++k) {
-      T g[3][3], Phi[3][3];
+      for (int k = 0; k < N; ++k) {
+        T g[3][3], Phi[3][3];
 #pragma unroll
-      for (int c = 0; c < 3; ++c)
+        for (int c = 0; c < 3; ++c)
 #pragma unroll
-        for (int d = 0; d < 3; ++d) g[c][d] = G[c][d][k];
-      if constexpr (VAR == V_COMPACT) {
-        qp_compact<3, T>(g, cch[k], cch[k][9], cch[k][10], cch[k] + 11, Phi);
-      } else {
-        const double w = wxy * P.qw[k < N - 1 - k ? k : N - 1 - k];
-        T aw[7];
+          for (int d = 0; d < 3; ++d) g[c][d] = G[c][d][k];
+        if constexpr (VAR == V_COMPACT) {
+          qp_compact<3, T>(g, cch[k], cch[k][9], cch[k][10], cch[k] + 11, Phi);
+        } else {
+          const double w = point_weight(k);
+          T aw[7];
 #pragma unroll
-        for (int q = 0; q < 7; ++q) aw[q] = T(cell_c[q] * w);
-        if constexpr (RECOMP) qp_compact<3, T>(g, K[k], cch[k][0], aw[0], aw + 1, Phi);
-        else qp_compact<3, T>(g, cch[k], cch[k][9], aw[0], aw + 1, Phi);
+          for (int q = 0; q < 7; ++q) aw[q] = T(cell_c[q] * w);
+          if constexpr (ADJ) {
+            // du = -A w, dmu = -sum (b - I) : g dw, dlambda = -sum 2 ln J tr g dw
+            // with g = G K: tr g = tr(K G), b : g dw = Jc B : G w, B = det R R^T
+            const T lnJ = cch[k][0], dw = aw[0];
+            T tr = T(0), bg = T(0), Ki[3][3], Jc[3][3];
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+              for (int c = 0; c < 3; ++c) {
+                Ki[d][c] = K[k][3 * d + c];
+                tr = fma(Ki[d][c], g[c][d], tr);
+              }
+            inverse<3>(Ki, Jc);
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+              for (int d = 0; d < 3; ++d) {
+                T s = T(0);
+#pragma unroll
+                for (int e = 0; e < 3; ++e) s = fma(Jc[i][e], aw[1 + voigt_index<3>(e, d)], s);
+                bg = fma(s, g[i][d], bg);
+              }
+            dmu -= bg - tr * dw;
+            dlam -= T(2) * lnJ * tr * dw;
+#pragma unroll
+            for (int q = 1; q < 7; ++q) aw[q] *= -mu;
+            qp_compact<3, T>(g, K[k], -(mu - T(2) * lambda * lnJ) * dw, T(-2) * lambda * dw, aw + 1, Phi);
+          } else if constexpr (RECOMP) qp_compact<3, T>(g, K[k], cch[k][0], aw[0], aw + 1, Phi);
+          else qp_compact<3, T>(g, cch[k], cch[k][9], aw[0], aw + 1, Phi);
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) G[c][d][k] = Phi[c][d];
       }
 #pragma unroll
-      for (int c = 0; c < 3; ++c)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) G[c][d][k] = Phi[c][d];
+      for (int c = 0; c < 3; ++c) SF3::integrate_column(P.sf, A + c * NQP + j, G[c]);
+      if constexpr (ADJ) {
+        red[slot * 2 * NL + j] = dmu;
+        red[slot * 2 * NL + NL + j] = dlam;
+      }
     }
-#pragma unroll
-    for (int c = 0; c < 3; ++c) SF3::integrate_column(P.sf, A + c * NQP + j, G[c]);
   }
   wave_lds_fence();
   if (pln) SF3::integrate_plane(P.sf, plane);
+  if constexpr (ADJ)
+    if (has && j < 2) {
+      // the cell's columns in order (same wave)
+      T s = T(0);
+#pragma unroll
+      for (int q = 0; q < NL; ++q) s += red[slot * 2 * NL + j * NL + q];
+      (j == 0 ? P.dmu : P.dlambda)[P.perm[cell]] = double(s);
+    }
   lds_barrier();
   // sum the cells' results per tile node (fixed order), one write per node
 #pragma unroll

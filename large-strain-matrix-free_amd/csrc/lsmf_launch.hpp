@@ -23,6 +23,9 @@ template <int DIM, int N> struct Launch {
   template <int VAR> static constexpr bool planes_ok() {
     return DIM == 3 && N == 3 && (VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U);
   }
+  template <typename T, int VAR> static constexpr bool kinematic_planes() {
+    return DIM == 3 && N == 3 && sizeof(T) == 8 && (VAR == V_RESIDUAL || VAR == V_ADJOINT);
+  }
   // K from the displacement: that kernel only (cache_variant)
   static constexpr bool recompute_ok() { return DIM == 3 && N == 3; }
 
@@ -31,8 +34,20 @@ template <int DIM, int N> struct Launch {
   template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
   static int launch_vmult(const lsmf_op *op, const VmultParams<T> &P, int n, unsigned nv, hipStream_t s) {
     if (op->tile_kind == kTileWide) {
-      if constexpr (planes_ok<VAR>() && PH == (PH_SF | PH_QD))
+      if constexpr (planes_ok<VAR>() && PH == (PH_SF | PH_QD)) {
         hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR>), dim3(n, nv), dim3((PlaneShape<N, T>::WG)), 0, s, P);
+        return 0;
+      }
+      if constexpr (kinematic_planes<T, VAR>()) {
+        // residual and VJP in formulation 1 on affine cells
+        if (op->d_cgeo && op->formulation == 1) {
+          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR>), dim3(n, nv), dim3((PlaneShape<N, T>::WG)), 0,
+                             s, P);
+          return 0;
+        }
+      }
+      if constexpr (planes_ok<VAR>() && PH == (PH_SF | PH_QD))
+        return LSMF_ERR_UNSUPPORTED;
       else if constexpr (wide_ok<VAR>())
         hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide>), dim3(n, nv),
                            dim3(tile_threads<kTileWide>()), 0, s, P);
@@ -99,6 +114,7 @@ template <int DIM, int N> struct Launch {
     P.dlambda = op->adj_dlambda;
     P.perm = op->d_perm;
     P.caff = op->d_caff;
+    P.cgeo = op->d_cgeo;
     for (int k = 0; k < 3; ++k) P.qw[k] = op->h_qw[k];
     static_assert(sizeof(P.sf) / sizeof(P.sf[0]) >= 2 * EvenOdd<N, T>::PK, "1D matrices do not fit the kernel arguments");
     pack_sf<T>(op, P.sf);

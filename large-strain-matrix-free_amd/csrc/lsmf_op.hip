@@ -146,7 +146,7 @@ template <typename T> int dalloc(T **p, size_t n, const char *what) {
 }
 
 void free_op(lsmf_op *op) {
-  void *ptrs[] = {op->d_uc,   op->d_idx,  op->d_coords,    op->d_tab,  op->d_tab64, op->d_mu64,     op->d_lambda64,
+  void *ptrs[] = {op->d_cgeo, op->d_uc,   op->d_idx,  op->d_coords,    op->d_tab,  op->d_tab64, op->d_mu64,     op->d_lambda64,
                   op->d_mu,   op->d_lambda,    op->d_cache, op->d_caff, op->d_diag, op->d_inv_diag, op->d_cons,
                   op->d_bad,  op->d_perm,      op->d_tile_nodes, op->d_tile_info, op->d_tile_tables,
                   op->d_tile_buf, op->d_orphan, op->d_hang, op->d_hptr,
@@ -972,6 +972,28 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
   for (int i = 0; i < 2 * N * N; ++i) op->h_sf[i] = tab[i];
   for (int k = 0; k < (N + 1) / 2; ++k) op->h_qw[k] = t1.qw[k];
 
+  // affine cells' geometry for the residual and its VJP on wide Q2 tiles
+  std::vector<double> cgeo;
+  if (recompute_k(op)) {
+    cgeo.resize((size_t)nc * kAffineStride);
+    int corner[8];
+    for (int v = 0; v < 8; ++v) corner[v] = p * ((v & 1) + N * ((v >> 1 & 1) + N * (v >> 2 & 1)));
+    for (int pos = 0; pos < nc; ++pos) {
+      const int32_t *cn = mesh->cell_nodes + (size_t)op->perm[pos] * nqp;
+      double X[24], J[3][3], R[3][3];
+      for (int v = 0; v < 8; ++v)
+        for (int i = 0; i < 3; ++i) X[v * 3 + i] = mesh->coords[(size_t)cn[corner[v]] * 3 + i];
+      affine_jacobian<3>(X, J);
+      double *g = &cgeo[(size_t)pos * kAffineStride];
+      g[0] = inverse<3>(J, R);
+      for (int v = 0; v < 6; ++v) {
+        const int i = voigt_first<3>(v), j = voigt_second<3>(v);
+        g[1 + v] = g[0] * (R[i][0] * R[j][0] + R[i][1] * R[j][1] + R[i][2] * R[j][2]);
+      }
+      for (int i = 0; i < 3; ++i)
+        for (int d = 0; d < 3; ++d) g[7 + 3 * i + d] = J[i][d];
+    }
+  }
   // the tile tables in one piece: tiles by colour, private bits, shared nodes, slots
   std::vector<uint32_t> tile_tables(tt.list.begin(), tt.list.end());
   for (const auto *v : {&tt.priv, &tt.sum_node, &tt.sum_slot}) tile_tables.insert(tile_tables.end(), v->begin(), v->end());
@@ -988,6 +1010,7 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
       (rc = dalloc(&op->d_u64, op->n_dofs, "displacement")) ||
       (rc = dalloc((char **)&op->d_cache, (size_t)op->n_fields * op->field_stride * es, "cache")) ||
       (cache_variant(op) == V_COMPACT_U && (rc = dalloc((char **)&op->d_uc, op->n_dofs * es, "cached displacement"))) ||
+      (!cgeo.empty() && (rc = dalloc(&op->d_cgeo, cgeo.size(), "cell geometry"))) ||
       (cell_constants(op) &&
        (rc = dalloc(&op->d_caff, (size_t)nc * kAffineStride, "cell constants"))) ||
       (rc = dalloc((char **)&op->d_diag, op->n_dofs * es, "diagonal")) ||
@@ -1063,6 +1086,9 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
     e = hipMemcpy(op->d_tile_nodes, tt.nodes.data(), tt.nodes.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
   if (e == hipSuccess && !tt.info.empty())
     e = hipMemcpy(op->d_tile_info, tt.info.data(), tt.info.size() * sizeof(int32_t), hipMemcpyHostToDevice);
+  if (e == hipSuccess && !cgeo.empty())
+    e = hipMemcpy(op->d_cgeo, cgeo.data(), cgeo.size() * sizeof(double), hipMemcpyHostToDevice);
+  op->bytes_idx += cgeo.size() * sizeof(double);
   if (e == hipSuccess && !tile_tables.empty()) {
     e = hipMemcpy(op->d_tile_tables, tile_tables.data(), tile_tables.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
     op->d_tile_list = reinterpret_cast<const int32_t *>(op->d_tile_tables);

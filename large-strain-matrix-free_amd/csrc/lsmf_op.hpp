@@ -77,6 +77,7 @@ struct lsmf_op {
   void *d_cache = nullptr;
   double *d_caff = nullptr;         // affine compact form: [sorted cell][kAffineStride]
   void *d_uc = nullptr;             // u of the last cache() where the products recompute K from it
+  double *d_cgeo = nullptr;         // affine cells' geometry (VmultParams::cgeo), where the residual uses it
   void *d_diag = nullptr, *d_inv_diag = nullptr;
   int32_t *d_cons = nullptr;        // constrained DoF list
   int n_cons = 0;

@@ -125,3 +125,36 @@ def test_products_keep_the_cached_state(device):
     op.cache()
     op.vmult(ys[0], x)
     assert rel(ys[0].cpu().numpy(), oracle_op(mesh, mu, lam, 0 * u, cons, "tensor4").vmult(x.cpu().numpy())) < 1e-12
+
+
+@pytest.mark.parametrize("geometry", ["sheared", "cook"])
+@pytest.mark.parametrize("n", [[1, 1, 1], [9, 2, 1], [10, 3, 5], [19, 5, 2]], ids=str)
+def test_residual_and_vjp(n, geometry, device):
+    """internal forces against the oracle; du of the VJP is -A w (oracle), and
+    w . R is linear in each cell's mu and lambda with coefficients dmu, dlambda"""
+    import torch
+    print(f"[residual] n={n} {geometry}", flush=True)
+    mesh, mu, lam, u, cons = problem(3, 2, n, geometry)
+    op = lsmf.NeoHookOperator(mesh, caching="tensor4", constrained=cons)
+    op.set_linearization(torch.tensor(u, device=device))
+
+    def residual(m, l):
+        op.set_material(m, l)
+        r = torch.full((mesh.n_dofs,), float("nan"), dtype=torch.float64, device=device)
+        op.residual(r)
+        return r.cpu().numpy()
+
+    rng = np.random.default_rng(6)
+    w, hm, hl = rng.standard_normal(mesh.n_dofs), rng.random(mesh.n_cells), rng.random(mesh.n_cells)
+    base, more_mu, more_lam = residual(mu, lam), residual(mu + hm, lam), residual(mu, lam + hl)
+    ref = oracle_op(mesh, mu, lam, u, cons, "tensor4")
+    expect = ref.residual()
+    assert np.abs(base - expect).max() < 1e-12 * np.abs(expect).max()
+    op.set_material(mu, lam)
+    du = torch.full((mesh.n_dofs,), float("nan"), dtype=torch.float64, device=device)
+    dmu, dlam = (torch.full((mesh.n_cells,), float("nan"), dtype=torch.float64, device=device) for _ in range(2))
+    op.residual_vjp(torch.tensor(w, device=device), du, dmu, dlam)
+    assert rel(du.cpu().numpy(), -ref.vmult(w, plain=True)) < 1e-12
+    for h, other, grad in ((hm, more_mu, dmu), (hl, more_lam, dlam)):
+        terms = w * (other - base)  # rounding of the difference of two residuals
+        assert abs(float(h @ grad.cpu().numpy()) - terms.sum()) < 1e-12 * np.abs(w * base).sum()
