@@ -1758,14 +1758,16 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
 //
 // The residual (one evaluation, of u) and its VJP (u, then w) on affine cells
 // take the same way: 48^3 147 -> 82 us and 206 -> 146 us, relative error of the
-// pair against 64 bits 1.8e-14 -> 1.3e-14.
+// pair against 64 bits 1.8e-14 -> 1.3e-14.  So does the scalar form (c cached)
+// on its 9x1x1 tiles: 48^3 FP64 212 -> 138 us, FP32 122 -> 85 us, and the FP32
+// error falls from 1.9e-6 to 1.7e-7 (no tau = mu F F^T - c I to cancel).
 // ------------------------------------------------------------------------
-template <int N, typename T> struct PlaneShape {
+template <int N, typename T, int TILE> struct PlaneShape {
   // Q2: ten lanes (nine used) and a padded slot per cell, so that planes
   // (lanes 9 values apart) and columns (neighbours) spread over all banks
   static constexpr int LPC = N == 3 ? 10 : N * N;  // lanes per cell
   static constexpr int CPV = 64 / LPC;             // cells per wave
-  static constexpr int CPW = TileShape<3, N, tile_threads<kTileWide>()>::CPW;
+  static constexpr int CPW = TileShape<3, N, tile_threads<TILE>()>::CPW;
   static constexpr int WAVES = (CPW + CPV - 1) / CPV;
   static constexpr int WG = 64 * WAVES;
   static constexpr int SLOT = N == 3 ? (sizeof(T) == 8 ? 250 : 266) : 9 * N * N * N;
@@ -1874,13 +1876,14 @@ template <int N, typename T, int VAR> constexpr int planes_min_waves() {
   return VAR == V_ADJOINT ? 2 : sizeof(T) == 8 ? 3 : 4;
 }
 
-template <int N, typename T, int VAR, bool ADD, bool CONSTR>
-__global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T, VAR>())) k_vmult_planes(const VmultParams<T> P) {
+template <int N, typename T, int VAR, bool ADD, bool CONSTR, int TILE>
+__global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_waves<N, T, VAR>())) k_vmult_planes(const VmultParams<T> P) {
   constexpr bool RES = VAR == V_RESIDUAL, ADJ = VAR == V_ADJOINT;  // affine cells, nothing cached
-  static_assert(VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U || RES || ADJ);
-  constexpr bool AFFINE = VAR != V_COMPACT, RECOMP = VAR == V_COMPACT_U || RES || ADJ;
-  using PS = PlaneShape<N, T>;
-  using TS = TileShape<3, N, tile_threads<kTileWide>()>;
+  constexpr bool SCAL = VAR == V_SCALAR, GEO = RES || ADJ || SCAL;  // affine cells, c cached; cgeo and material
+  static_assert(VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U || GEO);
+  constexpr bool AFFINE = VAR != V_COMPACT, RECOMP = VAR == V_COMPACT_U || GEO;
+  using PS = PlaneShape<N, T, TILE>;
+  using TS = TileShape<3, N, tile_threads<TILE>()>;
   using SF3 = SFPlane<N, T>;
   constexpr int NQP = N * N * N, NL = N * N, TN = TS::TN, WG = PS::WG, PP = N - 1;
   constexpr int NF = CacheFields<3, VAR>::value;  // 0: RES, ADJ
@@ -1937,7 +1940,7 @@ __global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T
 #pragma unroll
     for (int k = 0; k < CROUNDS; ++k) {
       const int i = t + k * WG < n_ca ? t + k * WG : 0;
-      ca[k] = (RES || ADJ ? P.cgeo : P.caff)[(size_t)(first + i / NCA) * kAffineStride + i % NCA];
+      ca[k] = (GEO ? P.cgeo : P.caff)[(size_t)(first + i / NCA) * kAffineStride + i % NCA];
     }
   __builtin_amdgcn_sched_barrier(0);
   T cch[N][NF > 0 ? NF : 1];
@@ -1946,7 +1949,7 @@ __global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T
 #pragma unroll
     for (int k = 0; k < N; ++k) load_cache<T, NF>(P.cache, cq + k * NL, P.fs, cch[k]);
   T mu = T(0), lambda = T(0);
-  if constexpr (RES || ADJ) {
+  if constexpr (GEO) {
     mu = P.mu[cell];
     lambda = P.lambda[cell];
   }
@@ -2090,6 +2093,11 @@ __global__ void __launch_bounds__((PlaneShape<N, T>::WG), (planes_min_waves<N, T
 #pragma unroll
             for (int q = 1; q < 7; ++q) aw[q] *= -mu;
             qp_compact<3, T>(g, K[k], -(mu - T(2) * lambda * lnJ) * dw, T(-2) * lambda * dw, aw + 1, Phi);
+          } else if constexpr (SCAL) {
+            const T dw = aw[0];
+#pragma unroll
+            for (int q = 1; q < 7; ++q) aw[q] *= mu;
+            qp_compact<3, T>(g, K[k], cch[k][0] * dw, T(2) * lambda * dw, aw + 1, Phi);
           } else if constexpr (RECOMP) qp_compact<3, T>(g, K[k], cch[k][0], aw[0], aw + 1, Phi);
           else qp_compact<3, T>(g, cch[k], cch[k][9], aw[0], aw + 1, Phi);
         }

@@ -35,13 +35,15 @@ template <int DIM, int N> struct Launch {
   static int launch_vmult(const lsmf_op *op, const VmultParams<T> &P, int n, unsigned nv, hipStream_t s) {
     if (op->tile_kind == kTileWide) {
       if constexpr (planes_ok<VAR>() && PH == (PH_SF | PH_QD)) {
-        hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR>), dim3(n, nv), dim3((PlaneShape<N, T>::WG)), 0, s, P);
+        hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide>), dim3(n, nv),
+                           dim3((PlaneShape<N, T, kTileWide>::WG)), 0, s, P);
         return 0;
       }
       if constexpr (kinematic_planes<T, VAR>()) {
         // residual and VJP in formulation 1 on affine cells
         if (op->d_cgeo && op->formulation == 1) {
-          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR>), dim3(n, nv), dim3((PlaneShape<N, T>::WG)), 0,
+          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide>), dim3(n, nv),
+                           dim3((PlaneShape<N, T, kTileWide>::WG)), 0,
                              s, P);
           return 0;
         }
@@ -56,6 +58,14 @@ template <int DIM, int N> struct Launch {
     } else if constexpr (VAR == V_COMPACT_U) {
       return LSMF_ERR_UNSUPPORTED;
     } else if (op->tile_kind == 1) {
+      if constexpr (DIM == 3 && N == 3 && VAR == V_SCALAR && PH == (PH_SF | PH_QD)) {
+        // formulation 1 on affine cells with the Q1 metric
+        if (op->d_cgeo && op->formulation == 1) {
+          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, 1>), dim3(n, nv),
+                             dim3((PlaneShape<N, T, 1>::WG)), 0, s, P);
+          return 0;
+        }
+      }
       hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, 1>), dim3(n, nv), dim3(kWG), 0, s, P);
     } else {
       hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, 0>), dim3(grid_for(n), nv), dim3(kWG), 0, s, P);

@@ -972,9 +972,11 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
   for (int i = 0; i < 2 * N * N; ++i) op->h_sf[i] = tab[i];
   for (int k = 0; k < (N + 1) / 2; ++k) op->h_qw[k] = t1.qw[k];
 
-  // affine cells' geometry for the residual and its VJP on wide Q2 tiles
+  // affine cells' geometry: residual and VJP on wide Q2 tiles, scalar products
+  // on the others
   std::vector<double> cgeo;
-  if (recompute_k(op)) {
+  if (recompute_k(op) || (op->caching == LSMF_CACHING_SCALAR && op->tile_kind == 1 && dim == 3 && N == 3 &&
+                          op->affine && !op->curved)) {
     cgeo.resize((size_t)nc * kAffineStride);
     int corner[8];
     for (int v = 0; v < 8; ++v) corner[v] = p * ((v & 1) + N * ((v >> 1 & 1) + N * (v >> 2 & 1)));

@@ -158,3 +158,25 @@ def test_residual_and_vjp(n, geometry, device):
     for h, other, grad in ((hm, more_mu, dmu), (hl, more_lam, dlam)):
         terms = w * (other - base)  # rounding of the difference of two residuals
         assert abs(float(h @ grad.cpu().numpy()) - terms.sum()) < 1e-12 * np.abs(w * base).sum()
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("fp32", 2e-5)])
+@pytest.mark.parametrize("n", [[1, 1, 1], [9, 1, 1], [10, 3, 5], [19, 2, 2]], ids=str)
+@pytest.mark.parametrize("geometry", ["sheared", "cook"])
+def test_scalar_products(n, geometry, precision, tol, device):
+    """scalar caching on affine cells (planes and columns) and on bilinear ones,
+    formulation 1, then 0, then 1 again, against the oracle"""
+    import torch
+    print(f"[scalar] n={n} {geometry} {precision}", flush=True)
+    mesh, mu, lam, u, cons = problem(3, 2, n, geometry)
+    op = lsmf.NeoHookOperator(mesh, precision=precision, caching="scalar", constrained=cons)
+    op.set_material(mu, lam)
+    v = np.random.default_rng(4).standard_normal(mesh.n_dofs).astype(np.float32).astype(np.float64)
+    for formulation in (1, 0, 1):
+        assert lsmf._lib.lsmf_set_formulation(op._h, formulation) == lsmf.LSMF_OK
+        op.set_linearization(torch.tensor(u, device=device))
+        op.cache()
+        expect = oracle_op(mesh, mu, lam, u, cons, "scalar", formulation).vmult(v)
+        y = torch.full((mesh.n_dofs,), float("nan"), dtype=op.dtype, device=device)
+        op.vmult(y, torch.tensor(v, device=device).to(op.dtype))
+        assert rel(y.double().cpu().numpy(), expect) < tol, formulation
