@@ -216,7 +216,10 @@ lsmf_status lsmf_compute_diagonal(lsmf_op *op, lsmf_stream stream);
  * (include/mf_nh_operator.h:612-706): dst = A src (add = 0) or dst += A src
  * (add != 0).  Constrained rows act as identity (:703-705) unless
  * LSMF_MASK_PLAIN.  The operator is symmetric, so Tvmult = vmult.  dst and
- * src must not alias. */
+ * src must not alias.  Tiled operators of up to 4 M DoF run a product in one
+ * launch over all tiles on the first stream that uses the operator; calls on
+ * other streams and captured calls take one launch per tile colour, with the
+ * same results, so products on several streams share no state. */
 lsmf_status lsmf_vmult(lsmf_op *op, void *dst, const void *src, int add, unsigned mask, lsmf_stream stream);
 
 /* n_vectors products dst_b = A src_b of lsmf_vmult (set mode, constrained

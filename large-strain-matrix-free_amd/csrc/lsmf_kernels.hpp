@@ -1,5 +1,5 @@
 // lsmf_kernels.hpp -- HIP kernels of the matrix-free Neo-Hookean tangent for
-// gfx950 (MI355X), one fused kernel per cell colour:
+// gfx950 (MI355X), one fused kernel per cell colour or over all tiles:
 //   gather (index table with constraint bits) -> LDS
 //   -> sum-factorized gradient (1D matrices, one thread per quadrature point)
 //   -> pointwise tangent (scalar / tensor2 / tensor4 caches, FP64 or FP32)
