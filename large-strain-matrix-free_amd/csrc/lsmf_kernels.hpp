@@ -1149,7 +1149,8 @@ template <typename Number> struct VmultParams {
   double *__restrict__ dlambda;
   const int32_t *__restrict__ perm;
   const double *__restrict__ caff;  // affine compact form: [sorted cell][kAffineStride]
-  // affine cells' geometry, the same layout: det(J_ref), det(J_ref) J_ref^-1 J_ref^-T, J_ref
+  // affine cells' geometry, the same layout: det(J_ref), det(J_ref) J_ref^-1 J_ref^-T and
+  // J_ref^-1 (residual and VJP, wide tiles) or J_ref (scalar products)
   const double *__restrict__ cgeo;
   double qw[3];                     // 1D quadrature weights, the first half (symmetric)
   // even-odd forms of the 1D matrices S and D (EvenOdd<N>::PK values each,
@@ -1757,8 +1758,10 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
 // VALU and LDS each busy about half the time, nine waves per CU.
 //
 // The residual (one evaluation, of u) and its VJP (u, then w) on affine cells
-// take the same way: 48^3 147 -> 82 us and 206 -> 146 us, relative error of the
-// pair against 64 bits 1.8e-14 -> 1.3e-14.  So does the scalar form (c cached)
+// take the same way: 48^3 pair 377 -> 276 us, relative error against 64 bits
+// 1.1e-14 -> 6.1e-15.  Both evaluate F and tau as k_vmult does: the shorter flux
+// Jc A - c dw K^T (267 us) is a difference of terms that cancel without strain
+// and left 1e-16 there.  So does the scalar form (c cached)
 // on its 9x1x1 tiles: 48^3 FP64 212 -> 138 us, FP32 122 -> 85 us, and the FP32
 // error falls from 1.9e-6 to 1.7e-7 (no tau = mu F F^T - c I to cancel).
 // ------------------------------------------------------------------------
@@ -1982,11 +1985,26 @@ __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_wave
       for (int i = 0; i < N; ++i) x[y][i] = v[origin + (y * TS::NX + i) * 3];
   };
   const double *cell_c = caff_all + (AFFINE && has ? slot * NCA : 0);
-  T K[RECOMP ? N : 1][9];
+  T K[RECOMP ? N : 1][9];  // ADJ: Grad_xi u
   const double wxy = AFFINE ? weight_1d<N>(P.qw, j % N) * weight_1d<N>(P.qw, (j / N) % N) : 0.0;
   auto point_weight = [&](int k) { return wxy * P.qw[k < N - 1 - k ? k : N - 1 - k]; };
+  // RES, ADJ: F = I + Grad_xi u R, K = R F^-1 with R = J_ref^-1; returns det F.
+  // Like tau and b - I from F, exact without strain: F = I there to the last bit.
+  auto deformation = [&](const T (&Gu)[3][3], T (&F)[3][3], T (&Kr)[3][3]) {
+    T R[3][3], Fi[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) R[i][d] = T(cell_c[7 + 3 * i + d]);
+    grad_times<3>(Gu, R, F);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) F[i][i] += T(1);
+    const T J = inverse<3>(F, Fi);
+    grad_times<3>(R, Fi, Kr);
+    return J;
+  };
   if constexpr (RECOMP) {
-    // K = (J_ref + Grad_xi u)^-1 at the column's points
+    // Grad_xi u at the column's points, K = (J_ref + Grad_xi u)^-1
     if (pln) {
       T x[N][N];
       gather(tile_u, x);
@@ -1999,28 +2017,42 @@ __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_wave
       for (int c = 0; c < 3; ++c) SF3::evaluate_column(P.sf, A + c * NQP + j, G[c]);
 #pragma unroll
       for (int k = 0; k < N; ++k) {
-        T Jc[3][3], Ki[3][3];
+        T Gk[3][3];
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
-          for (int d = 0; d < 3; ++d) Jc[i][d] = T(cell_c[7 + 3 * i + d]) + G[i][d][k];
-        const T dc = inverse<3>(Jc, Ki);
+          for (int d = 0; d < 3; ++d) Gk[i][d] = G[i][d][k];
         if constexpr (RES) {
-          // -(tau F^-T) J_ref^-T dw = -(Jc A - c dw K^T), A = mu dw R R^T
-          // (mu F F^T K^T = mu F R^T and F = Jc R)
-          const T w = T(point_weight(k)), dw = cell_c[0] * w, mw = mu * w;
-          const T cdw = (mu - T(2) * lambda * T(log(double(dc / cell_c[0])))) * dw;
+          // -tau K^T dw
+          T F[3][3], Kr[3][3], tau[3][3], Phi[3][3];
+          const T J = deformation(Gk, F, Kr);
+          const T dw = cell_c[0] * point_weight(k), cs = mu - T(2) * lambda * T(log(double(J)));
+#pragma unroll
+          for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int b = 0; b < 3; ++b) {
+              T s = F[a][0] * F[b][0];
+#pragma unroll
+              for (int e = 1; e < 3; ++e) s = fma(F[a][e], F[b][e], s);
+              tau[a][b] = mu * s - (a == b ? cs : T(0));
+            }
+          flux_times_kt<3>(tau, Kr, Phi);
 #pragma unroll
           for (int i = 0; i < 3; ++i)
 #pragma unroll
-            for (int d = 0; d < 3; ++d) {
-              T s = T(0);
+            for (int d = 0; d < 3; ++d) G[i][d][k] = -Phi[i][d] * dw;
+        } else if constexpr (ADJ) {
 #pragma unroll
-              for (int e = 0; e < 3; ++e) s = fma(Jc[i][e], cell_c[1 + voigt_index<3>(e, d)], s);
-              G[i][d][k] = fma(cdw, Ki[d][i], -mw * s);
-            }
+          for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) K[k][3 * i + d] = Gk[i][d];
         } else {
-          if constexpr (ADJ) cch[k][0] = T(log(double(dc / cell_c[0])));
+          T Jc[3][3], Ki[3][3];
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) Jc[i][d] = T(cell_c[7 + 3 * i + d]) + Gk[i][d];
+          inverse<3>(Jc, Ki);
 #pragma unroll
           for (int d = 0; d < 3; ++d)
 #pragma unroll
@@ -2068,31 +2100,30 @@ __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_wave
           for (int q = 0; q < 7; ++q) aw[q] = T(cell_c[q] * w);
           if constexpr (ADJ) {
             // du = -A w, dmu = -sum (b - I) : g dw, dlambda = -sum 2 ln J tr g dw
-            // with g = G K: tr g = tr(K G), b : g dw = Jc B : G w, B = det R R^T
-            const T lnJ = cch[k][0], dw = aw[0];
-            T tr = T(0), bg = T(0), Ki[3][3], Jc[3][3];
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-#pragma unroll
-              for (int c = 0; c < 3; ++c) {
-                Ki[d][c] = K[k][3 * d + c];
-                tr = fma(Ki[d][c], g[c][d], tr);
-              }
-            inverse<3>(Ki, Jc);
+            T Gk[3][3], F[3][3], Kr[3][3], gx[3][3], Kf[9];
 #pragma unroll
             for (int i = 0; i < 3; ++i)
 #pragma unroll
-              for (int d = 0; d < 3; ++d) {
-                T s = T(0);
+              for (int d = 0; d < 3; ++d) Gk[i][d] = K[k][3 * i + d];
+            const T lnJ = T(log(double(deformation(Gk, F, Kr)))), dw = aw[0];
+            grad_times<3>(g, Kr, gx);
+            T bg = T(0);
 #pragma unroll
-                for (int e = 0; e < 3; ++e) s = fma(Jc[i][e], aw[1 + voigt_index<3>(e, d)], s);
-                bg = fma(s, g[i][d], bg);
+            for (int a = 0; a < 3; ++a)
+#pragma unroll
+              for (int b = 0; b < 3; ++b) {
+                Kf[3 * a + b] = Kr[a][b];
+                T s = F[a][0] * F[b][0];
+#pragma unroll
+                for (int e = 1; e < 3; ++e) s = fma(F[a][e], F[b][e], s);
+                bg = fma(s - (a == b ? T(1) : T(0)), gx[a][b], bg);
               }
-            dmu -= bg - tr * dw;
+            const T tr = gx[0][0] + gx[1][1] + gx[2][2];
+            dmu -= bg * dw;
             dlam -= T(2) * lnJ * tr * dw;
 #pragma unroll
             for (int q = 1; q < 7; ++q) aw[q] *= -mu;
-            qp_compact<3, T>(g, K[k], -(mu - T(2) * lambda * lnJ) * dw, T(-2) * lambda * dw, aw + 1, Phi);
+            qp_compact<3, T>(g, Kf, -(mu - T(2) * lambda * lnJ) * dw, T(-2) * lambda * dw, aw + 1, Phi);
           } else if constexpr (SCAL) {
             const T dw = aw[0];
 #pragma unroll

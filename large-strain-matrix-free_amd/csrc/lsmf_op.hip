@@ -993,7 +993,7 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
         g[1 + v] = g[0] * (R[i][0] * R[j][0] + R[i][1] * R[j][1] + R[i][2] * R[j][2]);
       }
       for (int i = 0; i < 3; ++i)
-        for (int d = 0; d < 3; ++d) g[7 + 3 * i + d] = J[i][d];
+        for (int d = 0; d < 3; ++d) g[7 + 3 * i + d] = recompute_k(op) ? R[i][d] : J[i][d];
     }
   }
   // the tile tables in one piece: tiles by colour, private bits, shared nodes, slots
