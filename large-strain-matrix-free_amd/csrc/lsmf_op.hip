@@ -351,10 +351,12 @@ bool support_points_curved(const lsmf_mesh_desc *m, int dim, int p, int nqp) {
   return false;
 }
 
-// Every cell's Q1 vertex map is affine to the rounding of the coordinates:
-// the mixed differences of its vertices (xy, yz, zx, xyz) vanish, so J_ref
-// is one matrix per cell.  The bound is absolute, a few units in the last
-// place of the largest coordinate: what representing the vertices costs.
+// Every cell's Q1 vertex map is affine to the rounding of its coordinates: the
+// mixed differences of its vertices (xy, yz, zx, xyz) vanish, so J_ref is one
+// matrix per cell.  The bound is a few units in the last place of the cell's
+// own largest coordinate, what representing its vertices costs and what the
+// weighted sums of q1_jacobian lose in any case; the extent of the mesh, or a
+// node that no cell has, says nothing about a cell.
 bool cells_affine(const lsmf_mesh_desc *m, int dim, int p, int nqp) {
   const int N = p + 1, NV = 1 << dim;
   int corner[8];
@@ -363,22 +365,23 @@ bool cells_affine(const lsmf_mesh_desc *m, int dim, int p, int nqp) {
     for (int d = 0; d < dim; ++d, stride *= N) a += ((v >> d) & 1) * p * stride;
     corner[v] = a;
   }
-  double top = 0.0;
-  for (size_t i = 0; i < (size_t)m->n_nodes * dim; ++i) top = std::max(top, std::fabs(m->coords[i]));
-  const double tol = 8.0 * std::numeric_limits<double>::epsilon() * top;
   for (int c = 0; c < m->n_cells; ++c) {
     const int32_t *cn = m->cell_nodes + (size_t)c * nqp;
-    for (int i = 0; i < dim; ++i) {
-      double X[8];
-      for (int v = 0; v < NV; ++v) X[v] = m->coords[(size_t)cn[corner[v]] * dim + i];
+    double X[8][3], top = 0.0;
+    for (int v = 0; v < NV; ++v)
+      for (int i = 0; i < dim; ++i) {
+        X[v][i] = m->coords[(size_t)cn[corner[v]] * dim + i];
+        top = std::max(top, std::fabs(X[v][i]));
+      }
+    const double tol = 8.0 * std::numeric_limits<double>::epsilon() * top;
+    for (int i = 0; i < dim; ++i)
       // vertex v against the affine map of vertex 0 and its neighbours
       for (int v = 3; v < NV; ++v) {
-        double x = X[0];
+        double x = X[0][i];
         for (int d = 0; d < dim; ++d)
-          if ((v >> d) & 1) x += X[1 << d] - X[0];
-        if (!(std::fabs(x - X[v]) <= tol)) return false;
+          if ((v >> d) & 1) x += X[1 << d][i] - X[0][i];
+        if (!(std::fabs(x - X[v][i]) <= tol)) return false;
       }
-    }
   }
   return true;
 }
