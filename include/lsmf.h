@@ -176,7 +176,12 @@ lsmf_status lsmf_set_material_two(lsmf_op *op, const uint8_t *material_id, doubl
  * + mu/2 (tr b_bar - d), kappa = lambda + 2 mu / 3, whose operator caches
  * J^{-1/d} only (include/mf_nh_operator.h:467-487, 1001-1181).  Formulation 0
  * runs with scalar or tensor4 caching (LSMF_ERR_UNSUPPORTED otherwise) and
- * has no residual VJP.  Call before cache(). */
+ * has no residual VJP.  Call before cache().  tensor4 operators on meshes with
+ * the Q1 metric keep other values per point in formulation 0, whose memory the
+ * switch allocates (LSMF_ERR_OUT_OF_MEMORY: the formulation stays as it was).
+ * Their products recorded in a graph stay valid: a replay gives the product of
+ * the formulation and state that cache() cached last, and both formulations
+ * keep their memory from the first recorded product on. */
 lsmf_status lsmf_set_formulation(lsmf_op *op, int formulation);
 
 /* The displacement argument of NeoHookOperator::initialize

@@ -1097,9 +1097,18 @@ __device__ __forceinline__ void apply_epilogue(const Epilogue<T> &ep, T *dst, co
   store_node<DIM, T>(ep.x + at, x);
 }
 
+// which formulation's values a tensor4 operator has cached, and where: written
+// by cache(), read by recorded products
+struct FormState {
+  int formulation;
+  // global memory: loads through it stay global loads, as those through the kernel arguments are
+  const __attribute__((address_space(1))) void *cache;
+};
+
 template <typename Number> struct VmultParams {
   const uint32_t *__restrict__ idx;   // [cells][NQP] sorted cells
   const Number *__restrict__ cache;   // SoA caches
+  const FormState *__restrict__ form;  // recorded tensor4 products: run if this formulation is cached, from where it is
   size_t fs;                          // field stride = n_cells * NQP
   const Number *__restrict__ tab;     // S, D, St, Dt, qp, qw (Number)
   const Number *src;
@@ -1158,6 +1167,15 @@ template <typename Number> struct VmultParams {
   // read from the kernel arguments
   Number sf[2 * 15];
 };
+
+// The cached values of VAR, or nullptr where a recorded product's formulation is
+// not the cached one and the launch has nothing to do (uniform).
+template <int VAR, typename T> __device__ __forceinline__ const T *cached_values(const VmultParams<T> &P) {
+  if constexpr (VAR == V_TENSOR4 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U)
+    if (P.form)
+      return P.form->formulation == (VAR == V_TENSOR4 ? 0 : 1) ? (const T *)(P.form->cache) : nullptr;
+  return P.cache;
+}
 
 // 1D weight of Gauss point i from the symmetric half in the kernel arguments
 template <int N> __device__ __forceinline__ double weight_1d(const double *qw, int i) {
@@ -1328,6 +1346,8 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
   __shared__ T lds[CPW * SLOTW + TABN + (KIN ? CPW * NC * DIM : 0) + RED];
   __shared__ T tile_v[TILE ? TN * DIM : 1];         // tile nodes' source values
   __shared__ uint32_t tile_c[TILE && KIN ? TN : 1];  // tile nodes' codes (kinematics)
+  const T *__restrict__ cache = cached_values<VAR>(P);
+  if (P.form && !cache) return;
   T *tab = lds + CPW * SLOTW;
   T *Xall = tab + TABN;
   T *Rall = Xall + (KIN ? CPW * NC * DIM : 0);
@@ -1401,7 +1421,7 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
   const int r_s = on ? r : 0;
   __builtin_amdgcn_sched_barrier(0);
   T cch[NF > 0 ? NF : 1];
-  if constexpr ((PH & PH_QD) && NF > 0 && !RECOMP) load_cache<T, NF>(P.cache, cell_s * NQP + r_s, P.fs, cch);
+  if constexpr ((PH & PH_QD) && NF > 0 && !RECOMP) load_cache<T, NF>(cache, cell_s * NQP + r_s, P.fs, cch);
   double caff[VAR == V_COMPACT_AFFINE ? 1 + Voigt<DIM>::NV : 1];
   if constexpr ((PH & PH_QD) && VAR == V_COMPACT_AFFINE)
 #pragma unroll
@@ -1899,6 +1919,8 @@ __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_wave
   __shared__ double caff_all[CA];
   __shared__ T tile_u[RECOMP ? TN * 3 : 1];
   __shared__ T red[ADJ ? PS::CPW * 2 * NL : 1];  // columns' shares of dmu, dlambda
+  const T *__restrict__ cache = cached_values<VAR>(P);
+  if (P.form && !cache) return;
   const T *src = P.src + (size_t)blockIdx.y * P.vstride;  // an epilogue updates it in place
   T *dst = P.dst + (size_t)blockIdx.y * P.vstride;
   const int t = threadIdx.x, wave = t / 64, lane = t % 64;
@@ -1950,7 +1972,7 @@ __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_wave
   const size_t cq = (size_t)cell * NQP + (col ? j : 0);
   if constexpr (NF > 0)
 #pragma unroll
-    for (int k = 0; k < N; ++k) load_cache<T, NF>(P.cache, cq + k * NL, P.fs, cch[k]);
+    for (int k = 0; k < N; ++k) load_cache<T, NF>(cache, cq + k * NL, P.fs, cch[k]);
   T mu = T(0), lambda = T(0);
   if constexpr (GEO) {
     mu = P.mu[cell];

@@ -198,6 +198,7 @@ template <int DIM, int N> struct Launch {
   template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
   static int run_tiles(const lsmf_op *op, T *dst, const T *src, int identity, hipStream_t s,
                        const Epilogue<T> &ep = Epilogue<T>()) {
+    if (op->ws_capture) (void)both_formulations(op, s);  // its owner's graph
     VmultParams<T> P = tile_params<T, VAR>(op);
     P.ep = ep;
     P.src = src;
@@ -228,10 +229,44 @@ template <int DIM, int N> struct Launch {
     return run_colours<T, VAR, ADD, CONSTR, PH>(op, dst, src, s);
   }
 
+  // A product recorded in a caller's graph: the caller may switch the
+  // formulation, cache and replay, so where the formulations take other kernels
+  // both are recorded, and on a replay the one whose values are cached runs
+  // (*P.form).  The owner of a bound operator records its graphs anew instead.
+  static bool both_formulations(const lsmf_op *op, hipStream_t s) {
+    if (!op->d_form || !capturing(s)) return false;
+    op->recorded = true;
+    return !(op->ws_capture && s == op->ws_stream);
+  }
+  template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
+  static int launch_recorded(const lsmf_op *op, VmultParams<T> P, int n, unsigned nv, hipStream_t s) {
+    P.form = op->d_form;
+    P.u = static_cast<const T *>(VAR == V_COMPACT_U ? op->d_uc : op->d_u);
+    return launch_vmult<T, VAR, ADD, CONSTR, PH>(op, P, n, nv, s);
+  }
+  // one colour's cell kernel, or with both the kernels of both formulations
+  template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
+  static int launch_colour(const lsmf_op *op, const VmultParams<T> &P, int n, unsigned nv, bool both, hipStream_t s) {
+    if (!both) return launch_vmult<T, VAR, ADD, CONSTR, PH>(op, P, n, nv, s);
+    if constexpr (VAR == V_TENSOR4 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U) {
+      const int rc = launch_recorded<T, V_TENSOR4, ADD, CONSTR, PH>(op, P, n, nv, s);
+      if (rc) return rc;
+      switch (compact_variant(op)) {
+        case V_COMPACT: return launch_recorded<T, V_COMPACT, ADD, CONSTR, PH>(op, P, n, nv, s);
+        case V_COMPACT_AFFINE: return launch_recorded<T, V_COMPACT_AFFINE, ADD, CONSTR, PH>(op, P, n, nv, s);
+        default:
+          if constexpr (recompute_ok() && sizeof(T) == 8)
+            return launch_recorded<T, V_COMPACT_U, ADD, CONSTR, PH>(op, P, n, nv, s);
+      }
+    }
+    return LSMF_ERR_UNSUPPORTED;
+  }
+
   // one launch per colour; the tiled layout launches one workgroup per tile
   template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
   static int run_colours(const lsmf_op *op, T *dst, const T *src, hipStream_t s) {
     const int nc = n_colours(op);
+    const bool both = both_formulations(op, s);
     for (int k = 0; k < nc; ++k) {
       VmultParams<T> P = params<T, VAR>(op, k);
       P.src = src;
@@ -239,7 +274,7 @@ template <int DIM, int N> struct Launch {
       const int n = P.cell_end - P.cell_begin;
       if (n <= 0) continue;
       if (op->prof) op->prof->before(s);
-      const int rc = launch_vmult<T, VAR, ADD, CONSTR, PH>(op, P, n, 1, s);
+      const int rc = launch_colour<T, VAR, ADD, CONSTR, PH>(op, P, n, 1, both, s);
       if (op->prof) op->prof->after(s);
       if (rc) return rc;
     }
@@ -326,6 +361,7 @@ template <int DIM, int N> struct Launch {
     const int kMaxY = op->n_node_cons > 0 ? kHangBatch : 65535;
     const size_t n = op->n_dofs;
     const int nc = n_colours(op);
+    const bool both = both_formulations(op, s);
     for (int v0 = 0; v0 < nvec; v0 += kMaxY) {
       const unsigned nv = (unsigned)std::min(nvec - v0, kMaxY);
       T *d = dst + (size_t)v0 * n;
@@ -342,7 +378,7 @@ template <int DIM, int N> struct Launch {
         P.vstride = n;
         const int nb = P.cell_end - P.cell_begin;
         if (nb <= 0) continue;
-        const int rc = launch_vmult<T, VAR, false, true, FULL>(op, P, nb, nv, s);
+        const int rc = launch_colour<T, VAR, false, true, FULL>(op, P, nb, nv, both, s);
         if (rc) return rc;
       }
       if (op->n_node_cons > 0) hang_gather<T, true>(op, d, n, nv, s);

@@ -57,13 +57,14 @@ size_t elem_size(const lsmf_op *op) { return op->precision == LSMF_FP64 ? sizeof
 static bool recompute_k(const lsmf_op *op) {
   return op->affine && op->precision == LSMF_FP64 && op->dim == 3 && op->N == 3 && op->tile_kind == kTileWide;
 }
+int compact_variant(const lsmf_op *op) {
+  return recompute_k(op) ? V_COMPACT_U : op->affine ? V_COMPACT_AFFINE : V_COMPACT;
+}
 int cache_variant(const lsmf_op *op) {
-  const bool compact = op->formulation == 1 && !op->curved;
   switch (op->caching) {
     case LSMF_CACHING_TENSOR4:
     case LSMF_CACHING_TENSOR2:
-      if (compact && recompute_k(op)) return V_COMPACT_U;
-      if (compact) return op->affine ? V_COMPACT_AFFINE : V_COMPACT;
+      if (op->formulation == 1 && !op->curved) return compact_variant(op);
       return op->caching == LSMF_CACHING_TENSOR4 ? V_TENSOR4 : V_TENSOR2;
     case LSMF_CACHING_TENSOR4_NS: return V_TENSOR4_NS;
     case LSMF_CACHING_SCALAR: return V_SCALAR;
@@ -85,17 +86,16 @@ void bind_stream(lsmf_op *op, hipStream_t s) {
   op->ws_capture = true;
 }
 
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;  // the legacy stream while another one captures: launches fail too
+}
+
 TileBufferLock::TileBufferLock(const lsmf_op *op, hipStream_t s) {
   if (!op->d_tile_buf || s == hipStreamPerThread) return;  // that handle is a stream per thread
-  if (!op->ws_capture) {
-    // a captured product may be replayed on any stream
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
-      (void)hipGetLastError();
-      return;
-    }
-    if (st != hipStreamCaptureStatusNone) return;
-  }
+  if (!op->ws_capture && capturing(s)) return;  // a captured product may be replayed on any stream
   std::unique_lock<std::mutex> lock(op->ws_mu);
   if (!op->ws_bound) {
     op->ws_bound = true;
@@ -146,7 +146,7 @@ template <typename T> int dalloc(T **p, size_t n, const char *what) {
 }
 
 void free_op(lsmf_op *op) {
-  void *ptrs[] = {op->d_cgeo, op->d_uc,   op->d_idx,  op->d_coords,    op->d_tab,  op->d_tab64, op->d_mu64,     op->d_lambda64,
+  void *ptrs[] = {op->d_form, op->d_cache_other, op->d_cgeo, op->d_uc,   op->d_idx,  op->d_coords,    op->d_tab,  op->d_tab64, op->d_mu64,     op->d_lambda64,
                   op->d_mu,   op->d_lambda,    op->d_cache, op->d_caff, op->d_diag, op->d_inv_diag, op->d_cons,
                   op->d_bad,  op->d_perm,      op->d_tile_nodes, op->d_tile_info, op->d_tile_tables,
                   op->d_tile_buf, op->d_orphan, op->d_hang, op->d_hptr,
@@ -570,6 +570,10 @@ int build_tiles(lsmf_op *op, const lsmf_mesh_desc *mesh, const long long n[3], c
   return LSMF_OK;
 }
 
+__global__ void k_set_form(lsmf::FormState *f, int formulation, const void *cache) {
+  f->formulation = formulation;
+  f->cache = (const __attribute__((address_space(1))) void *)cache;
+}
 __global__ void k_convert_f64_f32(const double *__restrict__ a, float *__restrict__ b, size_t n) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) b[i] = float(a[i]);
@@ -601,6 +605,11 @@ lsmf_status cache_with_counter(lsmf_op *op, int *bad_dev, hipStream_t s, const c
   hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, s, bad_dev);
   int rc = launch_table(op->dim, op->N)->cache(op, bad_dev, s);
   if (rc) return fail(rc, std::string(what) + ": kernel launch failed");
+  if (op->d_form && op->form_cache != op->d_cache) {
+    hipLaunchKernelGGL(k_set_form, dim3(1), dim3(1), 0, s, op->d_form, op->formulation, (const void *)op->d_cache);
+    LSMF_HIP_TRY(hipGetLastError(), "cache: formulation");
+    op->form_cache = op->d_cache;
+  }
   int bad = 0;
   LSMF_HIP_TRY(hipMemcpyAsync(&bad, bad_dev, sizeof(int), hipMemcpyDeviceToHost, s), "cache: read det F count");
   LSMF_HIP_TRY(hipStreamSynchronize(s), "cache: synchronize");
@@ -1018,6 +1027,7 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
       (!cgeo.empty() && (rc = dalloc(&op->d_cgeo, cgeo.size(), "cell geometry"))) ||
       (cell_constants(op) &&
        (rc = dalloc(&op->d_caff, (size_t)nc * kAffineStride, "cell constants"))) ||
+      (op->caching == LSMF_CACHING_TENSOR4 && !op->curved && (rc = dalloc(&op->d_form, 1, "formulation"))) ||
       (rc = dalloc((char **)&op->d_diag, op->n_dofs * es, "diagonal")) ||
       (rc = dalloc((char **)&op->d_inv_diag, op->n_dofs * es, "inverse diagonal")) ||
       (rc = dalloc(&op->d_cons, cons.size(), "constrained list")) || (rc = dalloc(&op->d_bad, 1, "counter")) ||
@@ -1209,22 +1219,30 @@ lsmf_status lsmf_set_formulation(lsmf_op *op, int formulation) {
   op->cached = false;
   op->diag_ok = false;
   if (formulation == op->formulation) return LSMF_OK;
-  // the cached values of the other formulation take another amount of memory
+  // the cached values of the other formulation take another amount of memory;
+  // the ones that a recorded product may still read stay
   const int before = op->formulation;
   op->formulation = formulation;
   const int nf = n_cache_fields(op);
   if (nf != op->n_fields) {
-    void *p = nullptr;
     const size_t es = elem_size(op);
-    const int rc = dalloc((char **)&p, (size_t)nf * op->field_stride * es, "cache");
+    void *p = op->d_cache_other;
+    op->d_cache_other = nullptr;
+    const int rc = p ? 0 : dalloc((char **)&p, (size_t)nf * op->field_stride * es, "cache");
     if (rc) {
       op->formulation = before;
       return rc;
     }
-    (void)hipFree(op->d_cache);
+    if (op->recorded) {
+      op->d_cache_other = op->d_cache;
+    } else {
+      (void)hipFree(op->d_cache);
+      op->form_cache = nullptr;  // its address may come back
+    }
     op->d_cache = p;
     op->n_fields = nf;
   }
+  ++op->form_changes;
   op->bytes_cache = cache_bytes(op);
   return LSMF_OK;
 }

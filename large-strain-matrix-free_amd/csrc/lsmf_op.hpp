@@ -47,6 +47,10 @@ struct Profiler {
 // vectors per k_hang_gather pass of a batched product (the size of d_hbuf)
 constexpr int kHangBatch = 8;
 
+namespace lsmf {
+struct FormState;  // lsmf_kernels.hpp
+}
+
 struct lsmf_op {
   lsmf::Profiler *prof = nullptr;
   // shape
@@ -75,6 +79,15 @@ struct lsmf_op {
   double *d_u64 = nullptr;          // linearisation state copy
   void *d_u = nullptr;              // operator precision copy (scalar variant)
   void *d_cache = nullptr;
+  // tensor4 operators whose formulations keep different cached values: a product
+  // recorded in a caller's graph launches the kernels of both, and a replay runs
+  // the one that d_form names.  From the first recorded product on, each
+  // formulation keeps its own memory (d_cache_other: the one not in use)
+  lsmf::FormState *d_form = nullptr;
+  void *d_cache_other = nullptr;
+  const void *form_cache = nullptr;  // *d_form as last written (nullptr: never)
+  int form_changes = 0;
+  mutable bool recorded = false;
   double *d_caff = nullptr;         // affine compact form: [sorted cell][kAffineStride]
   void *d_uc = nullptr;             // u of the last cache() where the products recompute K from it
   double *d_cgeo = nullptr;         // affine cells' geometry (VmultParams::cgeo), where the residual uses it
@@ -185,5 +198,9 @@ struct LaunchTable {
 const LaunchTable *launch_table(int dim, int N);
 // the Variant whose cached values the operator's products read
 int cache_variant(const lsmf_op *op);
+// the same for tensor2 / tensor4 operators with the Q1 metric in formulation 1
+int compact_variant(const lsmf_op *op);
+// work submitted to s now goes into a graph
+bool capturing(hipStream_t s);
 
 }  // namespace lsmf

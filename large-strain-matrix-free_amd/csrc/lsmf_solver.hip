@@ -529,6 +529,10 @@ template <typename T> class GMG : public GMGBase {
     }
     // the V-cycle is a fixed sequence of launches between two setups:
     // capture it once and replay it (launch overhead of the small levels)
+    // (the finest operator is the caller's too: a graph of its other
+    // formulation's kernels is recorded anew once that formulation is cached)
+    const lsmf_op *fine = lv_.back().op->handle();
+    if (fine->cached && fine->form_changes != graph_forms_) drop_graph();
     if (!graph_exec_ || z != graph_z_ || r != graph_r_) {
       drop_graph();
       hipGraph_t g = nullptr;
@@ -539,6 +543,7 @@ template <typename T> class GMG : public GMGBase {
       (void)hipGraphDestroy(g);
       graph_z_ = z;
       graph_r_ = r;
+      graph_forms_ = fine->form_changes;
     }
     hip_check(hipGraphLaunch(graph_exec_, s_), "graph launch");
   }
@@ -754,6 +759,7 @@ template <typename T> class GMG : public GMGBase {
   hipGraphExec_t graph_exec_ = nullptr;
   double *graph_z_ = nullptr;
   const double *graph_r_ = nullptr;
+  int graph_forms_ = 0;  // the finest operator's form_changes
 };
 
 }  // namespace lsmf
