@@ -1123,7 +1123,6 @@ template <typename Number> struct VmultParams {
   int curved;       // support points off the Q1 maps: Eulerian Q_p metric (scalar variants)
   const uint32_t *__restrict__ tnodes;  // tiled layout: [tile][TN] node codes
   const int32_t *__restrict__ tinfo;    // tiled layout: [tile][2] first cell, extents
-  const int32_t *__restrict__ tlist;    // coloured launches: the tiles by colour; nullptr: tile = block
   // one launch over all tiles (nullptr: coloured launches): a tile writes the
   // nodes that only it touches (bit set in tpriv, TW words per tile) and
   // leaves its share of the others in tbuf [tile][TN][DIM] for k_tile_sum
@@ -1170,7 +1169,8 @@ template <typename Number> struct VmultParams {
 
 // The cached values of VAR, or nullptr where a recorded product's formulation is
 // not the cached one and the launch has nothing to do (uniform).
-template <int VAR, typename T> __device__ __forceinline__ const T *cached_values(const VmultParams<T> &P) {
+template <int VAR, bool ONE, typename T> __device__ __forceinline__ const T *cached_values(const VmultParams<T> &P) {
+  if constexpr (ONE) return P.cache;  // not recorded, or in a graph of the operator's owner
   if constexpr (VAR == V_TENSOR4 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U)
     if (P.form)
       return P.form->formulation == (VAR == V_TENSOR4 ? 0 : 1) ? (const T *)(P.form->cache) : nullptr;
@@ -1326,7 +1326,8 @@ template <int VAR, int TILE> constexpr int vmult_min_waves() {
   return TILE != kTileWide ? 1 : VAR == V_TENSOR2 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE ? 6 : 4;
 }
 
-template <int DIM, int N, typename T, int VAR, bool ADD, bool CONSTR, unsigned PH, int TILE>
+// ONE: all tiles in this launch (see k_tile_sum), else one colour's.
+template <int DIM, int N, typename T, int VAR, bool ADD, bool CONSTR, unsigned PH, int TILE, bool ONE>
 __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TILE>())) k_vmult(const VmultParams<T> P) {
   using CS = CellShape<DIM, N>;
   // threads and cells of this workgroup: a tile, or CS::CPW cells
@@ -1346,8 +1347,8 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
   __shared__ T lds[CPW * SLOTW + TABN + (KIN ? CPW * NC * DIM : 0) + RED];
   __shared__ T tile_v[TILE ? TN * DIM : 1];         // tile nodes' source values
   __shared__ uint32_t tile_c[TILE && KIN ? TN : 1];  // tile nodes' codes (kinematics)
-  const T *__restrict__ cache = cached_values<VAR>(P);
-  if (P.form && !cache) return;
+  const T *__restrict__ cache = cached_values<VAR, ONE>(P);
+  if (!ONE && P.form && !cache) return;
   T *tab = lds + CPW * SLOTW;
   T *Xall = tab + TABN;
   T *Rall = Xall + (KIN ? CPW * NC * DIM : 0);
@@ -1380,7 +1381,7 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
   size_t node = 0;
   // tiled layout: slot -> (sx, sy, sz) in the tile, lane t < TN -> tile node
   const int sx = slot % TS::TX, sy = (slot / TS::TX) % TS::TY, sz = slot / (TS::TX * TS::TY);
-  const int tile = TILE && P.tlist ? P.tlist[P.cell_begin + L] : P.cell_begin + L;
+  const int tile = P.cell_begin + L;
   uint32_t tcode = 0;
   bool tvalid = false, tshared = false;  // tshared: the node's sum is k_tile_sum's
   size_t tnode = 0;
@@ -1397,7 +1398,7 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
     tcode = P.tnodes[(size_t)tile * TN + (t < TN ? t : 0)];
     tvalid = t < TN && tcode != kNoNode;
     tnode = tvalid ? (tcode & kNodeMask) : 0;
-    if (P.tbuf) {
+    if constexpr (ONE) {
       const uint32_t *priv = P.tpriv + (size_t)tile * TS::TW;
       tshared = !((priv[t < TN ? t / 32 : 0] >> (t % 32)) & 1u);
     }
@@ -1406,7 +1407,7 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
     // read-modify-write: no other tile of this colour (of the launch: a
     // private node) touches the node, so they do not change before this tile
     // writes them
-    if (tvalid && (ADD ? !tshared : !P.tbuf && !(tcode & kFirstBit))) load_node<DIM, T>(dst + tnode * DIM, dv);
+    if (tvalid && (ADD ? !tshared : !ONE && !(tcode & kFirstBit))) load_node<DIM, T>(dst + tnode * DIM, dv);
   } else {
     cell = P.cell_begin + L * CPW + slot;
     active = on && (cell < P.cell_end);
@@ -1714,9 +1715,9 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
       T nv[DIM];
 #pragma unroll
       for (int c = 0; c < DIM; ++c) nv[c] = tile_v[t * DIM + c] + acc[c];  // destination: 0 on first touch
-      if (tshared) {
+      if (ONE && tshared) {
         store_node<DIM, T>(P.tbuf + ((size_t)tile * TN + t) * DIM, nv);
-      } else if (CONSTR && !ADD && P.ep.kind != EP_STORE) {
+      } else if (ONE && CONSTR && !ADD && P.ep.kind != EP_STORE) {
         apply_epilogue<DIM, T>(P.ep, dst, src, tnode, tcode, nv);
       } else if (!CONSTR || !((tcode >> kConsShift) & ((1u << DIM) - 1u))) {
         store_node<DIM, T>(dst + tnode * DIM, nv);
@@ -1725,7 +1726,7 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
         for (int c = 0; c < DIM; ++c) {
           if (!((tcode >> (kConsShift + c)) & 1u)) dst[tnode * DIM + c] = nv[c];
           // the identity on a constrained DoF (coloured launches: k_constrained_identity)
-          else if (P.tbuf && P.identity)
+          else if (ONE && P.identity)
             dst[tnode * DIM + c] = (ADD ? tile_v[t * DIM + c] : T(0)) + src[tnode * DIM + c];
         }
       }
@@ -1899,7 +1900,7 @@ template <int N, typename T, int VAR> constexpr int planes_min_waves() {
   return VAR == V_ADJOINT ? 2 : sizeof(T) == 8 ? 3 : 4;
 }
 
-template <int N, typename T, int VAR, bool ADD, bool CONSTR, int TILE>
+template <int N, typename T, int VAR, bool ADD, bool CONSTR, int TILE, bool ONE>
 __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_waves<N, T, VAR>())) k_vmult_planes(const VmultParams<T> P) {
   constexpr bool RES = VAR == V_RESIDUAL, ADJ = VAR == V_ADJOINT;  // affine cells, nothing cached
   constexpr bool SCAL = VAR == V_SCALAR, GEO = RES || ADJ || SCAL;  // affine cells, c cached; cgeo and material
@@ -1919,13 +1920,13 @@ __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_wave
   __shared__ double caff_all[CA];
   __shared__ T tile_u[RECOMP ? TN * 3 : 1];
   __shared__ T red[ADJ ? PS::CPW * 2 * NL : 1];  // columns' shares of dmu, dlambda
-  const T *__restrict__ cache = cached_values<VAR>(P);
-  if (P.form && !cache) return;
+  const T *__restrict__ cache = cached_values<VAR, ONE>(P);
+  if (!ONE && P.form && !cache) return;
   const T *src = P.src + (size_t)blockIdx.y * P.vstride;  // an epilogue updates it in place
   T *dst = P.dst + (size_t)blockIdx.y * P.vstride;
   const int t = threadIdx.x, wave = t / 64, lane = t % 64;
   const int L = xcd_remap(blockIdx.x, gridDim.x);
-  const int tile = P.tlist ? P.tlist[P.cell_begin + L] : P.cell_begin + L;
+  const int tile = P.cell_begin + L;
   const int first = P.tinfo[2 * (size_t)tile], ext = P.tinfo[2 * (size_t)tile + 1];
   const int ex = ext & 0xff, ey = (ext >> 8) & 0xff, ez = ext >> 16;
   // lane -> cell of the wave and its plane / column
@@ -1945,7 +1946,7 @@ __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_wave
     const int n = t + k * WG;
     tcode[k] = n < TN ? P.tnodes[(size_t)tile * TN + n] : kNoNode;
     tshared[k] = false;
-    if (P.tbuf) tshared[k] = !((P.tpriv[(size_t)tile * TS::TW + (n < TN ? n / 32 : 0)] >> (n % 32)) & 1u);
+    if constexpr (ONE) tshared[k] = !((P.tpriv[(size_t)tile * TS::TW + (n < TN ? n / 32 : 0)] >> (n % 32)) & 1u);
   }
 #pragma unroll
   for (int k = 0; k < ROUNDS; ++k) {
@@ -1955,7 +1956,7 @@ __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_wave
     if constexpr (!RES) load_node<3, T>(src + node * 3, sv[k]);
 #pragma unroll
     for (int c = 0; c < 3; ++c) dv[k][c] = T(0);
-    if (valid && (ADD ? !tshared[k] : !P.tbuf && !(tcode[k] & kFirstBit))) load_node<3, T>(dst + node * 3, dv[k]);
+    if (valid && (ADD ? !tshared[k] : !ONE && !(tcode[k] & kFirstBit))) load_node<3, T>(dst + node * 3, dv[k]);
   }
   __builtin_amdgcn_sched_barrier(0);
   // the cells' constants (consecutive cells) wait in LDS
@@ -2200,9 +2201,9 @@ __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_wave
 #pragma unroll
     for (int c = 0; c < 3; ++c) nv[c] = tile_v[n * 3 + c] + acc[c];
     const size_t node = tcode[k] & kNodeMask;
-    if (tshared[k]) {
+    if (ONE && tshared[k]) {
       store_node<3, T>(P.tbuf + ((size_t)tile * TN + n) * 3, nv);
-    } else if (CONSTR && !ADD && P.ep.kind != EP_STORE) {
+    } else if (ONE && CONSTR && !ADD && P.ep.kind != EP_STORE) {
       apply_epilogue<3, T>(P.ep, dst, src, node, tcode[k], nv);
     } else if (!CONSTR || !((tcode[k] >> kConsShift) & 7u)) {
       store_node<3, T>(dst + node * 3, nv);
@@ -2210,7 +2211,7 @@ __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_wave
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         if (!((tcode[k] >> (kConsShift + c)) & 1u)) dst[node * 3 + c] = nv[c];
-        else if (P.tbuf && P.identity)
+        else if (ONE && P.identity)
           dst[node * 3 + c] = (ADD ? tile_v[n * 3 + c] : T(0)) + src[node * 3 + c];
       }
     }
@@ -2794,7 +2795,7 @@ __global__ void __launch_bounds__(tile_threads<TILE>()) k_diagonal_tiles(const V
   const bool on = slot < CPW;
   const int sl = on ? slot : 0;
   const int L = xcd_remap(blockIdx.x, gridDim.x);
-  const int tile = P.tlist ? P.tlist[P.cell_begin + L] : P.cell_begin + L;
+  const int tile = P.cell_begin + L;
   const int first = P.tinfo[2 * (size_t)tile], ext = P.tinfo[2 * (size_t)tile + 1];
   const int ex = ext & 0xff, ey = (ext >> 8) & 0xff, ez = ext >> 16;
   const int sx = slot % TS::TX, sy = (slot / TS::TX) % TS::TY, sz = slot / (TS::TX * TS::TY);

@@ -29,20 +29,20 @@ template <int DIM, int N> struct Launch {
   // K from the displacement: that kernel only (cache_variant)
   static constexpr bool recompute_ok() { return DIM == 3 && N == 3; }
 
-  // one colour's fused cell kernel: n tiles (tiled layouts) or n cells, nv
-  // vectors (grid y)
-  template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
+  // one colour's fused cell kernel, or with ONE all tiles': n tiles (tiled
+  // layouts) or n cells, nv vectors (grid y)
+  template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH, bool ONE = false>
   static int launch_vmult(const lsmf_op *op, const VmultParams<T> &P, int n, unsigned nv, hipStream_t s) {
     if (op->tile_kind == kTileWide) {
       if constexpr (planes_ok<VAR>() && PH == (PH_SF | PH_QD)) {
-        hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide>), dim3(n, nv),
+        hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide, ONE>), dim3(n, nv),
                            dim3((PlaneShape<N, T, kTileWide>::WG)), 0, s, P);
         return 0;
       }
       if constexpr (kinematic_planes<T, VAR>()) {
         // residual and VJP in formulation 1 on affine cells
         if (op->d_cgeo && op->formulation == 1) {
-          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide>), dim3(n, nv),
+          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide, ONE>), dim3(n, nv),
                            dim3((PlaneShape<N, T, kTileWide>::WG)), 0,
                              s, P);
           return 0;
@@ -51,7 +51,7 @@ template <int DIM, int N> struct Launch {
       if constexpr (planes_ok<VAR>() && PH == (PH_SF | PH_QD))
         return LSMF_ERR_UNSUPPORTED;
       else if constexpr (wide_ok<VAR>())
-        hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide>), dim3(n, nv),
+        hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide, ONE>), dim3(n, nv),
                            dim3(tile_threads<kTileWide>()), 0, s, P);
       else
         return LSMF_ERR_UNSUPPORTED;
@@ -61,14 +61,16 @@ template <int DIM, int N> struct Launch {
       if constexpr (DIM == 3 && N == 3 && VAR == V_SCALAR && PH == (PH_SF | PH_QD)) {
         // formulation 1 on affine cells with the Q1 metric
         if (op->d_cgeo && op->formulation == 1) {
-          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, 1>), dim3(n, nv),
+          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, 1, ONE>), dim3(n, nv),
                              dim3((PlaneShape<N, T, 1>::WG)), 0, s, P);
           return 0;
         }
       }
-      hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, 1>), dim3(n, nv), dim3(kWG), 0, s, P);
+      hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, 1, ONE>), dim3(n, nv), dim3(kWG), 0, s, P);
+    } else if constexpr (ONE) {
+      return LSMF_ERR_UNSUPPORTED;
     } else {
-      hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, 0>), dim3(grid_for(n), nv), dim3(kWG), 0, s, P);
+      hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, 0, false>), dim3(grid_for(n), nv), dim3(kWG), 0, s, P);
     }
     return 0;
   }
@@ -104,9 +106,8 @@ template <int DIM, int N> struct Launch {
     P.cell_end = ptr[k + 1];
     P.formulation = op->formulation;
     P.curved = op->curved;
-    P.tnodes = op->d_tile_nodes;
-    P.tinfo = op->d_tile_info;
-    P.tlist = op->d_tile_list;
+    P.tnodes = op->d_ctile_nodes;
+    P.tinfo = op->d_ctile_info;
     P.hang = op->d_hang;
     P.hcons = op->d_hcons;
     P.hbuf = static_cast<T *>(op->d_hbuf);
@@ -161,7 +162,8 @@ template <int DIM, int N> struct Launch {
   // parameters of one launch over all tiles
   template <typename T, int VAR> static VmultParams<T> tile_params(const lsmf_op *op) {
     VmultParams<T> P = params<T, VAR>(op, 0);
-    P.tlist = nullptr;
+    P.tnodes = op->d_tile_nodes;
+    P.tinfo = op->d_tile_info;
     P.cell_begin = 0;
     P.cell_end = op->tile_ptr.back();
     P.tpriv = op->d_tile_priv;
@@ -205,7 +207,7 @@ template <int DIM, int N> struct Launch {
     P.dst = dst;
     P.identity = identity;
     if (op->prof) op->prof->before(s);
-    const int rc = launch_vmult<T, VAR, ADD, CONSTR, PH>(op, P, P.cell_end, 1, s);
+    const int rc = launch_vmult<T, VAR, ADD, CONSTR, PH, true>(op, P, P.cell_end, 1, s);
     if (rc) return rc;
     tile_sum<T, ADD, CONSTR>(op, dst, src, identity, s, ep);
     if (op->prof) op->prof->after(s);

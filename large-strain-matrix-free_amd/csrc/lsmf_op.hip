@@ -407,11 +407,12 @@ bool tile_dims(int dim, int N, int kind, TileDims &t) {
 }
 
 // Tiles of a logically structured mesh (cell grid cell_at, n cells per
-// direction) in grid order, coloured by the parity of their position so that
-// no two tiles of one colour share a node.  Fills perm (tile order, the cells
-// of a tile consecutive in slot order), the tile node table (node ids from
-// the cells' own node lists; first-touch bit: the node's first tile in colour
-// order), tile info, the tiles by colour, and for products in one launch the
+// direction), coloured by the parity of their position so that no two tiles of
+// one colour share a node, in the order of the grid where products run in one
+// launch and by colour elsewhere.  Fills perm (tile order, the cells of a tile
+// consecutive in slot order), the tile node table (node ids from the cells'
+// own node lists; first-touch bit: the node's first tile in colour order),
+// tile info, and for products in one launch the tables by colour, the
 // private-node bits and the shared nodes with their slots.  Returns
 // kNotTileable when cells that share a tile node position disagree about its
 // node (the cells layout then serves the mesh).
@@ -426,8 +427,8 @@ constexpr int kNotTileable = 1;
 // colours) 50 / 58 (2.1 M), 190 / 173 (8.4 M).
 constexpr size_t kOneLaunchDofs = 4000000;
 struct TileTables {
-  std::vector<uint32_t> nodes, priv, sum_node, sum_slot;
-  std::vector<int32_t> info, list;
+  std::vector<uint32_t> nodes, cnodes, priv, sum_node, sum_slot;
+  std::vector<int32_t> info, cinfo;
 };
 int build_tiles(lsmf_op *op, const lsmf_mesh_desc *mesh, const long long n[3], const std::vector<int32_t> &cell_at,
                 TileTables &tt) {
@@ -441,13 +442,14 @@ int build_tiles(lsmf_op *op, const lsmf_mesh_desc *mesh, const long long n[3], c
   std::vector<uint8_t> tcol(n_tiles);
   for (long long b = 0; b < n_tiles; ++b)
     tcol[b] = (uint8_t)((b % TXn & 1) | ((b / TXn % TYn & 1) << 1) | ((b / (TXn * TYn) & 1) << 2));
-  tt.list.clear();
-  tt.list.reserve(n_tiles);
+  const bool one = op->n_dofs <= kOneLaunchDofs;
+  std::vector<int32_t> by_colour;
+  by_colour.reserve(n_tiles);
   op->tile_ptr.assign(n_col + 1, 0);
   for (int col = 0; col < n_col; ++col) {
     for (long long b = 0; b < n_tiles; ++b)
-      if (tcol[b] == col) tt.list.push_back((int32_t)b);
-    op->tile_ptr[col + 1] = (int)tt.list.size();
+      if (tcol[b] == col) by_colour.push_back((int32_t)b);
+    op->tile_ptr[col + 1] = (int)by_colour.size();
   }
   op->perm.assign(op->n_cells, 0);
   op->inv_perm.assign(op->n_cells, 0);
@@ -470,13 +472,14 @@ int build_tiles(lsmf_op *op, const lsmf_mesh_desc *mesh, const long long n[3], c
   }
   std::vector<const int32_t *> cell_nodes(td.tx * td.ty * td.tz);
   int pos = 0;
-  for (long long b = 0; b < n_tiles; ++b) {
+  for (long long i = 0; i < n_tiles; ++i) {
+    const long long b = one ? i : by_colour[i];
     const long long bx = b % TXn, by = (b / TXn) % TYn, bz = b / (TXn * TYn);
     const int ex = (int)std::min<long long>(td.tx, n[0] - bx * td.tx);
     const int ey = (int)std::min<long long>(td.ty, n[1] - by * td.ty);
     const int ez = (int)std::min<long long>(td.tz, n[2] - bz * td.tz);
-    tt.info[(size_t)b * 2] = pos;
-    tt.info[(size_t)b * 2 + 1] = ex | (ey << 8) | (ez << 16);
+    tt.info[(size_t)i * 2] = pos;
+    tt.info[(size_t)i * 2 + 1] = ex | (ey << 8) | (ez << 16);
     auto tile_cell = [&](int sx, int sy, int sz) {
       return cell_at[(bx * td.tx + sx) + n[0] * ((by * td.ty + sy) + n[1] * (bz * td.tz + sz))];
     };
@@ -505,7 +508,7 @@ int build_tiles(lsmf_op *op, const lsmf_mesh_desc *mesh, const long long n[3], c
       if (node < 0) continue;
       if ((cols[node] >> tcol[b]) & 1u) return kNotTileable;  // two tiles of one colour share a node
       cols[node] |= (uint8_t)(1u << tcol[b]);
-      tt.nodes[(size_t)b * td.tn + l] = (uint32_t)node;
+      tt.nodes[(size_t)i * td.tn + l] = (uint32_t)node;
     }
   }
   if (pos != op->n_cells) return fail(LSMF_ERR_INVALID_ARGUMENT, "tiles: cell count mismatch");
@@ -516,14 +519,14 @@ int build_tiles(lsmf_op *op, const lsmf_mesh_desc *mesh, const long long n[3], c
         if (mesh->constrained[node * dim + comp]) bits |= 1u << (kConsShift + comp);
     return bits;
   };
-  if (op->n_dofs > kOneLaunchDofs) {
-    for (long long b = 0; b < n_tiles; ++b)
+  if (!one) {
+    for (long long i = 0; i < n_tiles; ++i)
       for (int l = 0; l < td.tn; ++l) {
-        uint32_t &code = tt.nodes[(size_t)b * td.tn + l];
+        uint32_t &code = tt.nodes[(size_t)i * td.tn + l];
         if (code == kNoNode) continue;
         const uint32_t node = code;
         code |= cons_bits(node);
-        if (!(cols[node] & ((1u << tcol[b]) - 1u))) code |= kFirstBit;
+        if (!(cols[node] & ((1u << tcol[by_colour[i]]) - 1u))) code |= kFirstBit;
       }
     return LSMF_OK;
   }
@@ -567,6 +570,12 @@ int build_tiles(lsmf_op *op, const lsmf_mesh_desc *mesh, const long long n[3], c
       }
       if (!below) code |= kFirstBit;
     }
+  tt.cnodes.reserve(tt.nodes.size());
+  tt.cinfo.reserve(tt.info.size());
+  for (const int32_t b : by_colour) {
+    tt.cnodes.insert(tt.cnodes.end(), tt.nodes.begin() + (size_t)b * td.tn, tt.nodes.begin() + (size_t)(b + 1) * td.tn);
+    tt.cinfo.insert(tt.cinfo.end(), {tt.info[(size_t)b * 2], tt.info[(size_t)b * 2 + 1]});
+  }
   return LSMF_OK;
 }
 
@@ -1008,9 +1017,10 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
         for (int d = 0; d < 3; ++d) g[7 + 3 * i + d] = recompute_k(op) ? R[i][d] : J[i][d];
     }
   }
-  // the tile tables in one piece: tiles by colour, private bits, shared nodes, slots
-  std::vector<uint32_t> tile_tables(tt.list.begin(), tt.list.end());
-  for (const auto *v : {&tt.priv, &tt.sum_node, &tt.sum_slot}) tile_tables.insert(tile_tables.end(), v->begin(), v->end());
+  // the tables of products in one launch in one piece: info and nodes by colour,
+  // private bits, shared nodes, slots
+  std::vector<uint32_t> tile_tables(tt.cinfo.begin(), tt.cinfo.end());
+  for (const auto *v : {&tt.cnodes, &tt.priv, &tt.sum_node, &tt.sum_slot}) tile_tables.insert(tile_tables.end(), v->begin(), v->end());
 
   const size_t es = elem_size(op);
   int rc = 0;
@@ -1104,10 +1114,13 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
   if (e == hipSuccess && !cgeo.empty())
     e = hipMemcpy(op->d_cgeo, cgeo.data(), cgeo.size() * sizeof(double), hipMemcpyHostToDevice);
   op->bytes_idx += cgeo.size() * sizeof(double);
+  op->d_ctile_nodes = op->d_tile_nodes;
+  op->d_ctile_info = op->d_tile_info;
   if (e == hipSuccess && !tile_tables.empty()) {
     e = hipMemcpy(op->d_tile_tables, tile_tables.data(), tile_tables.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
-    op->d_tile_list = reinterpret_cast<const int32_t *>(op->d_tile_tables);
-    op->d_tile_priv = op->d_tile_tables + tt.list.size();
+    op->d_ctile_info = reinterpret_cast<const int32_t *>(op->d_tile_tables);
+    op->d_ctile_nodes = op->d_tile_tables + tt.cinfo.size();
+    op->d_tile_priv = op->d_ctile_nodes + tt.cnodes.size();
     op->d_sum_node = op->d_tile_priv + tt.priv.size();
     op->d_sum_slot = op->d_sum_node + tt.sum_node.size();
   }
