@@ -861,25 +861,22 @@ __device__ __forceinline__ void qp_tensor4_ns(const T (&G)[DIM][DIM], const T *c
 template <int DIM, typename T>
 __device__ __forceinline__ void qp_compact(const T (&G)[DIM][DIM], const T *K, T cdw, T ldw, const T *A,
                                            T (&Phi)[DIM][DIM]) {
-  T X[DIM][DIM];  // K G
+  // row d of K G on its own: all of it at once costs the FP64 Q4 kernel spills
+  auto row = [&](int d, int e) {
+    T s = K[d * DIM] * G[0][e];
 #pragma unroll
-  for (int d = 0; d < DIM; ++d)
+    for (int j = 1; j < DIM; ++j) s = fma(K[d * DIM + j], G[j][e], s);
+    return s;
+  };
+  T tr = row(0, 0);
 #pragma unroll
-    for (int e = 0; e < DIM; ++e) {
-      T s = K[d * DIM] * G[0][e];
-#pragma unroll
-      for (int j = 1; j < DIM; ++j) s = fma(K[d * DIM + j], G[j][e], s);
-      X[d][e] = s;
-    }
-  T tr = X[0][0];
-#pragma unroll
-  for (int d = 1; d < DIM; ++d) tr += X[d][d];
+  for (int d = 1; d < DIM; ++d) tr += row(d, d);
   const T lt = ldw * tr;
 #pragma unroll
   for (int d = 0; d < DIM; ++d) {
-    T Y[DIM];  // row d of c dw X + lt I
+    T Y[DIM];  // row d of c dw K G + lt I
 #pragma unroll
-    for (int e = 0; e < DIM; ++e) Y[e] = e == d ? fma(cdw, X[d][e], lt) : cdw * X[d][e];
+    for (int e = 0; e < DIM; ++e) Y[e] = e == d ? fma(cdw, row(d, e), lt) : cdw * row(d, e);
 #pragma unroll
     for (int c = 0; c < DIM; ++c) {
       T s = Y[0] * K[c];
@@ -1320,8 +1317,10 @@ __device__ __forceinline__ void kinematics_collocation(const VmultParams<T> &P, 
 // ------------------------------------------------------------------------
 // Minimum waves per SIMD of the fused cell kernel (HIP's second
 // __launch_bounds__ argument): wide tiles at least 4 (two 512-thread
-// workgroups per CU, at most 128 VGPRs); the wide tensor2 kernel 6 (three
-// workgroups, at most 80 VGPRs, which its FP64 form needs no more than).
+// workgroups per CU, at most 128 VGPRs); the wide tensor2 and compact kernels 6
+// (three workgroups, at most 80 VGPRs).  The FP64 Q4 kernels just fit: a spilled
+// cached value is waited for before the sums start, which cost 64^3 tensor2
+// 1372 us against 1169 without spills, 32^3 245 against 201.
 template <int VAR, int TILE> constexpr int vmult_min_waves() {
   return TILE != kTileWide ? 1 : VAR == V_TENSOR2 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE ? 6 : 4;
 }
@@ -1346,7 +1345,7 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
   constexpr int SLOTW = (DIM == 3 ? 1 : 2) * NB * NQP;
   __shared__ T lds[CPW * SLOTW + TABN + (KIN ? CPW * NC * DIM : 0) + RED];
   __shared__ T tile_v[TILE ? TN * DIM : 1];         // tile nodes' source values
-  __shared__ uint32_t tile_c[TILE && KIN ? TN : 1];  // tile nodes' codes (kinematics)
+  __shared__ uint32_t tile_c[TILE ? TN : 1];  // tile nodes' codes
   const T *__restrict__ cache = cached_values<VAR, ONE>(P);
   if (!ONE && P.form && !cache) return;
   T *tab = lds + CPW * SLOTW;
@@ -1389,9 +1388,11 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
   T dv[DIM];
 #pragma unroll
   for (int c = 0; c < DIM; ++c) dv[c] = T(0);
+  int first = 0, ex = 0, ey = 0, ez = 0;  // the tile's cells
   if constexpr (TILE) {
-    const int first = P.tinfo[2 * (size_t)tile], ext = P.tinfo[2 * (size_t)tile + 1];
-    const int ex = ext & 0xff, ey = (ext >> 8) & 0xff, ez = ext >> 16;
+    const int ext = P.tinfo[2 * (size_t)tile + 1];
+    first = P.tinfo[2 * (size_t)tile];
+    ex = ext & 0xff, ey = (ext >> 8) & 0xff, ez = ext >> 16;
     active = on && sx < ex && sy < ey && sz < ez;
     cell = first + sx + ex * (sy + ey * sz);
     cell_s = active ? (size_t)cell : (size_t)first;
@@ -1420,20 +1421,37 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
     }
   }
   const int r_s = on ? r : 0;
+  // The cells' constants.  The FP64 wide kernels, at the limit of their registers,
+  // keep them in LDS: seven values per lane through the sums were eight spills.
+  // The others have the registers, and LDS reads they need not make (32^3 Q4 FP32
+  // 118 us, 125 from LDS).
+  constexpr int NCA = 1 + Voigt<DIM>::NV;
+  constexpr bool AFF = (PH & PH_QD) && VAR == V_COMPACT_AFFINE, LAFF = AFF && TILE == kTileWide && sizeof(T) == 8;
+  __shared__ double caff_all[LAFF ? CPW * NCA : 1];
+  static_assert(!LAFF || CPW * NCA <= WG, "one lane per cell constant");
+  double caff1 = 0.0;
+  if constexpr (LAFF) {
+    const int cs = t / NCA;  // cell of the tile
+    const int cx = cs % TS::TX, cy = (cs / TS::TX) % TS::TY, cz = cs / (TS::TX * TS::TY);
+    const bool has = t < CPW * NCA && cx < ex && cy < ey && cz < ez;
+    caff1 = P.caff[(size_t)(has ? first + cx + ex * (cy + ey * cz) : first) * kAffineStride + t % NCA];
+  }
   __builtin_amdgcn_sched_barrier(0);
   T cch[NF > 0 ? NF : 1];
   if constexpr ((PH & PH_QD) && NF > 0 && !RECOMP) load_cache<T, NF>(cache, cell_s * NQP + r_s, P.fs, cch);
-  double caff[VAR == V_COMPACT_AFFINE ? 1 + Voigt<DIM>::NV : 1];
-  if constexpr ((PH & PH_QD) && VAR == V_COMPACT_AFFINE)
+  double caff[AFF && !LAFF ? NCA : 1];
+  if constexpr (AFF && !LAFF)
 #pragma unroll
-    for (int k = 0; k < 1 + Voigt<DIM>::NV; ++k) caff[k] = P.caff[cell_s * kAffineStride + k];
+    for (int k = 0; k < NCA; ++k) caff[k] = P.caff[cell_s * kAffineStride + k];
   __builtin_amdgcn_sched_barrier(0);
 
   // tile-local index of this lane's node (tiled layout)
   const int ln = on ? (sx * (N - 1) + i0) + TS::NX * ((sy * (N - 1) + i1) + TS::NY * (sz * (N - 1) + i2)) : 0;
+  if constexpr (LAFF)
+    if (t < CPW * NCA) caff_all[t] = caff1;
   if constexpr (TILE) {
     if (t < TN) {
-      if constexpr (KIN) tile_c[t] = tcode;
+      tile_c[t] = tcode;
       if constexpr (VAR == V_RESIDUAL) {
         // no source values: the tile holds the destination values throughout
 #pragma unroll
@@ -1531,9 +1549,10 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
     } else if constexpr (VAR == V_COMPACT_AFFINE) {
       double w = weight_1d<N>(P.qw, i0) * weight_1d<N>(P.qw, i1);
       if constexpr (DIM == 3) w *= weight_1d<N>(P.qw, i2);
-      T aw[1 + Voigt<DIM>::NV];
+      const double *ca = LAFF ? caff_all + (on ? slot : 0) * NCA : caff;
+      T aw[NCA];
 #pragma unroll
-      for (int k = 0; k < 1 + Voigt<DIM>::NV; ++k) aw[k] = T(caff[k] * w);
+      for (int k = 0; k < NCA; ++k) aw[k] = T(ca[k] * w);
       qp_compact<DIM, T>(G, cch, cch[DIM * DIM], aw[0], aw + 1, Phi);
     } else if constexpr (VAR == V_TENSOR4) {
       qp_tensor4<DIM, T>(G, cch, Phi);
@@ -1676,6 +1695,11 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
   }
 
   if constexpr (TILE) {
+    // the node's code from LDS: in a register through the sums it was one too
+    // many for the FP64 Q4 kernels
+    tcode = t < TN ? tile_c[t] : kNoNode;
+    tvalid = tcode != kNoNode;
+    tnode = tvalid ? (tcode & kNodeMask) : 0;
     // sum the cells' results per tile node in LDS (fixed order), then one
     // write per node (distribute_local_to_global, :769-780).  In 3D the
     // results are read where the integration (or, without it, the gather)
