@@ -861,22 +861,25 @@ __device__ __forceinline__ void qp_tensor4_ns(const T (&G)[DIM][DIM], const T *c
 template <int DIM, typename T>
 __device__ __forceinline__ void qp_compact(const T (&G)[DIM][DIM], const T *K, T cdw, T ldw, const T *A,
                                            T (&Phi)[DIM][DIM]) {
-  // row d of K G on its own: all of it at once costs the FP64 Q4 kernel spills
-  auto row = [&](int d, int e) {
-    T s = K[d * DIM] * G[0][e];
+  T X[DIM][DIM];  // K G
 #pragma unroll
-    for (int j = 1; j < DIM; ++j) s = fma(K[d * DIM + j], G[j][e], s);
-    return s;
-  };
-  T tr = row(0, 0);
+  for (int d = 0; d < DIM; ++d)
 #pragma unroll
-  for (int d = 1; d < DIM; ++d) tr += row(d, d);
+    for (int e = 0; e < DIM; ++e) {
+      T s = K[d * DIM] * G[0][e];
+#pragma unroll
+      for (int j = 1; j < DIM; ++j) s = fma(K[d * DIM + j], G[j][e], s);
+      X[d][e] = s;
+    }
+  T tr = X[0][0];
+#pragma unroll
+  for (int d = 1; d < DIM; ++d) tr += X[d][d];
   const T lt = ldw * tr;
 #pragma unroll
   for (int d = 0; d < DIM; ++d) {
-    T Y[DIM];  // row d of c dw K G + lt I
+    T Y[DIM];  // row d of c dw X + lt I
 #pragma unroll
-    for (int e = 0; e < DIM; ++e) Y[e] = e == d ? fma(cdw, row(d, e), lt) : cdw * row(d, e);
+    for (int e = 0; e < DIM; ++e) Y[e] = e == d ? fma(cdw, X[d][e], lt) : cdw * X[d][e];
 #pragma unroll
     for (int c = 0; c < DIM; ++c) {
       T s = Y[0] * K[c];
@@ -1928,7 +1931,7 @@ template <int N, typename T, int VAR, bool ADD, bool CONSTR, int TILE, bool ONE>
 __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_waves<N, T, VAR>())) k_vmult_planes(const VmultParams<T> P) {
   constexpr bool RES = VAR == V_RESIDUAL, ADJ = VAR == V_ADJOINT;  // affine cells, nothing cached
   constexpr bool SCAL = VAR == V_SCALAR, GEO = RES || ADJ || SCAL;  // affine cells, c cached; cgeo and material
-  static_assert(VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U || GEO);
+  static_assert(VAR == V_COMPACT_U || GEO || (sizeof(T) == 4 && (VAR == V_COMPACT || VAR == V_COMPACT_AFFINE)));
   constexpr bool AFFINE = VAR != V_COMPACT, RECOMP = VAR == V_COMPACT_U || GEO;
   using PS = PlaneShape<N, T, TILE>;
   using TS = TileShape<3, N, tile_threads<TILE>()>;

@@ -19,9 +19,14 @@ template <int DIM, int N> struct Launch {
             VAR == V_COMPACT_U || VAR == V_RESIDUAL || VAR == V_ADJOINT);
   }
 
-  // products of the compact forms on wide tiles
-  template <int VAR> static constexpr bool planes_ok() {
-    return DIM == 3 && N == 3 && (VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U);
+  // products of the compact forms on wide tiles (lsmf_op::planes): K from the
+  // displacement, or cached in FP32.  With 17 cached FP64 values per point
+  // (bilinear cells) the line kernel is the faster one, the values of a plane
+  // lane's column do not fit its registers: 64^3 311 us against 410, 32^3 41.1
+  // against 48, on another stream 69.7 against 79.
+  template <typename T, int VAR> static constexpr bool planes_ok() {
+    return DIM == 3 && N == 3 &&
+           (VAR == V_COMPACT_U || (sizeof(T) == 4 && (VAR == V_COMPACT || VAR == V_COMPACT_AFFINE)));
   }
   template <typename T, int VAR> static constexpr bool kinematic_planes() {
     return DIM == 3 && N == 3 && sizeof(T) == 8 && (VAR == V_RESIDUAL || VAR == V_ADJOINT);
@@ -34,10 +39,12 @@ template <int DIM, int N> struct Launch {
   template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH, bool ONE = false>
   static int launch_vmult(const lsmf_op *op, const VmultParams<T> &P, int n, unsigned nv, hipStream_t s) {
     if (op->tile_kind == kTileWide) {
-      if constexpr (planes_ok<VAR>() && PH == (PH_SF | PH_QD)) {
-        hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide, ONE>), dim3(n, nv),
-                           dim3((PlaneShape<N, T, kTileWide>::WG)), 0, s, P);
-        return 0;
+      if constexpr (planes_ok<T, VAR>() && PH == (PH_SF | PH_QD)) {
+        if (op->planes) {
+          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide, ONE>), dim3(n, nv),
+                             dim3((PlaneShape<N, T, kTileWide>::WG)), 0, s, P);
+          return 0;
+        }
       }
       if constexpr (kinematic_planes<T, VAR>()) {
         // residual and VJP in formulation 1 on affine cells
@@ -48,7 +55,7 @@ template <int DIM, int N> struct Launch {
           return 0;
         }
       }
-      if constexpr (planes_ok<VAR>() && PH == (PH_SF | PH_QD))
+      if constexpr (VAR == V_COMPACT_U && PH == (PH_SF | PH_QD))
         return LSMF_ERR_UNSUPPORTED;
       else if constexpr (wide_ok<VAR>())
         hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide, ONE>), dim3(n, nv),

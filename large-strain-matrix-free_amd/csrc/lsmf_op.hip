@@ -55,7 +55,7 @@ size_t elem_size(const lsmf_op *op) { return op->precision == LSMF_FP64 ? sizeof
 // slots were padded.  FP32 operators keep K, which is rounded once from FP64;
 // from an FP32 displacement it would lose the digits of |u| / h.
 static bool recompute_k(const lsmf_op *op) {
-  return op->affine && op->precision == LSMF_FP64 && op->dim == 3 && op->N == 3 && op->tile_kind == kTileWide;
+  return op->affine && op->precision == LSMF_FP64 && op->planes;
 }
 int compact_variant(const lsmf_op *op) {
   return recompute_k(op) ? V_COMPACT_U : op->affine ? V_COMPACT_AFFINE : V_COMPACT;
@@ -774,6 +774,7 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
       return rc;
     }
   }
+  op->planes = op->tiled && dim == 3 && N == 3 && op->tile_kind == kTileWide;
   op->n_fields = n_cache_fields(op);
   // --- colouring (given and checked, or greedy first fit): no node is written
   // by two cells of one colour; used[n] = colours of the cells that write n.
@@ -996,8 +997,9 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
   // affine cells' geometry: residual and VJP on wide Q2 tiles, scalar products
   // on the others
   std::vector<double> cgeo;
-  if (recompute_k(op) || (op->caching == LSMF_CACHING_SCALAR && op->tile_kind == 1 && dim == 3 && N == 3 &&
-                          op->affine && !op->curved)) {
+  const bool kin_geo = op->affine && op->precision == LSMF_FP64 && dim == 3 && N == 3 && op->tile_kind == kTileWide;
+  if (kin_geo || (op->caching == LSMF_CACHING_SCALAR && op->tile_kind == 1 && dim == 3 && N == 3 && op->affine &&
+                  !op->curved)) {
     cgeo.resize((size_t)nc * kAffineStride);
     int corner[8];
     for (int v = 0; v < 8; ++v) corner[v] = p * ((v & 1) + N * ((v >> 1 & 1) + N * (v >> 2 & 1)));
@@ -1014,7 +1016,7 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
         g[1 + v] = g[0] * (R[i][0] * R[j][0] + R[i][1] * R[j][1] + R[i][2] * R[j][2]);
       }
       for (int i = 0; i < 3; ++i)
-        for (int d = 0; d < 3; ++d) g[7 + 3 * i + d] = recompute_k(op) ? R[i][d] : J[i][d];
+        for (int d = 0; d < 3; ++d) g[7 + 3 * i + d] = kin_geo ? R[i][d] : J[i][d];
     }
   }
   // the tables of products in one launch in one piece: info and nodes by colour,
