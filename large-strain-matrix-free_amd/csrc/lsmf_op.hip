@@ -50,10 +50,11 @@ size_t elem_size(const lsmf_op *op) { return op->precision == LSMF_FP64 ? sizeof
 // Q_p metric: K F is no longer J_ref^-1) and formulation 0 keep the stored
 // tensors.
 // K from the displacement instead of from memory (one cached value per point
-// instead of ten): FP64 operators on wide Q2 tiles of affine cells, 128^3
-// 1786 -> 1705 us, 64^3 287 -> 281, 32^3 43.5 -> 44.7 before that kernel's
-// slots were padded.  FP32 operators keep K, which is rounded once from FP64;
-// from an FP32 displacement it would lose the digits of |u| / h.
+// instead of ten), by the plane kernel: FP64 operators on wide Q2 tiles of affine
+// cells, with lsmf_op::planes.  Against the line kernel with K cached, us: 128^3
+// 1558 / 1820, 64^3 249 / 282, 32^3 39.7 / 41.1.  FP32 operators keep K, which is
+// rounded once from FP64; from an FP32 displacement it would lose the digits of
+// |u| / h.
 static bool recompute_k(const lsmf_op *op) {
   return op->affine && op->precision == LSMF_FP64 && op->planes;
 }
@@ -426,6 +427,15 @@ constexpr int kNotTileable = 1;
 // (24^3, 2.7 M), 117 / 118 (32^3, 6.4 M), 217 / 206 (40^3); 2D Q2 FP64 (4
 // colours) 50 / 58 (2.1 M), 190 / 173 (8.4 M).
 constexpr size_t kOneLaunchDofs = 4000000;
+// FP64 products on affine Q2 cells of kFewTiles + 1 to kLineTiles wide tiles keep
+// K and run the line kernel: there a launch lasts as long as one tile, and the
+// plane kernel's tile (two evaluations, one wave per six cells) takes longer.
+// Line / planes, us: 16^3 (256 tiles) 13.4 / 14.0 in one launch, 62 / 69 in
+// coloured ones (64 with the stored tensors), 8^3 (32) 12.0 / 12.4 and 32.7 / 34.9;
+// 20^3 (600) 20.8 / 19.8 and 62 / 68, 32^3 41.1 / 39.7.  Below, batches of unit
+// vectors (coarse matrices) count: 4^3 (8 tiles), 2187 vectors, 253 / 211.
+// FP32: the plane kernel at every size (16^3 11.8 / 11.7, 32^3 28 / 24.7).
+constexpr int kFewTiles = 16, kLineTiles = 512;
 struct TileTables {
   std::vector<uint32_t> nodes, cnodes, priv, sum_node, sum_slot;
   std::vector<int32_t> info, cinfo;
@@ -774,7 +784,10 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
       return rc;
     }
   }
-  op->planes = op->tiled && dim == 3 && N == 3 && op->tile_kind == kTileWide;
+  if (op->tiled && dim == 3 && N == 3 && op->tile_kind == kTileWide) {
+    const int n_tiles = op->tile_ptr.back();
+    op->planes = op->precision == LSMF_FP32 || n_tiles <= kFewTiles || n_tiles > kLineTiles;
+  }
   op->n_fields = n_cache_fields(op);
   // --- colouring (given and checked, or greedy first fit): no node is written
   // by two cells of one colour; used[n] = colours of the cells that write n.
