@@ -1108,7 +1108,7 @@ struct FormState {
 template <typename Number> struct VmultParams {
   const uint32_t *__restrict__ idx;   // [cells][NQP] sorted cells
   const Number *__restrict__ cache;   // SoA caches
-  const FormState *__restrict__ form;  // recorded tensor4 products: run if this formulation is cached, from where it is
+  const FormState *__restrict__ form;  // recorded tensor4 products: which formulation is cached, and where
   size_t fs;                          // field stride = n_cells * NQP
   const Number *__restrict__ tab;     // S, D, St, Dt, qp, qw (Number)
   const Number *src;
@@ -1167,15 +1167,10 @@ template <typename Number> struct VmultParams {
   Number sf[2 * 15];
 };
 
-// The cached values of VAR, or nullptr where a recorded product's formulation is
-// not the cached one and the launch has nothing to do (uniform).
-template <int VAR, bool ONE, typename T> __device__ __forceinline__ const T *cached_values(const VmultParams<T> &P) {
-  if constexpr (ONE) return P.cache;  // not recorded, or in a graph of the operator's owner
-  if constexpr (VAR == V_TENSOR4 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U)
-    if (P.form)
-      return P.form->formulation == (VAR == V_TENSOR4 ? 0 : 1) ? (const T *)(P.form->cache) : nullptr;
-  return P.cache;
-}
+// Launches of the cell kernels: one colour's tiles or cells, all tiles (see
+// k_tile_sum), or one colour's of a recorded tensor4 product whose formulation
+// may not be the one that is cached (*P.form: then there is nothing to do).
+enum LaunchMode { LM_COLOUR = 0, LM_ONE = 1, LM_RECORDED = 2 };
 
 // 1D weight of Gauss point i from the symmetric half in the kernel arguments
 template <int N> __device__ __forceinline__ double weight_1d(const double *qw, int i) {
@@ -1328,9 +1323,9 @@ template <int VAR, int TILE> constexpr int vmult_min_waves() {
   return TILE != kTileWide ? 1 : VAR == V_TENSOR2 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE ? 6 : 4;
 }
 
-// ONE: all tiles in this launch (see k_tile_sum), else one colour's.
+// ONE: all tiles in this launch, else one colour's.
 template <int DIM, int N, typename T, int VAR, bool ADD, bool CONSTR, unsigned PH, int TILE, bool ONE>
-__global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TILE>())) k_vmult(const VmultParams<T> P) {
+__device__ __forceinline__ void vmult_body(const VmultParams<T> &P, const T *__restrict__ cache) {
   using CS = CellShape<DIM, N>;
   // threads and cells of this workgroup: a tile, or CS::CPW cells
   constexpr int WG = tile_threads<TILE>();
@@ -1349,8 +1344,6 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
   __shared__ T lds[CPW * SLOTW + TABN + (KIN ? CPW * NC * DIM : 0) + RED];
   __shared__ T tile_v[TILE ? TN * DIM : 1];         // tile nodes' source values
   __shared__ uint32_t tile_c[TILE ? TN : 1];  // tile nodes' codes
-  const T *__restrict__ cache = cached_values<VAR, ONE>(P);
-  if (!ONE && P.form && !cache) return;
   T *tab = lds + CPW * SLOTW;
   T *Xall = tab + TABN;
   T *Rall = Xall + (KIN ? CPW * NC * DIM : 0);
@@ -1786,6 +1779,16 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
   }
 }
 
+template <int DIM, int N, typename T, int VAR, bool ADD, bool CONSTR, unsigned PH, int TILE, int MODE>
+__global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TILE>())) k_vmult(const VmultParams<T> P) {
+  if constexpr (MODE == LM_RECORDED) {
+    if (P.form->formulation == (VAR == V_TENSOR4 ? 0 : 1))
+      vmult_body<DIM, N, T, VAR, ADD, CONSTR, PH, TILE, false>(P, (const T *)(P.form->cache));
+  } else {
+    vmult_body<DIM, N, T, VAR, ADD, CONSTR, PH, TILE, MODE == LM_ONE>(P, P.cache);
+  }
+}
+
 // ------------------------------------------------------------------------
 // Fused product of the compact forms on wide 3D tiles: planes and columns.
 //
@@ -1928,7 +1931,7 @@ template <int N, typename T, int VAR> constexpr int planes_min_waves() {
 }
 
 template <int N, typename T, int VAR, bool ADD, bool CONSTR, int TILE, bool ONE>
-__global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_waves<N, T, VAR>())) k_vmult_planes(const VmultParams<T> P) {
+__device__ __forceinline__ void planes_body(const VmultParams<T> &P, const T *__restrict__ cache) {
   constexpr bool RES = VAR == V_RESIDUAL, ADJ = VAR == V_ADJOINT;  // affine cells, nothing cached
   constexpr bool SCAL = VAR == V_SCALAR, GEO = RES || ADJ || SCAL;  // affine cells, c cached; cgeo and material
   static_assert(VAR == V_COMPACT_U || GEO || (sizeof(T) == 4 && (VAR == V_COMPACT || VAR == V_COMPACT_AFFINE)));
@@ -1947,8 +1950,6 @@ __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_wave
   __shared__ double caff_all[CA];
   __shared__ T tile_u[RECOMP ? TN * 3 : 1];
   __shared__ T red[ADJ ? PS::CPW * 2 * NL : 1];  // columns' shares of dmu, dlambda
-  const T *__restrict__ cache = cached_values<VAR, ONE>(P);
-  if (!ONE && P.form && !cache) return;
   const T *src = P.src + (size_t)blockIdx.y * P.vstride;  // an epilogue updates it in place
   T *dst = P.dst + (size_t)blockIdx.y * P.vstride;
   const int t = threadIdx.x, wave = t / 64, lane = t % 64;
@@ -2242,6 +2243,34 @@ __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_wave
           dst[node * 3 + c] = (ADD ? tile_v[n * 3 + c] : T(0)) + src[node * 3 + c];
       }
     }
+  }
+}
+
+template <int N, typename T, int VAR, bool ADD, bool CONSTR, int TILE, int MODE>
+__global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_waves<N, T, VAR>())) k_vmult_planes(const VmultParams<T> P) {
+  if constexpr (MODE == LM_RECORDED) {
+    if (P.form->formulation == 1) planes_body<N, T, VAR, ADD, CONSTR, TILE, false>(P, (const T *)(P.form->cache));
+  } else {
+    planes_body<N, T, VAR, ADD, CONSTR, TILE, MODE == LM_ONE>(P, P.cache);
+  }
+}
+
+// One colour of a recorded tensor4 product in either formulation (*P.form), for
+// launches that leave the GPU idle anyway: a second launch, of which one has
+// nothing to do, costs 1.6 us on a replay, 13 us a product (16^3 Q2 FP64 75 us
+// against 62 for one formulation).  LDS and registers are those of both kernels
+// together, one workgroup per CU.  VAR: the compact form; PLANES: by the plane
+// kernel, whose workgroup is the smaller one.
+template <int DIM, int N, typename T, int VAR, bool ADD, bool CONSTR, unsigned PH, int TILE, bool PLANES>
+__global__ void __launch_bounds__(tile_threads<TILE>()) k_vmult_recorded(const VmultParams<T> P) {
+  const T *cache = (const T *)(P.form->cache);
+  if (P.form->formulation == 0) {
+    vmult_body<DIM, N, T, V_TENSOR4, ADD, CONSTR, PH, TILE, false>(P, cache);
+  } else if constexpr (PLANES) {
+    static_assert(PlaneShape<N, T, TILE>::WG <= tile_threads<TILE>());
+    if (threadIdx.x < PlaneShape<N, T, TILE>::WG) planes_body<N, T, VAR, ADD, CONSTR, TILE, false>(P, cache);
+  } else {
+    vmult_body<DIM, N, T, VAR, ADD, CONSTR, PH, TILE, false>(P, cache);
   }
 }
 

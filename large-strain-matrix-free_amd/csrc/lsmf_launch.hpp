@@ -34,14 +34,14 @@ template <int DIM, int N> struct Launch {
   // K from the displacement: that kernel only (cache_variant)
   static constexpr bool recompute_ok() { return DIM == 3 && N == 3; }
 
-  // one colour's fused cell kernel, or with ONE all tiles': n tiles (tiled
+  // one colour's fused cell kernel, or with LM_ONE all tiles': n tiles (tiled
   // layouts) or n cells, nv vectors (grid y)
-  template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH, bool ONE = false>
+  template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH, int MODE = LM_COLOUR>
   static int launch_vmult(const lsmf_op *op, const VmultParams<T> &P, int n, unsigned nv, hipStream_t s) {
     if (op->tile_kind == kTileWide) {
       if constexpr (planes_ok<T, VAR>() && PH == (PH_SF | PH_QD)) {
         if (op->planes) {
-          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide, ONE>), dim3(n, nv),
+          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide, MODE>), dim3(n, nv),
                              dim3((PlaneShape<N, T, kTileWide>::WG)), 0, s, P);
           return 0;
         }
@@ -49,7 +49,7 @@ template <int DIM, int N> struct Launch {
       if constexpr (kinematic_planes<T, VAR>()) {
         // residual and VJP in formulation 1 on affine cells
         if (op->d_cgeo && op->formulation == 1) {
-          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide, ONE>), dim3(n, nv),
+          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide, MODE>), dim3(n, nv),
                            dim3((PlaneShape<N, T, kTileWide>::WG)), 0,
                              s, P);
           return 0;
@@ -58,7 +58,7 @@ template <int DIM, int N> struct Launch {
       if constexpr (VAR == V_COMPACT_U && PH == (PH_SF | PH_QD))
         return LSMF_ERR_UNSUPPORTED;
       else if constexpr (wide_ok<VAR>())
-        hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide, ONE>), dim3(n, nv),
+        hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide, MODE>), dim3(n, nv),
                            dim3(tile_threads<kTileWide>()), 0, s, P);
       else
         return LSMF_ERR_UNSUPPORTED;
@@ -68,16 +68,16 @@ template <int DIM, int N> struct Launch {
       if constexpr (DIM == 3 && N == 3 && VAR == V_SCALAR && PH == (PH_SF | PH_QD)) {
         // formulation 1 on affine cells with the Q1 metric
         if (op->d_cgeo && op->formulation == 1) {
-          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, 1, ONE>), dim3(n, nv),
+          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, 1, MODE>), dim3(n, nv),
                              dim3((PlaneShape<N, T, 1>::WG)), 0, s, P);
           return 0;
         }
       }
-      hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, 1, ONE>), dim3(n, nv), dim3(kWG), 0, s, P);
-    } else if constexpr (ONE) {
+      hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, 1, MODE>), dim3(n, nv), dim3(kWG), 0, s, P);
+    } else if constexpr (MODE == LM_ONE) {
       return LSMF_ERR_UNSUPPORTED;
     } else {
-      hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, 0, false>), dim3(grid_for(n), nv), dim3(kWG), 0, s, P);
+      hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, 0, MODE>), dim3(grid_for(n), nv), dim3(kWG), 0, s, P);
     }
     return 0;
   }
@@ -214,7 +214,7 @@ template <int DIM, int N> struct Launch {
     P.dst = dst;
     P.identity = identity;
     if (op->prof) op->prof->before(s);
-    const int rc = launch_vmult<T, VAR, ADD, CONSTR, PH, true>(op, P, P.cell_end, 1, s);
+    const int rc = launch_vmult<T, VAR, ADD, CONSTR, PH, LM_ONE>(op, P, P.cell_end, 1, s);
     if (rc) return rc;
     tile_sum<T, ADD, CONSTR>(op, dst, src, identity, s, ep);
     if (op->prof) op->prof->after(s);
@@ -240,8 +240,9 @@ template <int DIM, int N> struct Launch {
 
   // A product recorded in a caller's graph: the caller may switch the
   // formulation, cache and replay, so where the formulations take other kernels
-  // both are recorded, and on a replay the one whose values are cached runs
-  // (*P.form).  The owner of a bound operator records its graphs anew instead.
+  // both are recorded, in one launch or two, and on a replay the one whose values
+  // are cached runs (*P.form).  The owner of a bound operator records its graphs anew instead.
+  static constexpr size_t kRecordedBlocks = 256;  // one workgroup per CU: one launch for both (k_vmult_recorded)
   static bool both_formulations(const lsmf_op *op, hipStream_t s) {
     if (!op->d_form || !capturing(s)) return false;
     op->recorded = true;
@@ -251,15 +252,44 @@ template <int DIM, int N> struct Launch {
   static int launch_recorded(const lsmf_op *op, VmultParams<T> P, int n, unsigned nv, hipStream_t s) {
     P.form = op->d_form;
     P.u = static_cast<const T *>(VAR == V_COMPACT_U ? op->d_uc : op->d_u);
-    return launch_vmult<T, VAR, ADD, CONSTR, PH>(op, P, n, nv, s);
+    const unsigned blocks = op->tile_kind ? (unsigned)n : grid_for(n);
+    if ((size_t)blocks * nv > kRecordedBlocks) {
+      const int rc = launch_vmult<T, V_TENSOR4, ADD, CONSTR, PH, LM_RECORDED>(op, P, n, nv, s);
+      return rc ? rc : launch_vmult<T, VAR, ADD, CONSTR, PH, LM_RECORDED>(op, P, n, nv, s);
+    }
+    constexpr bool PLANES = planes_ok<T, VAR>() && PH == (PH_SF | PH_QD);
+    if (op->tile_kind == kTileWide) {
+      if constexpr (PLANES)
+        if (op->planes) {
+          hipLaunchKernelGGL((k_vmult_recorded<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide, true>), dim3(blocks, nv),
+                             dim3(tile_threads<kTileWide>()), 0, s, P);
+          return 0;
+        }
+      if constexpr (wide_ok<VAR>() && !(VAR == V_COMPACT_U && PLANES)) {
+        hipLaunchKernelGGL((k_vmult_recorded<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide, false>), dim3(blocks, nv),
+                           dim3(tile_threads<kTileWide>()), 0, s, P);
+        return 0;
+      }
+    } else if constexpr (VAR != V_COMPACT_U) {
+      if (op->tile_kind == 1) {
+        if constexpr (!(DIM == 3 && (N == 5 || N == 3))) {  // tensor4 has wide tiles there
+          hipLaunchKernelGGL((k_vmult_recorded<DIM, N, T, VAR, ADD, CONSTR, PH, 1, false>), dim3(blocks, nv), dim3(kWG),
+                             0, s, P);
+          return 0;
+        }
+      } else {
+        hipLaunchKernelGGL((k_vmult_recorded<DIM, N, T, VAR, ADD, CONSTR, PH, 0, false>), dim3(blocks, nv), dim3(kWG), 0,
+                           s, P);
+        return 0;
+      }
+    }
+    return LSMF_ERR_UNSUPPORTED;
   }
   // one colour's cell kernel, or with both the kernels of both formulations
   template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH>
   static int launch_colour(const lsmf_op *op, const VmultParams<T> &P, int n, unsigned nv, bool both, hipStream_t s) {
     if (!both) return launch_vmult<T, VAR, ADD, CONSTR, PH>(op, P, n, nv, s);
     if constexpr (VAR == V_TENSOR4 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U) {
-      const int rc = launch_recorded<T, V_TENSOR4, ADD, CONSTR, PH>(op, P, n, nv, s);
-      if (rc) return rc;
       switch (compact_variant(op)) {
         case V_COMPACT: return launch_recorded<T, V_COMPACT, ADD, CONSTR, PH>(op, P, n, nv, s);
         case V_COMPACT_AFFINE: return launch_recorded<T, V_COMPACT_AFFINE, ADD, CONSTR, PH>(op, P, n, nv, s);

@@ -133,3 +133,38 @@ def test_vcycle_follows_the_fine_operator(device):
     for a, b in zip(*results):
         assert torch.equal(a, b)
     assert not torch.equal(results[0][0], results[0][1]) and torch.equal(results[0][0], results[0][-1])
+
+
+@pytest.mark.parametrize("precision,layout,n", [("fp64", "auto", [36, 40, 36]), ("fp32", "auto", [36, 40, 36]),
+                                                ("fp64", "cells", [28, 28, 28])], ids=lambda v: str(v).replace(" ", ""))
+def test_replays_of_many_tiles(precision, layout, n, device):
+    """more than 256 workgroups per colour, where the formulations' kernels are
+    recorded one after the other: replays give the eager products' bits"""
+    import torch
+    print(f"[recorded] {n} {precision} {layout}", flush=True)
+    mesh = lsmf.Mesh(3, 2, n)
+    rng = np.random.default_rng(3)
+    u, _ = lsmf.smooth_displacement(mesh.coords, 0.02, 7)
+    op = lsmf.NeoHookOperator(mesh, precision=precision, caching="tensor4", layout=layout)
+    op.set_material(1.0 + rng.random(mesh.n_cells), 2.0 + rng.random(mesh.n_cells))
+    ud = torch.tensor(u, device=device)
+    x = torch.tensor(rng.standard_normal(mesh.n_dofs), device=device).to(op.dtype)
+    y, z = torch.empty_like(x), torch.empty_like(x)
+    op.set_linearization(ud)
+    op.cache()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        op.vmult(y, x)
+    results = []
+    for formulation in (1, 0, 1):
+        lsmf._check(lsmf._lib.lsmf_set_formulation(op._h, formulation))
+        op.set_linearization(ud)
+        op.cache()
+        for _ in range(2):
+            y.fill_(float("nan"))
+            graph.replay()
+            op.vmult(z, x)
+            torch.cuda.synchronize()
+            assert torch.equal(y, z), formulation
+        results.append(z.clone())
+    assert torch.equal(results[0], results[2]) and not torch.equal(results[0], results[1])
