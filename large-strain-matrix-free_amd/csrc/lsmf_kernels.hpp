@@ -1230,7 +1230,8 @@ template <int DIM, int N, typename T, bool LINE = false, int CPW = CellShape<DIM
 __device__ __forceinline__ void kinematics_prologue(const VmultParams<T> &P, const T *tab, T *A, T *B, T *Xc,
                                                     bool on, bool active, uint32_t code, int r, int i0, int i1, int i2,
                                                     T (&F)[DIM][DIM], T (&Jri)[DIM][DIM], T &detJr, T (&Gu)[DIM][DIM],
-                                                    T *lds = nullptr, int t = 0, int slot = 0) {
+                                                    T *lds = nullptr, int t = 0, int slot = 0,
+                                                    bool affine = AFFINE) {
   constexpr int NQP = ipow(N, DIM);
   const int node = code & kNodeMask;
   if (active) {
@@ -1247,7 +1248,7 @@ __device__ __forceinline__ void kinematics_prologue(const VmultParams<T> &P, con
   else
     SF<DIM, N, T>::template evaluate<DIM>(tab, A, B, on, r, i0, i1, i2, Gu);
   T Jr[DIM][DIM];
-  if constexpr (AFFINE) affine_jacobian<DIM>(Xc, Jr);
+  if (AFFINE || affine) affine_jacobian<DIM>(Xc, Jr);
   else q1_jacobian<DIM, T, T>(Xc, tab + 4 * N * N, i0, i1, i2, Jr);
   detJr = inverse<DIM>(Jr, Jri);
   grad_times<DIM>(Gu, Jri, F);
@@ -2418,6 +2419,7 @@ struct CacheParams {
   int n_cells;
   int formulation;
   int curved;  // Eulerian Q_p metric for the spatial caches (tensor2, tensor4)
+  int affine;  // affine cells
   int *bad;
   double sf[2 * 15];  // even-odd 1D matrices, see VmultParams
 };
@@ -2453,7 +2455,8 @@ template <int DIM, int N, typename T, int VAR> __global__ void __launch_bounds__
   for (int k = 0; k < 2 * 15; ++k) KP.sf[k] = P.sf[k];
   double F[DIM][DIM], Jri[DIM][DIM], detJr, Gu[DIM][DIM], GX[DIM][DIM];
   kinematics_prologue<DIM, N, double, LINE, CPW, kWG, VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U>(
-      KP, tab, A, B, Xc, on, active, code, r, i0, i1, i2, F, Jri, detJr, Gu, lds, t, slot);
+      KP, tab, A, B, Xc, on, active, code, r, i0, i1, i2, F, Jri, detJr, Gu, lds, t, slot,
+      VAR == V_COMPACT_AFFINE || VAR == V_COMPACT_U || (VAR == V_COMPACT && P.affine));
   // the spatial caches carry the current metric: Eulerian Q_p on curved meshes
   constexpr bool SPATIAL = (VAR == V_TENSOR2 || VAR == V_TENSOR4);
   if (SPATIAL && P.curved)

@@ -13,8 +13,8 @@ template <int DIM, int N> struct Launch {
 
   // wide tiles exist for 3D Q4 and the variants that run on tensor2 /
   // tensor4 operators (their products, residual and residual VJP)
-  template <int VAR> static constexpr bool wide_ok() {
-    return DIM == 3 && (N == 5 || N == 3) &&
+  template <typename T, int VAR> static constexpr bool wide_ok() {
+    return DIM == 3 && (N == 5 || N == 3) && !(N == 3 && sizeof(T) == 8 && VAR == V_COMPACT_AFFINE) &&
            (VAR == V_TENSOR2 || VAR == V_TENSOR4 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE ||
             VAR == V_COMPACT_U || VAR == V_RESIDUAL || VAR == V_ADJOINT);
   }
@@ -57,7 +57,7 @@ template <int DIM, int N> struct Launch {
       }
       if constexpr (VAR == V_COMPACT_U && PH == (PH_SF | PH_QD))
         return LSMF_ERR_UNSUPPORTED;
-      else if constexpr (wide_ok<VAR>())
+      else if constexpr (wide_ok<T, VAR>())
         hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide, MODE>), dim3(n, nv),
                            dim3(tile_threads<kTileWide>()), 0, s, P);
       else
@@ -265,7 +265,7 @@ template <int DIM, int N> struct Launch {
                              dim3(tile_threads<kTileWide>()), 0, s, P);
           return 0;
         }
-      if constexpr (wide_ok<VAR>() && !(VAR == V_COMPACT_U && PLANES)) {
+      if constexpr (wide_ok<T, VAR>() && !(VAR == V_COMPACT_U && PLANES)) {
         hipLaunchKernelGGL((k_vmult_recorded<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide, false>), dim3(blocks, nv),
                            dim3(tile_threads<kTileWide>()), 0, s, P);
         return 0;
@@ -497,6 +497,7 @@ template <int DIM, int N> struct Launch {
     P.n_cells = op->n_cells;
     P.formulation = op->formulation;
     P.curved = op->curved;
+    P.affine = op->affine;
     P.bad = bad;
     pack_sf<double>(op, P.sf);
     hipLaunchKernelGGL((k_cache<DIM, N, T, VAR>), dim3(grid_for(op->n_cells)), dim3(kWG), 0, s, P);
@@ -548,7 +549,7 @@ template <int DIM, int N> struct Launch {
       if (op->caching == LSMF_CACHING_SCALAR_REFERENTIAL) P.curved = 0;
       if (n <= 0) return 0;
       if (op->tile_kind == kTileWide) {
-        if constexpr (wide_ok<VAR>())
+        if constexpr (wide_ok<T, VAR>())
           hipLaunchKernelGGL((k_diagonal_tiles<DIM, N, T, VAR, kTileWide>), dim3(n),
                              dim3(tile_threads<kTileWide>()), 0, s, P);
         else

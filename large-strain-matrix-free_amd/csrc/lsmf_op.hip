@@ -58,8 +58,17 @@ size_t elem_size(const lsmf_op *op) { return op->precision == LSMF_FP64 ? sizeof
 static bool recompute_k(const lsmf_op *op) {
   return op->affine && op->precision == LSMF_FP64 && op->planes;
 }
+// Wide-tile operators of up to kFewPoints points keep all values of the compact
+// form per point on affine cells too: their caches stay on the chip, and a load
+// of the cell's constants more is what such short launches wait for.  Per point /
+// per cell, us: 16^3 Q2 FP32 11.1 / 11.7 in one launch, 49.7 / 54 in coloured
+// ones, 16^3 Q4 (512 k points) FP64 30.0 / 30.0 and 68.4 / 72.9, FP32 20.4 / 20.3
+// and 53.5 / 59.7; 28^3 Q2 FP32 (593 k) 21.0 / 20.8, 32^3 Q4 FP64 216 / 200.
+constexpr size_t kFewPoints = (size_t)1 << 19;
 int compact_variant(const lsmf_op *op) {
-  return recompute_k(op) ? V_COMPACT_U : op->affine ? V_COMPACT_AFFINE : V_COMPACT;
+  if (recompute_k(op)) return V_COMPACT_U;
+  const bool few = op->tile_kind == kTileWide && op->field_stride <= kFewPoints;
+  return op->affine && !few ? V_COMPACT_AFFINE : V_COMPACT;
 }
 int cache_variant(const lsmf_op *op) {
   switch (op->caching) {
@@ -427,7 +436,7 @@ constexpr int kNotTileable = 1;
 // (24^3, 2.7 M), 117 / 118 (32^3, 6.4 M), 217 / 206 (40^3); 2D Q2 FP64 (4
 // colours) 50 / 58 (2.1 M), 190 / 173 (8.4 M).
 constexpr size_t kOneLaunchDofs = 4000000;
-// FP64 products on affine Q2 cells of kFewTiles + 1 to kLineTiles wide tiles keep
+// FP64 products on affine Q2 cells of kFewTiles + 1 to kLineTiles wide tiles cache
 // K and run the line kernel: there a launch lasts as long as one tile, and the
 // plane kernel's tile (two evaluations, one wave per six cells) takes longer.
 // Line / planes, us: 16^3 (256 tiles) 13.4 / 14.0 in one launch, 62 / 69 in
