@@ -159,7 +159,7 @@ void free_op(lsmf_op *op) {
   void *ptrs[] = {op->d_form, op->d_cache_other, op->d_cgeo, op->d_uc,   op->d_idx,  op->d_coords,    op->d_tab,  op->d_tab64, op->d_mu64,     op->d_lambda64,
                   op->d_mu,   op->d_lambda,    op->d_cache, op->d_caff, op->d_diag, op->d_inv_diag, op->d_cons,
                   op->d_bad,  op->d_perm,      op->d_tile_nodes, op->d_tile_info, op->d_tile_tables,
-                  op->d_tile_buf, op->d_orphan, op->d_hang, op->d_hptr,
+                  op->d_tile_buf, op->d_ctile_copy, op->d_orphan, op->d_hang, op->d_hptr,
                   op->d_hmaster, op->d_hw, op->d_hcons, op->d_hg_node, op->d_hg_ptr, op->d_hg_inst, op->d_hg_w,
                   op->d_hbuf, op->d_dcell, op->d_deptr, op->d_dtptr, op->d_dta, op->d_dtw, op->d_dbuf,
                   op->d_dg_node, op->d_dg_ptr, op->d_dg_ent};
@@ -377,21 +377,24 @@ bool cells_affine(const lsmf_mesh_desc *m, int dim, int p, int nqp) {
   }
   for (int c = 0; c < m->n_cells; ++c) {
     const int32_t *cn = m->cell_nodes + (size_t)c * nqp;
-    double X[8][3], top = 0.0;
-    for (int v = 0; v < NV; ++v)
-      for (int i = 0; i < dim; ++i) {
-        X[v][i] = m->coords[(size_t)cn[corner[v]] * dim + i];
-        top = std::max(top, std::fabs(X[v][i]));
-      }
-    const double tol = 8.0 * std::numeric_limits<double>::epsilon() * top;
+    const double *X[8];
+    for (int v = 0; v < NV; ++v) X[v] = m->coords + (size_t)cn[corner[v]] * dim;
+    // largest difference of a vertex from the affine map of vertex 0 and its
+    // neighbours; NaN counts as one
+    double off = 0.0;
     for (int i = 0; i < dim; ++i)
-      // vertex v against the affine map of vertex 0 and its neighbours
       for (int v = 3; v < NV; ++v) {
         double x = X[0][i];
         for (int d = 0; d < dim; ++d)
           if ((v >> d) & 1) x += X[1 << d][i] - X[0][i];
-        if (!(std::fabs(x - X[v][i]) <= tol)) return false;
+        const double e = std::fabs(x - X[v][i]);
+        if (!(e <= off) && !std::isnan(off)) off = e;
       }
+    if (off == 0.0) continue;
+    double top = 0.0;
+    for (int v = 0; v < NV; ++v)
+      for (int i = 0; i < dim; ++i) top = std::max(top, std::fabs(X[v][i]));
+    if (!(off <= 8.0 * std::numeric_limits<double>::epsilon() * top)) return false;
   }
   return true;
 }
@@ -446,8 +449,8 @@ constexpr size_t kOneLaunchDofs = 4000000;
 // FP32: the plane kernel at every size (16^3 11.8 / 11.7, 32^3 28 / 24.7).
 constexpr int kFewTiles = 16, kLineTiles = 512;
 struct TileTables {
-  std::vector<uint32_t> nodes, cnodes, priv, sum_node, sum_slot;
-  std::vector<int32_t> info, cinfo;
+  std::vector<uint32_t> nodes, priv, sum_node, sum_slot;
+  std::vector<int32_t> info, cinfo, by_colour;  // the last two: products in one launch
 };
 int build_tiles(lsmf_op *op, const lsmf_mesh_desc *mesh, const long long n[3], const std::vector<int32_t> &cell_at,
                 TileTables &tt) {
@@ -490,15 +493,32 @@ int build_tiles(lsmf_op *op, const lsmf_mesh_desc *mesh, const long long n[3], c
     at_ptr.push_back((int)at.size());
   }
   std::vector<const int32_t *> cell_nodes(td.tx * td.ty * td.tz);
+  auto extents = [&](long long b, int e[3]) {
+    e[0] = (int)std::min<long long>(td.tx, n[0] - b % TXn * td.tx);
+    e[1] = (int)std::min<long long>(td.ty, n[1] - b / TXn % TYn * td.ty);
+    e[2] = (int)std::min<long long>(td.tz, n[2] - b / (TXn * TYn) * td.tz);
+  };
+  // place of each tile in the tables, and its first cell in tile order; the walk
+  // below is in the order of the grid, as the mesh lies in memory
+  std::vector<int32_t> place(n_tiles);
   int pos = 0;
   for (long long i = 0; i < n_tiles; ++i) {
     const long long b = one ? i : by_colour[i];
-    const long long bx = b % TXn, by = (b / TXn) % TYn, bz = b / (TXn * TYn);
-    const int ex = (int)std::min<long long>(td.tx, n[0] - bx * td.tx);
-    const int ey = (int)std::min<long long>(td.ty, n[1] - by * td.ty);
-    const int ez = (int)std::min<long long>(td.tz, n[2] - bz * td.tz);
+    int e[3];
+    extents(b, e);
+    place[b] = (int32_t)i;
     tt.info[(size_t)i * 2] = pos;
-    tt.info[(size_t)i * 2 + 1] = ex | (ey << 8) | (ez << 16);
+    tt.info[(size_t)i * 2 + 1] = e[0] | (e[1] << 8) | (e[2] << 16);
+    pos += e[0] * e[1] * e[2];
+  }
+  if (pos != op->n_cells) return fail(LSMF_ERR_INVALID_ARGUMENT, "tiles: cell count mismatch");
+  for (long long b = 0; b < n_tiles; ++b) {
+    const long long bx = b % TXn, by = (b / TXn) % TYn, bz = b / (TXn * TYn);
+    int e[3];
+    extents(b, e);
+    const int ex = e[0], ey = e[1], ez = e[2];
+    const size_t i = (size_t)place[b];
+    pos = tt.info[i * 2];
     auto tile_cell = [&](int sx, int sy, int sz) {
       return cell_at[(bx * td.tx + sx) + n[0] * ((by * td.ty + sy) + n[1] * (bz * td.tz + sz))];
     };
@@ -527,10 +547,9 @@ int build_tiles(lsmf_op *op, const lsmf_mesh_desc *mesh, const long long n[3], c
       if (node < 0) continue;
       if ((cols[node] >> tcol[b]) & 1u) return kNotTileable;  // two tiles of one colour share a node
       cols[node] |= (uint8_t)(1u << tcol[b]);
-      tt.nodes[(size_t)i * td.tn + l] = (uint32_t)node;
+      tt.nodes[i * td.tn + l] = (uint32_t)node;
     }
   }
-  if (pos != op->n_cells) return fail(LSMF_ERR_INVALID_ARGUMENT, "tiles: cell count mismatch");
   auto cons_bits = [&](size_t node) {
     uint32_t bits = 0;
     if (mesh->constrained)
@@ -539,13 +558,13 @@ int build_tiles(lsmf_op *op, const lsmf_mesh_desc *mesh, const long long n[3], c
     return bits;
   };
   if (!one) {
-    for (long long i = 0; i < n_tiles; ++i)
+    for (long long b = 0; b < n_tiles; ++b)
       for (int l = 0; l < td.tn; ++l) {
-        uint32_t &code = tt.nodes[(size_t)i * td.tn + l];
+        uint32_t &code = tt.nodes[(size_t)place[b] * td.tn + l];
         if (code == kNoNode) continue;
         const uint32_t node = code;
         code |= cons_bits(node);
-        if (!(cols[node] & ((1u << tcol[by_colour[i]]) - 1u))) code |= kFirstBit;
+        if (!(cols[node] & ((1u << tcol[b]) - 1u))) code |= kFirstBit;
       }
     return LSMF_OK;
   }
@@ -589,15 +608,17 @@ int build_tiles(lsmf_op *op, const lsmf_mesh_desc *mesh, const long long n[3], c
       }
       if (!below) code |= kFirstBit;
     }
-  tt.cnodes.reserve(tt.nodes.size());
   tt.cinfo.reserve(tt.info.size());
-  for (const int32_t b : by_colour) {
-    tt.cnodes.insert(tt.cnodes.end(), tt.nodes.begin() + (size_t)b * td.tn, tt.nodes.begin() + (size_t)(b + 1) * td.tn);
-    tt.cinfo.insert(tt.cinfo.end(), {tt.info[(size_t)b * 2], tt.info[(size_t)b * 2 + 1]});
-  }
+  for (const int32_t b : by_colour) tt.cinfo.insert(tt.cinfo.end(), {tt.info[(size_t)b * 2], tt.info[(size_t)b * 2 + 1]});
+  tt.by_colour = std::move(by_colour);
   return LSMF_OK;
 }
 
+__global__ void k_tiles_by_colour(uint32_t *__restrict__ out, const uint32_t *__restrict__ nodes,
+                                  const uint32_t *__restrict__ tiles, int tn) {
+  for (int l = threadIdx.x; l < tn; l += blockDim.x)
+    out[(size_t)blockIdx.x * tn + l] = nodes[(size_t)tiles[blockIdx.x] * tn + l];
+}
 __global__ void k_set_form(lsmf::FormState *f, int formulation, const void *cache) {
   f->formulation = formulation;
   f->cache = (const __attribute__((address_space(1))) void *)cache;
@@ -856,8 +877,8 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
   }
   // --- index table (sorted cells): node | constraint bits | first-touch bit
   std::vector<uint32_t> idx((size_t)nc * nqp);
-  for (int pos = 0; pos < nc; ++pos) {
-    const int c = op->perm[pos];
+  for (int c = 0; c < nc; ++c) {
+    const int pos = op->inv_perm[c];
     for (int a = 0; a < nqp; ++a) {
       const int nd = mesh->cell_nodes[(size_t)c * nqp + a];
       uint32_t code = (uint32_t)nd;
@@ -1025,8 +1046,9 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
     cgeo.resize((size_t)nc * kAffineStride);
     int corner[8];
     for (int v = 0; v < 8; ++v) corner[v] = p * ((v & 1) + N * ((v >> 1 & 1) + N * (v >> 2 & 1)));
-    for (int pos = 0; pos < nc; ++pos) {
-      const int32_t *cn = mesh->cell_nodes + (size_t)op->perm[pos] * nqp;
+    for (int c = 0; c < nc; ++c) {
+      const int pos = op->inv_perm[c];
+      const int32_t *cn = mesh->cell_nodes + (size_t)c * nqp;
       double X[24], J[3][3], R[3][3];
       for (int v = 0; v < 8; ++v)
         for (int i = 0; i < 3; ++i) X[v * 3 + i] = mesh->coords[(size_t)cn[corner[v]] * 3 + i];
@@ -1041,10 +1063,11 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
         for (int d = 0; d < 3; ++d) g[7 + 3 * i + d] = kin_geo ? R[i][d] : J[i][d];
     }
   }
-  // the tables of products in one launch in one piece: info and nodes by colour,
-  // private bits, shared nodes, slots
+  // the tables of products in one launch in one piece: info by colour, tiles by
+  // colour, private bits, shared nodes, slots
   std::vector<uint32_t> tile_tables(tt.cinfo.begin(), tt.cinfo.end());
-  for (const auto *v : {&tt.cnodes, &tt.priv, &tt.sum_node, &tt.sum_slot}) tile_tables.insert(tile_tables.end(), v->begin(), v->end());
+  tile_tables.insert(tile_tables.end(), tt.by_colour.begin(), tt.by_colour.end());
+  for (const auto *v : {&tt.priv, &tt.sum_node, &tt.sum_slot}) tile_tables.insert(tile_tables.end(), v->begin(), v->end());
 
   const size_t es = elem_size(op);
   int rc = 0;
@@ -1070,6 +1093,7 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
       (rc = dalloc(&op->d_tile_nodes, tt.nodes.size(), "tile nodes")) ||
       (rc = dalloc(&op->d_tile_info, tt.info.size(), "tile info")) ||
       (rc = dalloc(&op->d_tile_tables, tile_tables.size(), "tile tables")) ||
+      (!tt.by_colour.empty() && (rc = dalloc(&op->d_ctile_copy, tt.nodes.size(), "tile nodes by colour"))) ||
       (nnc > 0 && ((rc = dalloc(&op->d_hang, hang_tab.size(), "constraint table")) ||
                    (rc = dalloc(&op->d_hptr, hptr.size(), "constraint offsets")) ||
                    (rc = dalloc(&op->d_hmaster, hmaster.size(), "constraint masters")) ||
@@ -1143,8 +1167,14 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
   if (e == hipSuccess && !tile_tables.empty()) {
     e = hipMemcpy(op->d_tile_tables, tile_tables.data(), tile_tables.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
     op->d_ctile_info = reinterpret_cast<const int32_t *>(op->d_tile_tables);
-    op->d_ctile_nodes = op->d_tile_tables + tt.cinfo.size();
-    op->d_tile_priv = op->d_ctile_nodes + tt.cnodes.size();
+    op->d_ctile_nodes = op->d_ctile_copy;
+    const uint32_t *by_colour = op->d_tile_tables + tt.cinfo.size();
+    op->d_tile_priv = by_colour + tt.by_colour.size();
+    const size_t n_tiles = tt.by_colour.size(), tn = tt.nodes.size() / n_tiles;
+    hipLaunchKernelGGL(k_tiles_by_colour, dim3((unsigned)n_tiles), dim3(256), 0, nullptr, op->d_ctile_copy,
+                       op->d_tile_nodes, by_colour, (int)tn);
+    if (e == hipSuccess) e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // products may start on any stream
     op->d_sum_node = op->d_tile_priv + tt.priv.size();
     op->d_sum_slot = op->d_sum_node + tt.sum_node.size();
   }
@@ -1195,6 +1225,7 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
     }
   }
   op->bytes_idx += tt.nodes.size() * sizeof(uint32_t) + tt.info.size() * sizeof(int32_t);
+  if (op->d_ctile_copy) op->bytes_sum += tt.nodes.size() * sizeof(uint32_t);
   if (e != hipSuccess) {
     free_op(op);
     delete op;

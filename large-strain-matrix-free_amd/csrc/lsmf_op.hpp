@@ -112,6 +112,7 @@ struct lsmf_op {
   uint32_t *d_tile_nodes = nullptr;  // [n_tiles][TN] node | constraint bits | first-touch bit, or kNoNode
   int32_t *d_tile_info = nullptr;    // [n_tiles][2] first sorted cell, extents ex | ey << 8 | ez << 16
   uint32_t *d_tile_tables = nullptr;  // the memory of the tables below
+  uint32_t *d_ctile_copy = nullptr;         // memory of d_ctile_nodes where it is not d_tile_nodes
   const uint32_t *d_ctile_nodes = nullptr;  // the same two by colour
   const int32_t *d_ctile_info = nullptr;
   // products in one launch over all tiles (k_vmult, k_tile_sum):
