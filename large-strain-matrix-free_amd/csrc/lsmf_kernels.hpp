@@ -1818,14 +1818,15 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
 // error falls from 1.9e-6 to 1.7e-7 (no tau = mu F F^T - c I to cancel).
 // ------------------------------------------------------------------------
 template <int N, typename T, int TILE> struct PlaneShape {
-  // Q2: ten lanes (nine used) and a padded slot per cell, so that planes
-  // (lanes 9 values apart) and columns (neighbours) spread over all banks
-  static constexpr int LPC = N == 3 ? 10 : N * N;  // lanes per cell
-  static constexpr int CPV = 64 / LPC;             // cells per wave
+  // ten lanes (nine used) and a padded slot per cell, so that planes (lanes 9
+  // values apart) and columns (neighbours) spread over all banks
+  static_assert(N == 3, "Q2");
+  static constexpr int LPC = 10;        // lanes per cell
+  static constexpr int CPV = 64 / LPC;  // cells per wave
   static constexpr int CPW = TileShape<3, N, tile_threads<TILE>()>::CPW;
   static constexpr int WAVES = (CPW + CPV - 1) / CPV;
   static constexpr int WG = 64 * WAVES;
-  static constexpr int SLOT = N == 3 ? (sizeof(T) == 8 ? 250 : 266) : 9 * N * N * N;
+  static constexpr int SLOT = sizeof(T) == 8 ? 250 : 266;
 };
 // LDS order within a wave: the accesses of its lanes are in order in
 // hardware, this keeps the compiler to it
@@ -1931,17 +1932,22 @@ template <int N, typename T, int VAR> constexpr int planes_min_waves() {
   return VAR == V_ADJOINT ? 2 : sizeof(T) == 8 ? 3 : 4;
 }
 
-template <int N, typename T, int VAR, bool ADD, bool CONSTR, int TILE, bool ONE>
+template <int N, typename T, int VAR, bool ADD, bool CONSTR, unsigned PH, int TILE, bool ONE>
 __device__ __forceinline__ void planes_body(const VmultParams<T> &P, const T *__restrict__ cache) {
   constexpr bool RES = VAR == V_RESIDUAL, ADJ = VAR == V_ADJOINT;  // affine cells, nothing cached
-  constexpr bool SCAL = VAR == V_SCALAR, GEO = RES || ADJ || SCAL;  // affine cells, c cached; cgeo and material
-  static_assert(VAR == V_COMPACT_U || GEO || (sizeof(T) == 4 && (VAR == V_COMPACT || VAR == V_COMPACT_AFFINE)));
-  constexpr bool AFFINE = VAR != V_COMPACT, RECOMP = VAR == V_COMPACT_U || GEO;
+  constexpr bool SCAL = VAR == V_SCALAR;                           // affine cells, c cached
+  static_assert(VAR == V_COMPACT_U || RES || ADJ || SCAL ||
+                (sizeof(T) == 4 && (VAR == V_COMPACT || VAR == V_COMPACT_AFFINE)));
+  // phases (see k_vmult); the tangent's data belong to its phase
+  constexpr bool SUMS = PH & PH_SF, QD = PH & PH_QD;
+  static_assert((SUMS && QD) || !(RES || ADJ));
+  constexpr bool GEO = QD && (RES || ADJ || SCAL);  // geometry table and material
+  constexpr bool AFFINE = QD && VAR != V_COMPACT, RECOMP = QD && (VAR == V_COMPACT_U || GEO);
   using PS = PlaneShape<N, T, TILE>;
   using TS = TileShape<3, N, tile_threads<TILE>()>;
   using SF3 = SFPlane<N, T>;
   constexpr int NQP = N * N * N, NL = N * N, TN = TS::TN, WG = PS::WG, PP = N - 1;
-  constexpr int NF = CacheFields<3, VAR>::value;  // 0: RES, ADJ
+  constexpr int NF = QD ? CacheFields<3, VAR>::value : 0;  // 0: RES, ADJ
   constexpr int ROUNDS = (TN + WG - 1) / WG;
   constexpr int NCA = RECOMP ? 16 : 7;  // constants per cell
   constexpr int CA = AFFINE ? PS::CPW * NCA : 1;
@@ -2129,13 +2135,23 @@ __device__ __forceinline__ void planes_body(const VmultParams<T> &P, const T *__
         if (t + k * WG < TN)
 #pragma unroll
           for (int c = 0; c < 3; ++c) tile_v[(t + k * WG) * 3 + c] = dv[k][c];
-      if (pln) SF3::evaluate_plane(P.sf, plane, x);
+      if (pln) {
+        if constexpr (SUMS) {
+          SF3::evaluate_plane(P.sf, plane, x);
+        } else {
+#pragma unroll
+          for (int y = 0; y < N; ++y)
+#pragma unroll
+            for (int i = 0; i < N; ++i) plane[y * N + i] = x[y][i];
+        }
+      }
     }
     wave_lds_fence();
-    if (col) {
+    if (SUMS && col) {
       T G[3][3][N], dmu = T(0), dlam = T(0);
 #pragma unroll
       for (int c = 0; c < 3; ++c) SF3::evaluate_column(P.sf, A + c * NQP + j, G[c]);
+      if constexpr (QD)
 #pragma unroll
       for (int k = 0; k < N; ++k) {
         T g[3][3], Phi[3][3];
@@ -2198,7 +2214,7 @@ __device__ __forceinline__ void planes_body(const VmultParams<T> &P, const T *__
     }
   }
   wave_lds_fence();
-  if (pln) SF3::integrate_plane(P.sf, plane);
+  if (SUMS && pln) SF3::integrate_plane(P.sf, plane);
   if constexpr (ADJ)
     if (has && j < 2) {
       // the cell's columns in order (same wave)
@@ -2247,12 +2263,12 @@ __device__ __forceinline__ void planes_body(const VmultParams<T> &P, const T *__
   }
 }
 
-template <int N, typename T, int VAR, bool ADD, bool CONSTR, int TILE, int MODE>
+template <int N, typename T, int VAR, bool ADD, bool CONSTR, unsigned PH, int TILE, int MODE>
 __global__ void __launch_bounds__((PlaneShape<N, T, TILE>::WG), (planes_min_waves<N, T, VAR>())) k_vmult_planes(const VmultParams<T> P) {
   if constexpr (MODE == LM_RECORDED) {
-    if (P.form->formulation == 1) planes_body<N, T, VAR, ADD, CONSTR, TILE, false>(P, (const T *)(P.form->cache));
+    if (P.form->formulation == 1) planes_body<N, T, VAR, ADD, CONSTR, PH, TILE, false>(P, (const T *)(P.form->cache));
   } else {
-    planes_body<N, T, VAR, ADD, CONSTR, TILE, MODE == LM_ONE>(P, P.cache);
+    planes_body<N, T, VAR, ADD, CONSTR, PH, TILE, MODE == LM_ONE>(P, P.cache);
   }
 }
 
@@ -2269,7 +2285,7 @@ __global__ void __launch_bounds__(tile_threads<TILE>()) k_vmult_recorded(const V
     vmult_body<DIM, N, T, V_TENSOR4, ADD, CONSTR, PH, TILE, false>(P, cache);
   } else if constexpr (PLANES) {
     static_assert(PlaneShape<N, T, TILE>::WG <= tile_threads<TILE>());
-    if (threadIdx.x < PlaneShape<N, T, TILE>::WG) planes_body<N, T, VAR, ADD, CONSTR, TILE, false>(P, cache);
+    if (threadIdx.x < PlaneShape<N, T, TILE>::WG) planes_body<N, T, VAR, ADD, CONSTR, PH, TILE, false>(P, cache);
   } else {
     vmult_body<DIM, N, T, VAR, ADD, CONSTR, PH, TILE, false>(P, cache);
   }

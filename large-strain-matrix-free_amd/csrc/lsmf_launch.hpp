@@ -11,22 +11,22 @@ namespace lsmf {
 template <int DIM, int N> struct Launch {
   using CS = CellShape<DIM, N>;
 
-  // wide tiles exist for 3D Q4 and the variants that run on tensor2 /
-  // tensor4 operators (their products, residual and residual VJP)
-  template <typename T, int VAR> static constexpr bool wide_ok() {
-    return DIM == 3 && (N == 5 || N == 3) && !(N == 3 && sizeof(T) == 8 && VAR == V_COMPACT_AFFINE) &&
-           (VAR == V_TENSOR2 || VAR == V_TENSOR4 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE ||
-            VAR == V_COMPACT_U || VAR == V_RESIDUAL || VAR == V_ADJOINT);
-  }
-
-  // products of the compact forms on wide tiles (lsmf_op::planes): K from the
-  // displacement, or cached in FP32.  With 17 cached FP64 values per point
+  // products of the compact forms on wide Q2 tiles that run the plane kernel: K
+  // from the displacement, or cached in FP32.  With 17 cached FP64 values per point
   // (bilinear cells) the line kernel is the faster one, the values of a plane
   // lane's column do not fit its registers: 64^3 311 us against 410, 32^3 41.1
   // against 48, on another stream 69.7 against 79.
   template <typename T, int VAR> static constexpr bool planes_ok() {
     return DIM == 3 && N == 3 &&
            (VAR == V_COMPACT_U || (sizeof(T) == 4 && (VAR == V_COMPACT || VAR == V_COMPACT_AFFINE)));
+  }
+  // wide tiles with the line kernel: 3D Q4 and Q2, the other variants that run on
+  // tensor2 / tensor4 operators (their products, residual and residual VJP)
+  template <typename T, int VAR> static constexpr bool wide_ok() {
+    return DIM == 3 && (N == 5 || N == 3) && !planes_ok<T, VAR>() &&
+           !(N == 3 && sizeof(T) == 8 && VAR == V_COMPACT_AFFINE) &&
+           (VAR == V_TENSOR2 || VAR == V_TENSOR4 || VAR == V_COMPACT || VAR == V_COMPACT_AFFINE ||
+            VAR == V_RESIDUAL || VAR == V_ADJOINT);
   }
   template <typename T, int VAR> static constexpr bool kinematic_planes() {
     return DIM == 3 && N == 3 && sizeof(T) == 8 && (VAR == V_RESIDUAL || VAR == V_ADJOINT);
@@ -39,25 +39,15 @@ template <int DIM, int N> struct Launch {
   template <typename T, int VAR, bool ADD, bool CONSTR, unsigned PH, int MODE = LM_COLOUR>
   static int launch_vmult(const lsmf_op *op, const VmultParams<T> &P, int n, unsigned nv, hipStream_t s) {
     if (op->tile_kind == kTileWide) {
-      if constexpr (planes_ok<T, VAR>() && PH == (PH_SF | PH_QD)) {
-        if (op->planes) {
-          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide, MODE>), dim3(n, nv),
+      if constexpr (planes_ok<T, VAR>() || kinematic_planes<T, VAR>()) {
+        // residual and VJP: formulation 1 on affine cells
+        if (planes_ok<T, VAR>() || (op->d_cgeo && op->formulation == 1)) {
+          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, PH, kTileWide, MODE>), dim3(n, nv),
                              dim3((PlaneShape<N, T, kTileWide>::WG)), 0, s, P);
           return 0;
         }
       }
-      if constexpr (kinematic_planes<T, VAR>()) {
-        // residual and VJP in formulation 1 on affine cells
-        if (op->d_cgeo && op->formulation == 1) {
-          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, kTileWide, MODE>), dim3(n, nv),
-                           dim3((PlaneShape<N, T, kTileWide>::WG)), 0,
-                             s, P);
-          return 0;
-        }
-      }
-      if constexpr (VAR == V_COMPACT_U && PH == (PH_SF | PH_QD))
-        return LSMF_ERR_UNSUPPORTED;
-      else if constexpr (wide_ok<T, VAR>())
+      if constexpr (wide_ok<T, VAR>())
         hipLaunchKernelGGL((k_vmult<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide, MODE>), dim3(n, nv),
                            dim3(tile_threads<kTileWide>()), 0, s, P);
       else
@@ -65,10 +55,10 @@ template <int DIM, int N> struct Launch {
     } else if constexpr (VAR == V_COMPACT_U) {
       return LSMF_ERR_UNSUPPORTED;
     } else if (op->tile_kind == 1) {
-      if constexpr (DIM == 3 && N == 3 && VAR == V_SCALAR && PH == (PH_SF | PH_QD)) {
+      if constexpr (DIM == 3 && N == 3 && VAR == V_SCALAR) {
         // formulation 1 on affine cells with the Q1 metric
         if (op->d_cgeo && op->formulation == 1) {
-          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, 1, MODE>), dim3(n, nv),
+          hipLaunchKernelGGL((k_vmult_planes<N, T, VAR, ADD, CONSTR, PH, 1, MODE>), dim3(n, nv),
                              dim3((PlaneShape<N, T, 1>::WG)), 0, s, P);
           return 0;
         }
@@ -257,17 +247,10 @@ template <int DIM, int N> struct Launch {
       const int rc = launch_vmult<T, V_TENSOR4, ADD, CONSTR, PH, LM_RECORDED>(op, P, n, nv, s);
       return rc ? rc : launch_vmult<T, VAR, ADD, CONSTR, PH, LM_RECORDED>(op, P, n, nv, s);
     }
-    constexpr bool PLANES = planes_ok<T, VAR>() && PH == (PH_SF | PH_QD);
     if (op->tile_kind == kTileWide) {
-      if constexpr (PLANES)
-        if (op->planes) {
-          hipLaunchKernelGGL((k_vmult_recorded<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide, true>), dim3(blocks, nv),
-                             dim3(tile_threads<kTileWide>()), 0, s, P);
-          return 0;
-        }
-      if constexpr (wide_ok<T, VAR>() && !(VAR == V_COMPACT_U && PLANES)) {
-        hipLaunchKernelGGL((k_vmult_recorded<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide, false>), dim3(blocks, nv),
-                           dim3(tile_threads<kTileWide>()), 0, s, P);
+      if constexpr (planes_ok<T, VAR>() || wide_ok<T, VAR>()) {
+        hipLaunchKernelGGL((k_vmult_recorded<DIM, N, T, VAR, ADD, CONSTR, PH, kTileWide, planes_ok<T, VAR>()>),
+                           dim3(blocks, nv), dim3(tile_threads<kTileWide>()), 0, s, P);
         return 0;
       }
     } else if constexpr (VAR != V_COMPACT_U) {
@@ -549,7 +532,7 @@ template <int DIM, int N> struct Launch {
       if (op->caching == LSMF_CACHING_SCALAR_REFERENTIAL) P.curved = 0;
       if (n <= 0) return 0;
       if (op->tile_kind == kTileWide) {
-        if constexpr (wide_ok<T, VAR>())
+        if constexpr (wide_ok<T, VAR>() || planes_ok<T, VAR>())
           hipLaunchKernelGGL((k_diagonal_tiles<DIM, N, T, VAR, kTileWide>), dim3(n),
                              dim3(tile_threads<kTileWide>()), 0, s, P);
         else

@@ -51,12 +51,13 @@ size_t elem_size(const lsmf_op *op) { return op->precision == LSMF_FP64 ? sizeof
 // tensors.
 // K from the displacement instead of from memory (one cached value per point
 // instead of ten), by the plane kernel: FP64 operators on wide Q2 tiles of affine
-// cells, with lsmf_op::planes.  Against the line kernel with K cached, us: 128^3
-// 1558 / 1820, 64^3 249 / 282, 32^3 39.7 / 41.1.  FP32 operators keep K, which is
-// rounded once from FP64; from an FP32 displacement it would lose the digits of
-// |u| / h.
+// cells, but for kFewTiles + 1 to kLineTiles of them.  Against the line kernel
+// with K cached, us: 128^3 1500 / 1820, 64^3 249 / 282, 32^3 39.7 / 41.1.  FP32
+// operators keep K, which is rounded once from FP64; from an FP32 displacement
+// it would lose the digits of |u| / h.
 static bool recompute_k(const lsmf_op *op) {
-  return op->affine && op->precision == LSMF_FP64 && op->planes;
+  return op->affine && op->precision == LSMF_FP64 && op->dim == 3 && op->N == 3 && op->tile_kind == kTileWide &&
+         !op->few_tiles;
 }
 // Wide-tile operators of up to kFewPoints points keep all values of the compact
 // form per point on affine cells too: their caches stay on the chip, and a load
@@ -814,10 +815,8 @@ lsmf_status lsmf_op_create(const lsmf_mesh_desc *mesh, const lsmf_op_options *op
       return rc;
     }
   }
-  if (op->tiled && dim == 3 && N == 3 && op->tile_kind == kTileWide) {
-    const int n_tiles = op->tile_ptr.back();
-    op->planes = op->precision == LSMF_FP32 || n_tiles <= kFewTiles || n_tiles > kLineTiles;
-  }
+  if (op->tiled && dim == 3 && N == 3 && op->tile_kind == kTileWide)
+    op->few_tiles = op->tile_ptr.back() > kFewTiles && op->tile_ptr.back() <= kLineTiles;
   op->n_fields = n_cache_fields(op);
   // --- colouring (given and checked, or greedy first fit): no node is written
   // by two cells of one colour; used[n] = colours of the cells that write n.

@@ -107,7 +107,7 @@ struct lsmf_op {
   // alone.  Tiles of colour k are entries [tile_ptr[k], tile_ptr[k+1])
   bool tiled = false;
   int tile_kind = 0;  // TILE argument of the cell kernels: 0 cells, 1 tiles, 2 wide tiles
-  bool planes = false;  // wide 3D Q2 tiles whose compact products may run k_vmult_planes
+  bool few_tiles = false;  // 3D Q2, kFewTiles + 1 to kLineTiles wide tiles (lsmf_op.hip)
   std::vector<int> tile_ptr;
   uint32_t *d_tile_nodes = nullptr;  // [n_tiles][TN] node | constraint bits | first-touch bit, or kNoNode
   int32_t *d_tile_info = nullptr;    // [n_tiles][2] first sorted cell, extents ex | ey << 8 | ez << 16

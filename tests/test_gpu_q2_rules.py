@@ -50,3 +50,38 @@ def test_products_about_the_rules(n, precision, tol, device):
     assert np.abs(y.double().cpu().numpy() - expect).max() < tol * np.abs(expect).max()
     op.compute_diagonal()
     assert np.abs(op.diagonal().double().cpu().numpy() - diag).max() < tol * np.abs(diag).max()
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-13), ("fp32", 1e-5)])
+@pytest.mark.parametrize("caching", ["tensor4", "scalar"])
+@pytest.mark.parametrize("n", [[1, 1, 1], [10, 3, 5], [8, 2, 17]], ids=str)
+@pytest.mark.parametrize("geometry", ["sheared", "cook"])
+def test_phase_masks(n, geometry, caching, precision, tol, device):
+    """products without the tangent, and without the sums, against those of the
+    cells layout, one launch and coloured launches alike"""
+    import torch
+    print(f"[phases] {n} {geometry} {caching} {precision}", flush=True)
+    mesh = lsmf.Mesh(3, 2, n, geometry="cook" if geometry == "cook" else "box")
+    if geometry == "sheared":
+        mesh.coords = np.ascontiguousarray(mesh.coords @ SHEAR.T)
+    rng = np.random.default_rng(3)
+    mu, lam = 1.0 + rng.random(mesh.n_cells), 2.0 + rng.random(mesh.n_cells)
+    u, _ = lsmf.smooth_displacement(mesh.coords, 0.02, 7)
+    cons = mesh.constrained_mask({0: [0, 1, 2], 1: [0]})
+    ops = []
+    for layout in ("auto", "cells"):
+        op = lsmf.NeoHookOperator(mesh, precision=precision, caching=caching, constrained=cons, layout=layout)
+        op.set_material(mu, lam)
+        op.set_linearization(torch.tensor(u, device=device))
+        op.cache()
+        ops.append(op)
+    x = torch.tensor(rng.standard_normal(mesh.n_dofs), device=device).to(ops[0].dtype)
+    for mask in ("rw", "rwsf", "default"):
+        y, z, w = (torch.full_like(x, float("nan")) for _ in range(3))
+        ops[1].vmult(w, x, mask=mask)
+        ops[0].vmult(y, x, mask=mask)
+        torch.cuda.synchronize()
+        ops[0].vmult(z, x, mask=mask, stream=torch.cuda.Stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(y, z), mask
+        assert float((y - w).abs().max()) < tol * float(w.abs().max()), mask
