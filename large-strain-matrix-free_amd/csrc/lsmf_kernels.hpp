@@ -854,10 +854,11 @@ __device__ __forceinline__ void qp_tensor4_ns(const T (&G)[DIM][DIM], const T *c
 // so a point needs 10 cached values in 3D instead of 17 (tensor2) or 36
 // (tensor4).  No difference of large terms is left for the product: in
 // tau = mu F F^T - c I they cancel at small strain.
-// The products are bound by the cached stream: 128^3 Q2 tensor4 FP64 3.86 ->
-// 1.77 ms (16.3 -> 4.5 GB cached), 61 x 67 x 59 Q2 tensor4 FP32 0.246 -> 0.165
-// ms, 64^3 Q4 tensor2 FP64 1.47 -> 1.33 ms; error against 64-bit references
-// 6.9e-15 -> 1.6e-15 (128^3 FP64), 1.4e-7 unchanged (FP32).
+// The stored-tensor products were bound by the cached stream; with this form
+// and the kernels that it made possible 128^3 Q2 tensor4 FP64 3.71 -> 1.50 ms (16.3
+// GB cached; here one value per point and cell constants, 0.9 GB), 61 x 67 x 59
+// Q2 tensor4 FP32 0.243 -> 0.145 ms, 64^3 Q4 tensor2 FP64 1.46 -> 1.17 ms; error
+// against 64-bit references 6.9e-15 -> 1.7e-15 (128^3 FP64), 1.4e-7 unchanged (FP32).
 template <int DIM, typename T>
 __device__ __forceinline__ void qp_compact(const T (&G)[DIM][DIM], const T *K, T cdw, T ldw, const T *A,
                                            T (&Phi)[DIM][DIM]) {
@@ -1799,23 +1800,24 @@ __global__ void __launch_bounds__(tile_threads<TILE>(), (vmult_min_waves<VAR, TI
 // plane of one component (N x N values at one z) and does x and y in
 // registers, then a column of N points (all components, three arrays each)
 // and does z, the tangent of its points and z transposed in registers, then
-// its plane again: 45 LDS accesses per point.  The lanes of a cell sit in one
-// wave, whose LDS accesses are in order, so only the tile's gather and the
+// its plane again: 45 LDS accesses per point.  A wave holds six cells, a cell's
+// lanes sit in one wave, whose LDS accesses are in order, so only the tile's gather and the
 // final sums need workgroup barriers.
 // 128^3 Q2 FP32 1052 -> 916 us, 48^3 79 -> 63 us: bound by memory (4.2 TB/s).
 // FP64 with the cached stream only 1814 -> 1786 us, bound by memory too (7.7
 // GB); V_COMPACT_U recomputes K = (J_ref + Grad_xi u)^-1, 4.4 GB: 1705 us, and
 // with the padded slots 1620 us (LDS bank conflicts 135 -> 22 of 525 kcycles),
-// 1555 us without the unit rows of the 1D matrices.  What is left is issue:
-// VALU and LDS each busy about half the time, nine waves per CU.
+// 1555 us without the unit rows of the 1D matrices, 1500 us without the branches
+// of the launch over all tiles.  What is left is issue: VALU and LDS each busy
+// about half the time, nine waves per CU.
 //
 // The residual (one evaluation, of u) and its VJP (u, then w) on affine cells
-// take the same way: 48^3 pair 377 -> 276 us, relative error against 64 bits
+// take the same way: 48^3 pair 377 -> 263 us, relative error against 64 bits
 // 1.1e-14 -> 6.1e-15.  Both evaluate F and tau as k_vmult does: the shorter flux
-// Jc A - c dw K^T (267 us) is a difference of terms that cancel without strain
-// and left 1e-16 there.  So does the scalar form (c cached)
-// on its 9x1x1 tiles: 48^3 FP64 212 -> 138 us, FP32 122 -> 85 us, and the FP32
-// error falls from 1.9e-6 to 1.7e-7 (no tau = mu F F^T - c I to cancel).
+// Jc A - c dw K^T is a difference of terms that cancel without strain and left
+// 1e-16 there.  So does the scalar form (c cached) on its 9x1x1 tiles: 48^3 FP64
+// 212 -> 135 us, FP32 122 -> 85 us, and the FP32 error falls from 1.9e-6 to 1.7e-7
+// (no tau = mu F F^T - c I to cancel).
 // ------------------------------------------------------------------------
 template <int N, typename T, int TILE> struct PlaneShape {
   // ten lanes (nine used) and a padded slot per cell, so that planes (lanes 9

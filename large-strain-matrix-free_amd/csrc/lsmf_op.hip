@@ -434,11 +434,12 @@ constexpr int kNotTileable = 1;
 // Largest operator whose products run in one launch: above it the tiles'
 // shares of common nodes travel to HBM and back and cost more than the
 // coloured launches' starts and tails save.  One launch against 8 coloured
-// ones, 3D Q2 tensor4 FP64, us: 13 / 59 (16^3), 42 / 66 (32^3), 128 / 156
-// (48^3, 2.7 M DoF), 276 / 284 (64^3, 6.4 M), 485 / 461 (80^3), 2116 / 1814
-// (128^3); scalar 203 / 218 (48^3), 493 / 450 (64^3); Q4 tensor4 FP32 52 / 78
-// (24^3, 2.7 M), 117 / 118 (32^3, 6.4 M), 217 / 206 (40^3); 2D Q2 FP64 (4
-// colours) 50 / 58 (2.1 M), 190 / 173 (8.4 M).
+// ones, us: 3D Q2 tensor4 FP64 40 / 68 (32^3), 110 / 138 (48^3, 2.7 M DoF), 165 /
+// 189 (56^3, 4.3 M), 250 / 246 (64^3, 6.4 M), 443 / 402 (80^3), 1889 / 1491
+// (128^3); FP32 145 / 155 (64^3), 251 / 234 (80^3); scalar 128 / 154 (48^3), 301 /
+// 285 (64^3); Q4 tensor4 FP32 51 / 75 (24^3, 2.7 M), 119 / 116 (32^3, 6.4 M), 222 /
+// 204 (40^3), tensor2 FP64 77 / 107 and 180 / 197; 2D Q2 FP64 (4 colours) 52 / 60
+// (2.1 M), 191 / 173 (8.4 M).
 constexpr size_t kOneLaunchDofs = 4000000;
 // FP64 products on affine Q2 cells of kFewTiles + 1 to kLineTiles wide tiles cache
 // K and run the line kernel: there a launch lasts as long as one tile, and the
