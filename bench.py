@@ -12,9 +12,10 @@ n_times = 10 loop, include/mf_elasticity.h:2354-2448), with x uniform in
 timed region.
 
 Prints one JSON line (stdout) with the throughput in GDoF/s, the HBM roofline
-of the fused cell kernel (algorithmic bytes of the reference's memory model,
-doc/large_strain.tex:739-753, divided by the kernel's event-timed duration)
-and a CPU baseline timed on the host.  Beside the headline it reports
+of the fused cell kernel (the bytes that the form of the tangent the operator
+runs has to read and write, divided by the kernel's event-timed duration), the
+bytes of the reference's memory model (doc/large_strain.tex:739-753) beside
+them, and a CPU baseline timed on the host.  Beside the headline it reports
   * the other caching variants and precisions on the same 128^3 mesh, each
     against its roofline (scalar also against the FP64 VALU peak),
   * renumbered meshes: the cells layout on the lexicographic numbering, and
@@ -68,6 +69,37 @@ def algorithmic_bytes(dim, caching, precision, n_qp, n_nodes):
         per_qp = nv + nv * nv + dim * dim + 1
         per_node = 2 * dim
     return es * (per_qp * n_qp + per_node * n_nodes)
+
+
+def form_bytes(mesh, caching, precision, tiled):
+    """bytes that one product has to read and write in the form its operator
+    runs: cached values per point, constants per cell, the displacement where K
+    is taken from it, node codes, source and result once each.  These meshes are
+    boxes (affine cells, Q1 metric) in formulation 1 with more than 2^19 points:
+    tensor2 and tensor4 run the compact form -- FP64 Q2 tiles c alone and 16
+    constants per cell, the others K and c (10) and 7 constants -- and scalar c
+    with 16 constants and the material (Q2 tiles)."""
+    es = 8 if precision == "fp64" else 4
+    N = mesh.degree + 1
+    q2_tiles = tiled and mesh.dim == 3 and mesh.degree == 2
+    per_cell, per_node = 0, 0
+    if caching == "scalar":
+        values, per_cell, per_node = 1, 16 * 8 + 2 * es, es * mesh.dim
+        tile = (171, 9) if q2_tiles else None
+        form = "c cached, K from the displacement"
+    elif caching in ("tensor2", "tensor4"):
+        recompute = q2_tiles and precision == "fp64"
+        values, per_cell = (1, 16 * 8) if recompute else (mesh.dim ** 2 + 1, 7 * 8)
+        per_node = es * mesh.dim if recompute else 0
+        tile = (285, 18) if q2_tiles else (425, 4) if tiled and mesh.dim == 3 and mesh.degree == 4 else None
+        form = "compact, c cached, K from the displacement" if recompute else "compact, K and c cached"
+    else:
+        raise ValueError(caching)
+    codes = mesh.n_cells * (tile[0] / tile[1] if tile else N ** mesh.dim) * 4
+    points = mesh.n_cells * N ** mesh.dim
+    kernel = "k_vmult_planes" if q2_tiles else "k_vmult"
+    return (int(es * values * points + per_cell * mesh.n_cells + (2 * mesh.dim * es + per_node) * mesh.n_nodes + codes),
+            form, f"{kernel} (fused gather, sums, tangent, sums, scatter)")
 
 
 def kernel_source_sha():
@@ -258,16 +290,18 @@ def vmult_record(mesh, mu, lam, ud, cons, caching, precision, steps, warmup, lay
     ms, ms_min, kern_ms, n_launch = timed_vmults(op, x, y, steps, warmup, torch)
     nq = mesh.degree + 1
     n_qp = mesh.n_cells * nq ** mesh.dim
-    alg = algorithmic_bytes(mesh.dim, caching, precision, n_qp, mesh.n_nodes)
+    model = algorithmic_bytes(mesh.dim, caching, precision, n_qp, mesh.n_nodes)
+    need, form, kernel = form_bytes(mesh, caching, precision, layout == "auto")
     launches = n_launch / steps
     avg_s = kern_ms / n_launch / 1e3
-    achieved = alg / launches / avg_s / 1e9
+    achieved = need / launches / avg_s / 1e9
     rec = {"caching": caching, "precision": precision, "layout": layout, "ms": round(ms, 4),
            "ms_min": round(ms_min, 4), "gdofs": round(mesh.n_dofs / ms / 1e6, 3),
            "kernel_avg_ms": round(avg_s * 1e3, 5), "launches_per_vmult": launches,
-           "algorithmic_bytes_per_vmult": int(alg),
+           "kernel": kernel, "form": form, "bytes_per_vmult": need,
            "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": round(achieved / HBM_PEAK_GBS, 4)},
+           "reference_model_bytes_per_vmult": int(model),
            "cache_bytes": op.memory_consumption()}
     if cfg_id is not None:
         tr, src = measured_traffic(cfg_id, caching, precision)
@@ -401,9 +435,9 @@ def adjoint_trade(cfg_id, reps, caching="tensor4"):
            "cache_build_ms": round(t_cache, 4), "cached_vmult_ms": round(t_vmult, 4),
            "vjp_state_bytes": 0, "cache_bytes": n_fields * 8 * n_qp,
            "cached_backward_bytes": (n_fields + nv + 1) * 8 * n_qp,
-           "note": f"VJP w.r.t. u, mu, lambda recomputes F, J, ln J per point; the cached alternative "
-                   f"({caching} cache + per-point b - I and ln J) would hold {n_fields} + {nv + 1} FP64 values "
-                   f"per point and apply the cached tangent for the u part"}
+           "note": f"VJP w.r.t. u, mu, lambda recomputes F, J, ln J per point; a backward that stored the "
+                   f"{caching} tangent (its tensors, b - I and ln J) would hold {n_fields} + {nv + 1} FP64 values "
+                   f"per point; cache_build_ms and cached_vmult_ms are of the operator's own, compact cache"}
     del op
     torch.cuda.empty_cache()
     return out
@@ -530,9 +564,11 @@ def main():
 
     nq = mesh.degree + 1
     n_qp = mesh.n_cells * nq ** mesh.dim
-    alg_bytes = algorithmic_bytes(mesh.dim, caching, args.precision, n_qp, mesh.n_nodes)
+    model_bytes = algorithmic_bytes(mesh.dim, caching, args.precision, n_qp, mesh.n_nodes)
+    need, form, kernel = (form_bytes(mesh, caching, args.precision, True) if caching in ("tensor2", "tensor4", "scalar")
+                          else (int(model_bytes), "stored", "k_vmult"))
     launches_per_vmult = n_launch / args.steps
-    bytes_per_launch = alg_bytes / launches_per_vmult
+    bytes_per_launch = need / launches_per_vmult
     avg_launch_s = kern_ms / n_launch / 1e3
     achieved = bytes_per_launch / avg_launch_s / 1e9
     traffic, traffic_src = (None, "not measured")
@@ -658,9 +694,12 @@ def main():
                    "precision": args.precision, "nu": cfg["nu"]},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "traffic_source": traffic_src,
-                     "kernel": "k_vmult (fused gather/SF/tangent/integrate/scatter, one launch per colour)",
+                     "kernel": kernel, "form": form,
                      "kernel_avg_ms": round(avg_launch_s * 1e3, 5), "launches_per_step": launches_per_vmult,
-                     "algorithmic_bytes_per_launch": int(bytes_per_launch)},
+                     "bytes_per_launch": int(bytes_per_launch),
+                     "note": "bytes that this form of the tangent has to read and write, over the kernel's time; "
+                             "traffic: measured HBM bytes per launch",
+                     "reference_model_bytes_per_launch": int(model_bytes / launches_per_vmult)},
         "cpu_baseline": cpu,
         "newton_solve": solve,
         "variants_same_mesh": variants_128,

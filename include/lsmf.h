@@ -224,7 +224,8 @@ lsmf_status lsmf_compute_diagonal(lsmf_op *op, lsmf_stream stream);
  * src must not alias.  Tiled operators of up to 4 M DoF run a product in one
  * launch over all tiles on the first stream that uses the operator; calls on
  * other streams and captured calls take one launch per tile colour, with the
- * same results, so products on several streams share no state. */
+ * same results, so products on several streams share no state.  A stream is
+ * known by its handle: destroy it only when its products have finished. */
 lsmf_status lsmf_vmult(lsmf_op *op, void *dst, const void *src, int add, unsigned mask, lsmf_stream stream);
 
 /* n_vectors products dst_b = A src_b of lsmf_vmult (set mode, constrained

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <mutex>
 #include <string>
@@ -87,7 +88,7 @@ struct lsmf_op {
   void *d_cache_other = nullptr;
   const void *form_cache = nullptr;  // *d_form as last written (nullptr: never)
   int form_changes = 0;
-  mutable bool recorded = false;
+  mutable std::atomic<bool> recorded{false};
   double *d_caff = nullptr;         // affine compact form: [sorted cell][kAffineStride]
   void *d_uc = nullptr;             // u of the last cache() where the products recompute K from it
   double *d_cgeo = nullptr;         // affine cells' geometry (VmultParams::cgeo), where the residual uses it
